@@ -413,8 +413,12 @@ void zheevd(dc2_context* c, Lane& L, int n, cplx* A, double* w, const char* what
   const int64_t nn = (int64_t)n * n;
   const bool native_ok = n >= 3 && n <= std::min(2048, c->native_max);
   const bool batched = c->batcher && !(c->native_min > 0 && n >= c->native_min);
+  // This library's solver also for rank-deficient matrices: its divide and conquer deflates
+  // the zero eigenvalues exactly (rocSOLVER's returned NaN there, which is why it takes Jacobi
+  // leaves instead: a RAS energy of 118 spinors with two 792 x 792 metrics took 53.6 ms with
+  // that, 22.4 ms with this).
   int method = c->eig_method >= 0 ? c->eig_method
-                                  : (kind == EigKind::rank_deficient ? 2 : (native_ok && !batched ? 4 : 1));
+                                  : (native_ok && !batched ? 4 : (kind == EigKind::rank_deficient ? 2 : 1));
   if (method == 4 && !native_ok) method = 1;
   cplx* keep = L.z("eig_keep", nn);
   DC2_HIP(hipMemcpyAsync(keep, A, nn * sizeof(cplx), hipMemcpyDeviceToDevice, L.stream));
