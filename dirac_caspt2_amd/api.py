@@ -403,6 +403,21 @@ def cdiag(ctx: Caspt2Context, c: np.ndarray, threshold: float = 0.0):
     return w, a, dimm.value
 
 
+def resolvent_energy(ctx: Caspt2Context, b: np.ndarray, y: np.ndarray, alpha: np.ndarray):
+    """dc2_resolvent_energy: (-sum_k Re(y_k^H u_k), sum_k |u_k|^2, iterations) for the columns y_k
+    of y with u_k = (b + alpha_k)^-1 y_k by conjugate gradients on the GPU, or None when a matrix
+    is not positive definite or a column does not converge."""
+    bf, yf = _fortran_complex(b), _fortran_complex(y)
+    al = np.ascontiguousarray(alpha, dtype=np.float64)
+    if bf.shape != (yf.shape[0],) * 2 or al.shape != yf.shape[1:]:
+        raise ValueError("b is n x n, y n x npert and alpha of npert values")
+    out = np.zeros(2)
+    it = ctypes.c_int32()
+    check("dc2_resolvent_energy", ctx.lib.dc2_resolvent_energy(ctx.h, bf.shape[0], yf.shape[1], _ptr(bf), _ptr(yf),
+                                                               _ptr(al), _ptr(out), ctypes.byref(it)))
+    return (float(out[0]), float(out[1]), it.value) if it.value else None
+
+
 def zgemm(ctx: Caspt2Context, opA: str, opB: str, M: int, N: int, K: int, alpha: complex, A, lda: int, sA: int,
           B, ldb: int, sB: int, beta: complex, C, ldc: int, sC: int, batch: int = 1):
     """C = alpha op(A) op(B) + beta C on device memory (DeviceArray buffers)."""

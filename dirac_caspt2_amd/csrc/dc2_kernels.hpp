@@ -155,6 +155,18 @@ void tri_dc(hipStream_t s, int n, double* w, const double* e, double* Z, void* w
 void hetrd_stats(int n, double* out);
 void hetrd_stats_reset();
 
+// ---------------------------------------------------------------- dc2_hpd.hip
+// out2 = {-sum_k Re(y_k^H u_k), sum_k |u_k|^2} with u_k = (Bt + alpha_k)^-1 y_k for the
+// Hermitian Bt (n x n, n <= cg_max_n()) and the npert columns of Y, by conjugate gradients.
+// false when a column's matrix is not positive definite, a column does not converge or its
+// residual is above 1e-12 |y|: nothing usable was computed and the caller diagonalises Bt.
+// work: cg_work_bytes(n, npert) of device memory; host2: two ints of page-locked memory;
+// partial: 2 npert doubles of device memory.  Synchronises the stream.
+int64_t cg_max_n();
+int64_t cg_work_bytes(int64_t n, int64_t npert);
+bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const cplx* Y, const double* alpha,
+                  void* work, int* host2, double* partial, double* out2, int* iterations = nullptr);
+
 // ---------------------------------------------------------------- dc2_pt2.hip
 struct Dens {
   int na;
@@ -200,6 +212,8 @@ void alphas(hipStream_t s, char X, int ni, int na, int ns, const double* eps, co
 // then a single-block final pass (deterministic order)
 void e2_reduce(hipStream_t s, int64_t dimm, int64_t npert, const cplx* X, const double* wb, const double* alpha,
                double* partial, int64_t npartial_max, double* out2);
+// out2 = the sums of np pairs (e, s) at partial, in a fixed order
+void sum_partials(hipStream_t s, int64_t np, const double* partial, double* out2);
 void e2_H(hipStream_t s, int ni, int ns, const cplx* Hb, const double* eps, double eshift, const int* ipairs,
           const int* spairs, double* partial, int64_t npartial_max, double* out2);
 int64_t e2_partials_needed(int64_t nwork);

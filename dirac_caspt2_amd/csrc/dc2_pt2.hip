@@ -666,6 +666,10 @@ void e2_reduce(hipStream_t s, int64_t dimm, int64_t npert, const cplx* X, const 
   hipLaunchKernelGGL(k_final2, dim3(1), dim3(RB), 0, s, nb, partial, out2);
   DC2_HIP(hipGetLastError());
 }
+void sum_partials(hipStream_t s, int64_t np, const double* partial, double* out2) {
+  hipLaunchKernelGGL(k_final2, dim3(1), dim3(RB), 0, s, np, partial, out2);
+  DC2_HIP(hipGetLastError());
+}
 int e2_schur_max_dropped() { return SCHUR_RMAX; }
 void e2_schur(hipStream_t s, int64_t m, int r, int64_t npert, const cplx* Gd, const cplx* Z, const double* f,
               const double* alpha, double* partial, double* out2) {

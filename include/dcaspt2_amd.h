@@ -134,6 +134,13 @@ int dc2_casmat(dc2_context* ctx, double* mat);
  * eigenvectors, w by the ascending eigenvalues, *dimm = count(w >= threshold)
  * (or n when threshold == 0) */
 int dc2_cdiag(dc2_context* ctx, double* c, int32_t n, int32_t* dimm, double* w, double threshold);
+/* sums over the npert columns y_k of Y (n x npert complex, host) with u_k = (B + alpha_k)^-1 y_k,
+ * B (n x n complex Hermitian, host, n <= 2048): out2 = { -sum Re(y_k^H u_k), sum |u_k|^2 }, the
+ * E2 and sumc2 of one subspace from B~ (solve_A_subspace.F90:197-257) by conjugate gradients on
+ * the GPU.  *iterations: the iterations taken, or 0 when some B + alpha_k is not positive
+ * definite or a column did not converge, and out2 is not set */
+int dc2_resolvent_energy(dc2_context* ctx, int32_t n, int64_t npert, const double* b, const double* y,
+                         const double* alpha, double* out2, int32_t* iterations);
 /* C = alpha op(A) op(B) + beta C on device memory, batched by strides;
  * opA in 'N','T','C'; opB in 'N','R' (conjugate, no transpose),'T','C' */
 int dc2_zgemm(dc2_context* ctx, char opA, char opB, int64_t M, int64_t N, int64_t K, const double* alpha,
