@@ -42,6 +42,7 @@ _SIGS = {
     "dc2_casmat": (c_int, [P, P]),
     "dc2_cdiag": (c_int, [P, P, c_int, P, P, c_dbl]),
     "dc2_resolvent_energy": (c_int, [P, c_int, c_i64, P, P, P, P, P]),
+    "dc2_whiten": (c_int, [P, c_int, P, P, c_dbl, P, P, P, P]),
     "dc2_zgemm": (c_int, [P, ctypes.c_char, ctypes.c_char, c_i64, c_i64, c_i64, P, P, c_i64, c_i64, P, c_i64, c_i64,
                           P, P, c_i64, c_i64, c_i64]),
     "dc2_zherk": (c_int, [P, c_i64, c_i64, P, c_i64, P, c_i64, c_int]),

@@ -418,6 +418,19 @@ def resolvent_energy(ctx: Caspt2Context, b: np.ndarray, y: np.ndarray, alpha: np
     return (float(out[0]), float(out[1]), it.value) if it.value else None
 
 
+def whiten(ctx: Caspt2Context, s: np.ndarray, b: np.ndarray, sigma: float = 1e-8):
+    """dc2_whiten: (L^-1, L^-1 b L^-H, smallest eigenvalue) of s = L L^H when every eigenvalue of s
+    is above sigma, else None."""
+    sf, bf = _fortran_complex(s), _fortran_complex(b)
+    if sf.shape != bf.shape or sf.shape[0] != sf.shape[1]:
+        raise ValueError("s and b are n x n")
+    linv, bt = np.zeros_like(sf, order="F"), np.zeros_like(sf, order="F")
+    lam, ok = ctypes.c_double(), ctypes.c_int32()
+    check("dc2_whiten", ctx.lib.dc2_whiten(ctx.h, sf.shape[0], _ptr(sf), _ptr(bf), float(sigma), _ptr(linv), _ptr(bt),
+                                           ctypes.byref(lam), ctypes.byref(ok)))
+    return (linv, bt, lam.value) if ok.value else None
+
+
 def zgemm(ctx: Caspt2Context, opA: str, opB: str, M: int, N: int, K: int, alpha: complex, A, lda: int, sA: int,
           B, ldb: int, sB: int, beta: complex, C, ldc: int, sC: int, batch: int = 1):
     """C = alpha op(A) op(B) + beta C on device memory (DeviceArray buffers)."""

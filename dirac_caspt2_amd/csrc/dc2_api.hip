@@ -927,6 +927,7 @@ int64_t count_retained(Lane& L, int64_t n, const double* w_dev, double& margin, 
 struct BlockPrep {
   int64_t n = 0, dimm = 0;
   bool cg = false;   // X_bc1 holds B~, not its eigenvectors
+  bool chol = false; // S^-1/2 is the inverse Cholesky factor in X_hLi, not U L^-1/2 in X_uc
   double margin = INFINITY;
 };
 BlockPrep solve_prep(dc2_context* c, Lane& L, char X, int64_t n, cplx* S, cplx* B, EigKind kind, double scale = 1.0) {
@@ -957,6 +958,53 @@ BlockPrep solve_prep(dc2_context* c, Lane& L, char X, int64_t n, cplx* S, cplx* 
   return p;
 }
 
+// S = L L^H instead of S -> cdiag, when every eigenvalue of S is above the threshold thr (the
+// second factorisation of chol_inverse): then all directions are retained and L^-1 serves as
+// S^-1/2 (the resolvents do not depend on the orthonormalisation).  Leaves L^-1 in X_hLi and B~
+// in X_bc1; S and B are kept.  False: some eigenvalue is below thr, or too close to it.
+bool chol_whiten(dc2_context* c, Lane& L, char X, int64_t n, const cplx* S, const cplx* B, double thr) {
+  hipStream_t s = L.stream;
+  auto nm = [X](const char* b) { return std::string(1, X) + b; };
+  const int64_t np = chol_np(n);
+  cplx* Li = L.z(nm("_hLi").c_str(), np * np);
+  cplx* work = L.z(nm("_hW").c_str(), chol_work_elems(n));
+  cplx* bc1 = L.z(nm("_bc1").c_str(), n * n);
+  int* flags = L.i(nm("_hflag").c_str(), 2);
+  set_gemm_tag(4);
+  chol_inverse(s, n, S, n, thr, work, Li, flags);
+  zgemm_congruence(s, n, Li, np, B, n, work, bc1, n);
+  set_gemm_tag(0);
+  int hf[2];
+  L.download(hf, flags, sizeof(hf));
+  if (c->debug)
+    std::fprintf(stderr, "dc2: Cholesky of the %c metric (n=%lld): %s\n", X, (long long)n,
+                 hf[0] || hf[1] ? "eigenvalues below the threshold" : "whole rank");
+  return hf[0] == 0 && hf[1] == 0;
+}
+
+// with the automatic eigensolver choice, where the resolvents take E2 from B~ (cg_route); not
+// with RAS limits, whose metrics are rank-deficient as a rule
+bool chol_route(const dc2_context* c, char X, int64_t n) {
+  return cg_route(c, X, n) && c->ras[0] + c->ras[1] + c->ras[2] == 0;
+}
+
+// the V-independent half of A's antisymmetric reduction (solve_prep) by the Cholesky factor;
+// scale as there.  The margin is the smallest eigenvalue's distance to the threshold.
+bool chol_prep(dc2_context* c, Lane& L, char X, int64_t n, const cplx* S, const cplx* B, double scale, BlockPrep& p) {
+  const double thr = 1.0e-8;
+  // a relative 1e-4 above the threshold: closer ones are left to the eigensolver
+  if (!chol_route(c, X, n) || !chol_whiten(c, L, X, n, S, B, 1.0001 * thr / scale)) return false;
+  double lam = 0.0;
+  if (!chol_lambda_min(L.stream, n, L.z((std::string(1, X) + "_hLi").c_str(), 1), L.z("lanczos", 4 * n + 256),
+                       reinterpret_cast<double*>(L.host(512 * sizeof(double), 1)), lam))
+    return false;
+  p.n = n;
+  p.dimm = n;
+  p.margin = std::min(p.margin, std::fabs(scale * lam - thr));
+  p.cg = p.chol = true;
+  return true;
+}
+
 // The V half (solve_A_subspace.F90:197-257): Y = (U L^-1/2)^H V, X = W^H Y, E2 and sumc2
 SolveOut solve_finish(dc2_context* c, Lane& L, char X, const BlockPrep& p, int64_t npert, const cplx* V,
                       const double* alpha) {
@@ -968,12 +1016,17 @@ SolveOut solve_finish(dc2_context* c, Lane& L, char X, const BlockPrep& p, int64
   auto nm = [X](const char* b) { return std::string(1, X) + b; };
   const int64_t n = p.n, dimm = p.dimm;
   const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
-  const cplx* uc = L.z(nm("_uc").c_str(), n * dimm);
   cplx* bc1 = L.z(nm("_bc1").c_str(), dimm * dimm);
   double* wb = L.d(nm("_wb").c_str(), dimm);
   cplx* Y = L.z(nm("_Y").c_str(), dimm * npert);
   set_gemm_tag(4);
-  zgemm(s, 'C', 'N', dimm, npert, n, one, uc, n, 0, V, n, 0, zero, Y, dimm, 0, 1);
+  if (p.chol) {
+    const int64_t np = chol_np(n);
+    zgemm(s, 'N', 'N', n, npert, n, one, L.z(nm("_hLi").c_str(), np * np), np, 0, V, n, 0, zero, Y, n, 0, 1);
+  } else {
+    const cplx* uc = L.z(nm("_uc").c_str(), n * dimm);
+    zgemm(s, 'C', 'N', dimm, npert, n, one, uc, n, 0, V, n, 0, zero, Y, dimm, 0, 1);
+  }
   set_gemm_tag(0);
   if (p.cg) {   // on failure (an intruder state) the eigendecomposition that solve_prep left out
     if (cg_energy(c, L, dimm, npert, bc1, Y, alpha, r)) return r;
@@ -996,6 +1049,7 @@ struct GramMetric {
   bool btilde = false;    // B~ formed before V was known: its eigendecomposition in X_bc1 / X_wbt,
   bool cg = false;        // or (cg) B~ itself in X_bc1
   bool thin = false;      // C through its thin factor: T's eigenvectors in X_Tthin, t L^-1/2 in X_TSthin
+  bool chol = false;      // thin, T's inverse Cholesky factor in X_hLi instead, B~ in X_bc1
   int64_t m = 0, dimm = 0;
   double margin = INFINITY;
   double seconds = 0.0;   // time spent on the lane before the subspace itself ran
@@ -1051,6 +1105,20 @@ GramMetric gram_eig(dc2_context* c, Lane& L, char X, int64_t n, const cplx* Y, c
     build_thin_c(s, na, c->ne, m, Phi, Av, PsiH);
     zherk_upper(s, nred, m, PsiH, nred, T, nred);
     check_finite(c, s, "Psi'^H Psi'", T, nred * nred);
+    if (chol_route(c, X, nred)) {
+      // whole rank, with every eigenvalue at least twice the threshold, so that the closest
+      // ones to it are the m - nred that vanish: B~ = L^-1 (Psi'^H F Psi') L^-H
+      cplx* PF = L.z(nm("_PsiF").c_str(), nred * m);
+      cplx* B = L.z(nm("_Bthin").c_str(), nred * nred);
+      scale_cols(s, nred, m, f, PsiH, PF);
+      zgemm_herm(s, nred, m, PF, nred, PsiH, nred, B, nred);
+      if (chol_whiten(c, L, X, nred, T, B, 2.0 * thr)) {
+        g.chol = g.btilde = g.cg = true;
+        g.dimm = nred;
+        g.margin = std::min(g.margin, thr);
+        return g;
+      }
+    }
     zheevd(c, L, (int)nred, T, lt, "a determinant-space metric", ras ? EigKind::rank_deficient : EigKind::general);
     g.margin = std::min(g.margin, thr);   // the m - nred eigenvalues of G that vanish identically
     g.dimm = count_retained(L, nred, lt, g.margin);
@@ -1112,7 +1180,7 @@ void gram_rotated_parts(dc2_context* c, Lane& L, char X, int64_t n, const GramMe
   if (!phi_current)
     build_phi(s, c->na, c->ne, X == 'A', c->nfull, c->rank_full.get(), c->Y1.get(), c->eps.get() + c->ni, m,
               L.l(nm("_strings").c_str(), m), L.z(nm("_Phi").c_str(), m * n), L.d(nm("_f").c_str(), m));
-  if (g.dimm > 0)
+  if (g.dimm > 0 && !g.thin)
     scale_cols_tail(s, m, g.dimm, L.z(nm("_G").c_str(), m * m), L.d(nm("_lam").c_str(), m),
                     L.z(nm("_GL").c_str(), m * g.dimm), true);
 }
@@ -1130,7 +1198,7 @@ GramMetric gram_metric(dc2_context* c, Lane& L, char X, int64_t n) {
 // resolvent (at most e2_schur_max_dropped() directions dropped).
 void gram_btilde(dc2_context* c, Lane& L, char X, GramMetric& g) {
   const int64_t m = g.m, dimm = g.dimm, nd = m - dimm;
-  if (m == 0 || dimm == 0 || (c->schur && nd <= e2_schur_max_dropped())) return;
+  if (m == 0 || dimm == 0 || g.btilde || (c->schur && nd <= e2_schur_max_dropped())) return;
   hipStream_t s = L.stream;
   auto nm = [X](const char* b) { return std::string(1, X) + b; };
   const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
@@ -1174,7 +1242,6 @@ SolveOut solve_block_gram(dc2_context* c, Lane& L, char X, const GramMetric& g, 
   const cplx* Phi = L.z(nm("_Phi").c_str(), m * n);
   cplx* G = L.z(nm("_G").c_str(), m * m);
   const double* f = L.d(nm("_f").c_str(), m);
-  const cplx* GL = L.z(nm("_GL").c_str(), m * dimm);
   const int64_t nd = m - dimm;
   const cplx* Gk = G + m * nd;
   cplx* Y = L.z(nm("_Y").c_str(), dimm * npert);
@@ -1185,13 +1252,20 @@ SolveOut solve_block_gram(dc2_context* c, Lane& L, char X, const GramMetric& g, 
     const int64_t nred = (int64_t)na * na * (na - 1) / 2;
     cplx* MV = L.z(nm("_MVthin").c_str(), nred * npert);
     cplx* W = L.z(nm("_Wthin").c_str(), nred * npert);
-    const cplx* TS = L.z(nm("_TSthin").c_str(), nred * dimm);
     thin_c_w(s, na, c->ne, npert, V, MV, W);
     set_gemm_tag(4);
-    zgemm(s, 'C', 'N', dimm, npert, nred, one, TS, nred, 0, W, nred, 0, zero, Y, dimm, 0, 1);
+    if (g.chol) {
+      const int64_t np = chol_np(nred);
+      zgemm(s, 'N', 'N', nred, npert, nred, one, L.z(nm("_hLi").c_str(), np * np), np, 0, W, nred, 0, zero, Y, nred, 0,
+            1);
+    } else {
+      const cplx* TS = L.z(nm("_TSthin").c_str(), nred * dimm);
+      zgemm(s, 'C', 'N', dimm, npert, nred, one, TS, nred, 0, W, nred, 0, zero, Y, dimm, 0, 1);
+    }
     set_gemm_tag(0);
   } else {
     cplx* P = L.z(nm("_P").c_str(), m * npert);
+    const cplx* GL = L.z(nm("_GL").c_str(), m * dimm);
     set_gemm_tag(4);
     zgemm(s, 'N', 'N', m, npert, n, one, Phi, m, 0, V, n, 0, zero, P, m, 0, 1);
     zgemm(s, 'C', 'N', dimm, npert, m, one, GL, m, 0, P, m, 0, zero, Y, dimm, 0, 1);
@@ -1346,7 +1420,8 @@ SubPrep subspace_prep(dc2_context* c, Lane& L, int k) {
       // S_full = K^H S_red K with K K^H = 2 I (a+_u a+_t = -a+_t a+_u, a+_t a+_t = 0), so the
       // nonzero eigenvalues of the reference's S are twice those of S_red: cutoff at 0.5e-8
       const bool ras = c->ras[0] + c->ras[1] + c->ras[2] != 0;
-      p.bp = solve_prep(c, L, X, nred, S, B, nred > mdet || (route.phi && ras) ? EigKind::rank_deficient
+      if (!route.phi || nred > mdet || !chol_prep(c, L, X, nred, S, B, 2.0, p.bp))
+        p.bp = solve_prep(c, L, X, nred, S, B, nred > mdet || (route.phi && ras) ? EigKind::rank_deficient
                                                                                  : EigKind::general, 2.0);
     } else {
       const EigKind kind = (X == 'A' || X == 'C') ? EigKind::rank_deficient : EigKind::general;
@@ -2313,6 +2388,32 @@ int dc2_resolvent_energy(dc2_context* c, int32_t n, int64_t npert, const double*
                                  reinterpret_cast<int*>(L.host(2 * sizeof(int), 1)), L.d("partial", 2 * npert), o2, &it);
     if (ok) L.download(out2, o2, 2 * sizeof(double));
     *iterations = ok ? it : 0;
+  });
+}
+
+int dc2_whiten(dc2_context* c, int32_t n, const double* S, const double* b, double sigma, double* linv, double* btilde,
+               double* lambda_min, int32_t* whole_rank) {
+  return guarded([&] {
+    DC2_CHECK(c && S && b && linv && btilde && lambda_min && whole_rank, 1, "null argument");
+    DC2_CHECK(n >= 1 && n <= 2048, 1, "n must be in 1..2048");
+    DC2_HIP(hipSetDevice(c->device));
+    Lane& L = *c->lane0;
+    const int64_t nn = (int64_t)n * n, np = chol_np(n);
+    DevBuf<cplx> Sd(nn), Bd(nn);
+    DC2_HIP(hipMemcpyAsync(Sd.get(), S, nn * sizeof(cplx), hipMemcpyHostToDevice, c->stream));
+    DC2_HIP(hipMemcpyAsync(Bd.get(), b, nn * sizeof(cplx), hipMemcpyHostToDevice, c->stream));
+    *whole_rank = 0;
+    if (!chol_whiten(c, L, 'W', n, Sd.get(), Bd.get(), sigma)) return;
+    const cplx* Li = L.z("W_hLi", np * np);
+    double lam = 0.0;
+    if (!chol_lambda_min(c->stream, n, Li, L.z("lanczos", 4 * (int64_t)n + 256),
+                         reinterpret_cast<double*>(L.host(512 * sizeof(double), 1)), lam))
+      return;
+    DC2_HIP(hipMemcpy2DAsync(linv, n * sizeof(cplx), Li, np * sizeof(cplx), n * sizeof(cplx), n, hipMemcpyDeviceToHost,
+                             c->stream));
+    copy_sync(c, btilde, L.z("W_bc1", nn), nn * sizeof(cplx), hipMemcpyDeviceToHost);
+    *lambda_min = lam;
+    *whole_rank = 1;
   });
 }
 

@@ -840,6 +840,11 @@ __global__ void k_scale_rows(int64_t m, int64_t ncol, const double* f, const cpl
   out[r + m * c] = cscale(in[r + m * c], f[r]);
 }
 
+__global__ void k_scale_cols(int64_t m, int64_t count, const double* f, const cplx* in, cplx* out) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < count) out[t] = cscale(in[t], f[t / m]);
+}
+
 }  // namespace
 
 void enumerate_dets(hipStream_t s, const DetParams& p, int* ff, int* fc, int* rf, int* rc, int64_t* full_dets,
@@ -1158,6 +1163,11 @@ void davidson_normalize(hipStream_t s, int64_t n, int ncol, cplx* T) {
   DC2_HIP(hipGetLastError());
 }
 
+void scale_cols(hipStream_t s, int64_t m, int64_t ncol, const double* f, const cplx* in, cplx* out) {
+  if (m <= 0 || ncol <= 0) return;
+  hipLaunchKernelGGL(k_scale_cols, dim3(cdiv(m * ncol, 256)), dim3(256), 0, s, m, m * ncol, f, in, out);
+  DC2_HIP(hipGetLastError());
+}
 void scale_rows(hipStream_t s, int64_t m, int64_t ncol, const double* f, const cplx* in, cplx* out) {
   if (m <= 0 || ncol <= 0) return;
   DC2_CHECK(ncol < 65536, 1, "scale_rows: too many columns for one grid dimension");

@@ -124,6 +124,12 @@ void zherk_upper(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda
 // the same upper tiles, reduction and mirror
 void zgemm_herm(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda, const cplx* B, int64_t ldb, cplx* C,
                 int64_t ldc, int split = 0);
+// C <- C - A^H A on and above the diagonal (A k x m), batched by strides
+void zherk_trailing(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda, int64_t sA, cplx* C, int64_t ldc,
+                    int64_t sC, int64_t batch);
+// C = L B L^H for Hermitian B and lower triangular L (zeros above its diagonal); T: n x n scratch
+void zgemm_congruence(hipStream_t s, int64_t n, const cplx* L, int64_t ldl, const cplx* B, int64_t ldb, cplx* T,
+                      cplx* C, int64_t ldc);
 // GEMM tuning table (exact shapes): the MFMA kernel variant (1..4: K tile 16/32 x LDS padding
 // 1/16) and split-K factor (1: none) chosen for (opA, opB, M, N, K, batch) by measurement.
 // gemm_tune times every candidate on scratch operands on stream s and installs the fastest;

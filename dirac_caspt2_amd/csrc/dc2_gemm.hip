@@ -144,12 +144,15 @@ __global__ __launch_bounds__(256) void k_zgemm(int64_t M, int64_t N, int64_t Kfu
 // transposed-operand stores and of the MFMA operand reads).
 // UPPER: only the tiles that reach the upper triangle (a Hermitian product; the tiles
 // entirely below the diagonal leave at once)
+// tri: zeros the operands are known to have, which end a tile's K loop early: TRI_A op(A) lower
+// triangular (k <= m), TRI_B op(B) upper triangular (k <= n)
+enum { TRI_NONE = 0, TRI_A = 1, TRI_B = 2 };
 template <char OPA, char OPB, int KB, int PAD, bool UPPER = false>
 __global__ __launch_bounds__(256) void k_zgemm2(int64_t M, int64_t N, int64_t Kfull, cplx alpha,
                                                 const cplx* __restrict__ A, int64_t lda, int64_t sA,
                                                 const cplx* __restrict__ B, int64_t ldb, int64_t sB,
                                                 cplx beta, cplx* __restrict__ C, int64_t ldc, int64_t sC, int sk,
-                                                int64_t kchunk) {
+                                                int64_t kchunk, int tri = TRI_NONE) {
   int64_t mt, nt;
   xcd_tile(gridDim.x, gridDim.y, blockIdx.x, blockIdx.y, mt, nt);
   if (UPPER && mt * BM > nt * BN + BN - 1) return;   // uniform
@@ -161,7 +164,9 @@ __global__ __launch_bounds__(256) void k_zgemm2(int64_t M, int64_t N, int64_t Kf
   B += bz * sB;
   C += (sk > 1 ? bz * sk + kz : bz) * sC;   // split K: partial kz of product bz
   const int64_t kbeg = kz * kchunk;
-  const int64_t kend = (kbeg + kchunk < Kfull) ? kbeg + kchunk : Kfull;
+  int64_t kend = (kbeg + kchunk < Kfull) ? kbeg + kchunk : Kfull;
+  if (tri == TRI_A && kend > (mt + 1) * BM) kend = (mt + 1) * BM;
+  if (tri == TRI_B && kend > (nt + 1) * BN) kend = (nt + 1) * BN;
   const int64_t m0 = mt * BM, n0 = nt * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
@@ -438,12 +443,13 @@ __global__ __launch_bounds__(256) void k_zgemm_tall(int64_t M, int64_t N, int64_
     if (j < N) w[M * j] = acc[j];
 }
 
-// the strict lower triangle as the conjugate of the upper one (the diagonal is kept)
+// the strict lower triangle as the conjugate of the upper one, the diagonal real
 __global__ void k_lower_from_upper(int64_t m, cplx* __restrict__ C, int64_t ldc) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= m * m) return;
   const int64_t i = t % m, j = t / m;
   if (i > j) C[i + ldc * j] = cconj(C[j + ldc * i]);
+  else if (i == j) C[i + ldc * j].y = 0.0;
 }
 
 // C = sum_kz W[kz] on and above the diagonal (the split-K partials of a Hermitian product,
@@ -660,19 +666,19 @@ void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, cplx alpha, const cp
   switch (variant) {
     case 1:
       hipLaunchKernelGGL((k_zgemm2<OPA, OPB, 16, 1>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB, b1,
-                         Cw, ldw, sw, sk, kchunk);
+                         Cw, ldw, sw, sk, kchunk, (int)TRI_NONE);
       break;
     case 2:
       hipLaunchKernelGGL((k_zgemm2<OPA, OPB, 16, 16>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB,
-                         b1, Cw, ldw, sw, sk, kchunk);
+                         b1, Cw, ldw, sw, sk, kchunk, (int)TRI_NONE);
       break;
     case 3:
       hipLaunchKernelGGL((k_zgemm2<OPA, OPB, 32, 1>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB, b1,
-                         Cw, ldw, sw, sk, kchunk);
+                         Cw, ldw, sw, sk, kchunk, (int)TRI_NONE);
       break;
     case 4:
       hipLaunchKernelGGL((k_zgemm2<OPA, OPB, 32, 16>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB,
-                         b1, Cw, ldw, sw, sk, kchunk);
+                         b1, Cw, ldw, sw, sk, kchunk, (int)TRI_NONE);
       break;
     default:
       hipLaunchKernelGGL((k_zgemm<OPA, OPB>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB, b1, Cw,
@@ -762,15 +768,46 @@ void zgemm_herm(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda,
     cplx* W = splitk_workspace(s, (size_t)sk * m * m);
     dim3 grid(T, T, (unsigned)sk);
     hipLaunchKernelGGL((k_zgemm2<'N', 'C', 16, 1, true>), grid, dim3(256), 0, s, m, m, k, one, A, lda, (int64_t)0, B,
-                       ldb, (int64_t)0, zero, W, m, m * m, sk, kchunk);
+                       ldb, (int64_t)0, zero, W, m, m * m, sk, kchunk, (int)TRI_NONE);
     hipLaunchKernelGGL(k_herk_reduce, dim3(cdiv(m * m, 256)), dim3(256), 0, s, m, sk, W, C, ldc);
     DC2_HIP(hipGetLastError());
     return;
   }
   dim3 grid(T, T, 1);
   hipLaunchKernelGGL((k_zgemm2<'N', 'C', 16, 1, true>), grid, dim3(256), 0, s, m, m, k, one, A, lda, (int64_t)0, B,
-                     ldb, (int64_t)0, zero, C, ldc, (int64_t)0, 1, k);
+                     ldb, (int64_t)0, zero, C, ldc, (int64_t)0, 1, k, (int)TRI_NONE);
   hipLaunchKernelGGL(k_lower_from_upper, dim3(cdiv(m * m, 256)), dim3(256), 0, s, m, C, ldc);
+  DC2_HIP(hipGetLastError());
+}
+
+// C <- C - A^H A on and above the diagonal (m x m, A k x m with k short), batched by strides:
+// the trailing update of a Cholesky factorisation
+void zherk_trailing(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda, int64_t sA, cplx* C, int64_t ldc,
+                    int64_t sC, int64_t batch) {
+  if (m <= 0) return;
+  const int64_t T = cdiv(m, BM);
+  DC2_CHECK(T < 65536 && batch < 65536, 1, "zherk_trailing: matrix too large for the grid");
+  dim3 grid(T, T, (unsigned)batch);
+  hipLaunchKernelGGL((k_zgemm2<'C', 'N', 16, 1, true>), grid, dim3(256), 0, s, m, m, k, mk(-1.0, 0.0), A, lda, sA, A,
+                     lda, sA, mk(1.0, 0.0), C, ldc, sC, 1, k, (int)TRI_NONE);
+  DC2_HIP(hipGetLastError());
+}
+
+// C = L B L^H (n x n, Hermitian B, L lower triangular with zeros above the diagonal): T = L B,
+// then the upper tiles of T L^H and their mirror; the K loops end at the triangle's edge, so
+// the two products take 1/2 and 1/3 of the full ones
+void zgemm_congruence(hipStream_t s, int64_t n, const cplx* L, int64_t ldl, const cplx* B, int64_t ldb, cplx* T,
+                      cplx* C, int64_t ldc) {
+  if (n <= 0) return;
+  const int64_t t = cdiv(n, BM);
+  DC2_CHECK(t < 65536, 1, "zgemm_congruence: matrix too large for the grid");
+  const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
+  dim3 grid(t, t, 1);
+  hipLaunchKernelGGL((k_zgemm2<'N', 'N', 16, 1>), grid, dim3(256), 0, s, n, n, n, one, L, ldl, (int64_t)0, B, ldb,
+                     (int64_t)0, zero, T, n, (int64_t)0, 1, n, (int)TRI_A);
+  hipLaunchKernelGGL((k_zgemm2<'N', 'C', 16, 1, true>), grid, dim3(256), 0, s, n, n, n, one, T, n, (int64_t)0, L, ldl,
+                     (int64_t)0, zero, C, ldc, (int64_t)0, 1, n, (int)TRI_B);
+  hipLaunchKernelGGL(k_lower_from_upper, dim3(cdiv(n * n, 256)), dim3(256), 0, s, n, C, ldc);
   DC2_HIP(hipGetLastError());
 }
 

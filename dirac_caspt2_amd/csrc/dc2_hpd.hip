@@ -234,4 +234,363 @@ bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const
   return poll();
 }
 
+// ------------------------------------------------------------------ Cholesky whitening
+//
+// When no eigenvalue of a metric S lies below the linear-dependency threshold, every
+// orthonormalisation of its space gives the same resolvents, and S = U^H U with L^-1 = U^-H
+// replaces the eigendecomposition: B~ = L^-1 B L^-H, y = L^-1 V.  That no eigenvalue is below
+// the threshold is decided by a second factorisation, of S - sigma I, whose pivots are all
+// positive exactly when every eigenvalue of S is above sigma (to rounding, as for an
+// eigensolver).  Both are factorised side by side as a batch of two: the panels are a chain of
+// dependent steps, each too small to fill the device.
+//
+// Per step of NB = 64 rows: k_chol_step, in which every workgroup eliminates the diagonal
+// block redundantly (64 steps with one workgroup barrier each, the block in registers) and
+// then multiplies its 64 columns of the block row by the block's inverse factor on the matrix
+// cores, and one trailing update of the upper tiles (zherk_trailing).  L^-1 from the inverse
+// diagonal blocks by merging neighbours, [[X, 0], [-Z U12^H X, Z]], doubling the block size.
+//
+// Bound by the chain of the 20 steps at n = 1274 (about 60 us each: the elimination 40, the
+// update 15), against 13.4 ms for the tridiagonalisation and 9 ms for the divide and conquer,
+// back-transformation and scaled products it replaces; the two factorisations, L^-1 and B~ take
+// 3.3 ms beside the other lanes.  324 spinors, FP64: 49.7 -> 39.9 ms per energy, split 37.7.
+
+namespace {
+
+constexpr int CH_NB = 64, CH_LS = CH_NB + 1;
+
+// W[b] (np x np): S in the leading n x n corner, less sigma_b on the diagonal (sigma_0 = 0), the
+// unit matrix below it
+__global__ __launch_bounds__(256) void k_chol_pack(int n, int np, const cplx* __restrict__ S, int64_t lds, double sigma,
+                                                   cplx* __restrict__ W) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= (int64_t)np * np) return;
+  const int i = (int)(t % np), j = (int)(t / np);
+  cplx v = mk(i == j ? 1.0 : 0.0, 0.0);
+  if (i < n && j < n) v = S[i + lds * j];
+  W[t] = v;
+  if (i == j && i < n) v.x -= sigma;
+  W[(int64_t)np * np + t] = v;
+}
+
+// Step kb: block row kb of U = L^H from W, and (workgroup 0 of each matrix) the inverse of its
+// diagonal block into Li.  flag[b] is set when a pivot of matrix b is not positive.
+__global__ __launch_bounds__(256) void k_chol_step(int np, int kb, const cplx* __restrict__ W, cplx* __restrict__ U,
+                                                   cplx* __restrict__ Li, int* __restrict__ flag) {
+  __shared__ cplx rowb[2][CH_NB], colb[2][CH_NB];
+  __shared__ double Ar[CH_NB][CH_LS], Ai[CH_NB][CH_LS], Br[CH_NB][CH_LS], Bi[CH_NB][CH_LS];
+  typedef double d4 __attribute__((ext_vector_type(4)));
+  const int64_t nn = (int64_t)np * np;
+  const int b = blockIdx.y, tid = threadIdx.x;
+  W += nn * b;
+  U += nn * b;
+  const int k0 = kb * CH_NB, n0 = k0 + CH_NB * (int)blockIdx.x;
+  // this workgroup's columns of the block row, in flight during the elimination
+  if (blockIdx.x > 0) {
+    for (int e = tid; e < CH_NB * CH_NB; e += 256) {
+      const int kk = e % CH_NB, nn_ = e / CH_NB;
+      const cplx v = W[(k0 + kk) + (int64_t)np * (n0 + nn_)];
+      Br[kk][nn_] = v.x;
+      Bi[kk][nn_] = v.y;
+    }
+  }
+  // thread (r, c) owns rows r + 16 x and columns c + 16 y; the lower triangle from the upper one
+  const int r = tid & 15, c = tid >> 4;
+  cplx a[4][4];
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      const int i = r + 16 * x, j = c + 16 * y;
+      const cplx v = W[(k0 + (i < j ? i : j)) + (int64_t)np * (k0 + (i < j ? j : i))];
+      a[x][y] = i < j ? v : (i == j ? mk(v.x, 0.0) : cconj(v));
+    }
+  if (r == 0)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) rowb[0][c + 16 * y] = a[0][y];
+  if (c == 0)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) colb[0][r + 16 * x] = a[x][0];
+  __syncthreads();
+  bool ok = true;
+  // elimination of column j from the rows below it, the multipliers taking its place: the strict
+  // lower triangle becomes the inverse of the unit factor, the diagonal keeps the pivots
+#pragma unroll
+  for (int xj = 0; xj < 4; ++xj) {
+    for (int jr = 0; jr < 16; ++jr) {
+      const int j = 16 * xj + jr, par = j & 1;
+      double piv = rowb[par][j].x;
+      if (!(piv > 0.0)) {
+        ok = false;
+        piv = 1.0;
+      }
+      const double ip = 1.0 / piv;
+      cplx rw[4];
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        rw[y] = rowb[par][c + 16 * y];
+        if (c + 16 * y == j) rw[y] = mk(1.0, 0.0);   // a_ij - m 1 after a_ij is dropped below: -m
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int i = r + 16 * x;
+        if (i > j) {
+          const cplx m = cscale(colb[par][i], ip);
+#pragma unroll
+          for (int y = 0; y < 4; ++y) {
+            cplx v = c + 16 * y == j ? mk(0.0, 0.0) : a[x][y];
+            a[x][y] = csub(v, cmul(m, rw[y]));
+          }
+        }
+      }
+      // publish row and column j + 1 (static register indices: the next block of 16 at jr = 15)
+      const int q = (j + 1) & 15;
+      if (jr < 15) {
+        if (r == q)
+#pragma unroll
+          for (int y = 0; y < 4; ++y) rowb[par ^ 1][c + 16 * y] = a[xj][y];
+        if (c == q)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) colb[par ^ 1][r + 16 * x] = a[x][xj];
+      } else if (xj < 3) {
+        if (r == 0)
+#pragma unroll
+          for (int y = 0; y < 4; ++y) rowb[par ^ 1][c + 16 * y] = a[xj < 3 ? xj + 1 : 3][y];
+        if (c == 0)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) colb[par ^ 1][r + 16 * x] = a[x][xj < 3 ? xj + 1 : 3];
+      }
+      __syncthreads();
+    }
+  }
+  if (!ok && tid == 0 && blockIdx.x == 0) flag[b] = 1;
+  // row i of the inverse factor: the unit inverse's row over the square root of its pivot
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+      if (r + 16 * x == c + 16 * y) colb[0][r + 16 * x] = a[x][y];
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const int i = r + 16 * x;
+    const double pv = colb[0][i].x;
+    const double s = 1.0 / sqrt(pv > 0.0 ? pv : 1.0);
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      const int j = c + 16 * y;
+      const cplx v = i > j ? cscale(a[x][y], s) : mk(i == j ? s : 0.0, 0.0);
+      Ar[j][i] = v.x;   // [k][m]
+      Ai[j][i] = v.y;
+      if (blockIdx.x == 0 && b == 0) Li[(k0 + i) + (int64_t)np * (k0 + j)] = v;
+    }
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) return;
+  // U[k0 + m, n0 + n] = sum_k Linv[m][k] W[k0 + k, n0 + n]
+  const int lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+  d4 accr[2][2], acci[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      accr[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+      acci[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+    }
+  for (int kk = 0; kk < CH_NB; kk += 4) {
+    const int kl = kk + (lane >> 4);
+    double ar[2], ai[2], br[2], bi[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      ar[x] = Ar[kl][wm + 16 * x + (lane & 15)];
+      ai[x] = Ai[kl][wm + 16 * x + (lane & 15)];
+      br[x] = Br[kl][wn + 16 * x + (lane & 15)];
+      bi[x] = Bi[kl][wn + 16 * x + (lane & 15)];
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        accr[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[x], br[y], accr[x][y], 0, 0, 0);
+        accr[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai[x], bi[y], accr[x][y], 0, 0, 0);
+        acci[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[x], bi[y], acci[x][y], 0, 0, 0);
+        acci[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[x], br[y], acci[x][y], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int row = wm + 16 * x + (lane >> 4) + 4 * q, col = wn + 16 * y + (lane & 15);
+        U[(k0 + row) + (int64_t)np * (n0 + col)] = mk(accr[x][y][q], acci[x][y][q]);
+      }
+}
+
+// Lanczos on S^-1 = L^-H L^-1: w = S^-1 v_j is given; alpha_j, the next vector and beta_j.
+// One workgroup; n <= 1024 * LZ_E.
+constexpr int LZ_T = 1024, LZ_E = 2, LZ_STEPS = 256;
+__global__ __launch_bounds__(LZ_T) void k_lanczos(int n, int j, const cplx* __restrict__ w, cplx* __restrict__ v,
+                                                  cplx* __restrict__ vold, double* __restrict__ ab) {
+  __shared__ double red[16];
+  auto sum = [&](double x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+    __syncthreads();
+    double t = 0.0;
+    for (int q = 0; q < 16; ++q) t += red[q];
+    return t;
+  };
+  cplx wv[LZ_E], vv[LZ_E];
+  const double bo = j > 0 ? ab[2 * (j - 1) + 1] : 0.0;
+  double a = 0.0;
+#pragma unroll
+  for (int e = 0; e < LZ_E; ++e) {
+    const int i = threadIdx.x + LZ_T * e;
+    wv[e] = vv[e] = mk(0.0, 0.0);
+    if (i < n) {
+      vv[e] = v[i];
+      wv[e] = w[i];
+      if (j > 0) {
+        const cplx o = vold[i];
+        wv[e] = mk(wv[e].x - bo * o.x, wv[e].y - bo * o.y);
+      }
+    }
+    a += vv[e].x * wv[e].x + vv[e].y * wv[e].y;
+  }
+  a = sum(a);
+  double b2 = 0.0;
+#pragma unroll
+  for (int e = 0; e < LZ_E; ++e) {
+    wv[e] = mk(wv[e].x - a * vv[e].x, wv[e].y - a * vv[e].y);
+    b2 += cabs2(wv[e]);
+  }
+  const double b = sqrt(sum(b2)), ib = b > 0.0 ? 1.0 / b : 0.0;
+#pragma unroll
+  for (int e = 0; e < LZ_E; ++e) {
+    const int i = threadIdx.x + LZ_T * e;
+    if (i < n) {
+      vold[i] = vv[e];
+      v[i] = cscale(wv[e], ib);
+    }
+  }
+  if (threadIdx.x == 0) {
+    ab[2 * j] = a;
+    ab[2 * j + 1] = b;
+  }
+}
+
+// a start vector with a part along every direction: unit-modulus entries of an integer hash
+__global__ void k_lanczos_start(int n, cplx* __restrict__ v) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  uint64_t z = 0x9E3779B97F4A7C15ull * (uint64_t)(i + 1);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z ^= z >> 27;
+  double sn, cs;
+  sincospi(2.0 * (double)(z >> 11) * 0x1.0p-53, &sn, &cs);
+  const double s = 1.0 / sqrt((double)n);
+  v[i] = mk(cs * s, sn * s);
+}
+
+}  // namespace
+
+int64_t chol_np(int64_t n) { return (n + CH_NB - 1) / CH_NB * CH_NB; }
+int64_t chol_work_elems(int64_t n) { return 4 * chol_np(n) * chol_np(n); }
+
+void chol_inverse(hipStream_t s, int64_t n, const cplx* S, int64_t lds, double sigma, cplx* work, cplx* Li, int* flags) {
+  const int64_t np = chol_np(n), nn = np * np;
+  DC2_CHECK(n >= 1 && n <= 4096, 1, "chol_inverse: n must be in 1..4096");
+  const int nb = (int)(np / CH_NB);
+  cplx* W = work;
+  cplx* U = W + 2 * nn;
+  const cplx one = mk(1.0, 0.0), mone = mk(-1.0, 0.0), zero = mk(0.0, 0.0);
+  DC2_HIP(hipMemsetAsync(flags, 0, 2 * sizeof(int), s));
+  hipLaunchKernelGGL(k_chol_pack, dim3(cdiv(nn, 256)), dim3(256), 0, s, (int)n, (int)np, S, lds, sigma, W);
+  fill_zero(s, Li, nn);
+  for (int kb = 0; kb < nb; ++kb) {
+    hipLaunchKernelGGL(k_chol_step, dim3(nb - kb, 2), dim3(256), 0, s, (int)np, kb, W, U, Li, flags);
+    const int64_t k0 = (int64_t)kb * CH_NB, k1 = k0 + CH_NB;
+    zherk_trailing(s, np - k1, CH_NB, U + k0 + np * k1, np, nn, W + k1 + np * k1, np, nn, 2);
+  }
+  DC2_HIP(hipGetLastError());
+  // merges of neighbouring blocks (sizes in units of CH_NB): blocks of b, the last one shorter;
+  // T (the first half of W) holds Z U12^H
+  for (int64_t b = 1; b < nb; b *= 2) {
+    const int64_t pairs = nb / (2 * b), step = 2 * b * CH_NB, h = b * CH_NB;
+    if (pairs > 0) {
+      zgemm(s, 'N', 'C', h, h, h, one, Li + h + np * h, np, step * (np + 1), U + np * h, np, step * (np + 1), zero, W, h,
+            h * h, pairs);
+      zgemm(s, 'N', 'N', h, h, h, mone, W, h, h * h, Li, np, step * (np + 1), zero, Li + h, np, step * (np + 1), pairs);
+    }
+    const int64_t rest = nb - 2 * b * pairs;   // a full block and a shorter one remain
+    if (rest > b) {
+      const int64_t o = pairs * step, t = (rest - b) * CH_NB;
+      zgemm(s, 'N', 'C', t, h, t, one, Li + (o + h) * (np + 1), np, 0, U + o + np * (o + h), np, 0, zero, W, t, 0, 1);
+      zgemm(s, 'N', 'N', t, h, h, mone, W, t, 0, Li + o * (np + 1), np, 0, zero, Li + (o + h) + np * o, np, 0, 1);
+    }
+  }
+}
+
+bool chol_lambda_min(hipStream_t s, int64_t n, const cplx* Li, cplx* work, double* host, double& lambda) {
+  const int64_t np = chol_np(n);
+  DC2_CHECK(n >= 1 && n <= (int64_t)LZ_T * LZ_E, 1, "chol_lambda_min: n must be in 1..2048");
+  cplx *v = work, *vold = v + n, *t = vold + n, *w = t + n;
+  double* ab = reinterpret_cast<double*>(w + n);
+  const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
+  hipLaunchKernelGGL(k_lanczos_start, dim3(cdiv(n, 256)), dim3(256), 0, s, (int)n, v);
+  const int steps = (int)std::min<int64_t>(n, LZ_STEPS);
+  for (int j = 0, seen = 0; j < steps;) {
+    const int stop = std::min(steps, j + 32);
+    for (; j < stop; ++j) {
+      zgemm(s, 'N', 'N', n, 1, n, one, Li, np, 0, v, n, 0, zero, t, n, 0, 1);
+      zgemm(s, 'C', 'N', n, 1, n, one, Li, np, 0, t, n, 0, zero, w, n, 0, 1);
+      hipLaunchKernelGGL(k_lanczos, dim3(1), dim3(LZ_T), 0, s, (int)n, j, w, v, vold, ab);
+    }
+    DC2_HIP(hipGetLastError());
+    DC2_HIP(hipMemcpyAsync(host + 2 * seen, ab + 2 * seen, 2 * (j - seen) * sizeof(double), hipMemcpyDeviceToHost, s));
+    DC2_HIP(hipStreamSynchronize(s));
+    seen = j;
+    // the largest eigenvalue theta of the tridiagonal by bisection on its Sturm count, and the
+    // last component of its eigenvector by the three-term recurrence from the end
+    double hi = 0.0;
+    for (int i = 0; i < j; ++i)
+      hi = std::max(hi, host[2 * i] + (i ? host[2 * i - 1] : 0.0) + (i + 1 < j ? host[2 * i + 1] : 0.0));
+    if (!(hi > 0.0 && hi < 1e300)) return false;
+    double lo = 0.0;
+    for (int k = 0; k < 200 && hi - lo > 4e-16 * hi; ++k) {
+      const double mid = 0.5 * (lo + hi);
+      bool above = false;   // some eigenvalue > mid: a positive pivot of T - mid
+      double d = 1.0;
+      for (int i = 0; i < j && !above; ++i) {
+        const double b = i ? host[2 * i - 1] : 0.0;
+        d = host[2 * i] - mid - (i ? b * b / d : 0.0);
+        above = d >= 0.0;
+      }
+      (above ? lo : hi) = mid;
+    }
+    const double theta = hi;
+    double sq = 1.0, x = 1.0, xn = 0.0;   // x_{j-1} = 1, going down
+    for (int i = j - 1; i > 0; --i) {
+      const double b = host[2 * i - 1];
+      if (!(b > 0.0)) break;   // an invariant subspace: the rest does not couple
+      const double xp = ((theta - host[2 * i]) * x - (i + 1 < j ? host[2 * i + 1] : 0.0) * xn) / b;
+      xn = x;
+      x = xp;
+      sq += x * x;
+      if (sq > 1e280) break;
+    }
+    // residual of the Ritz pair against theta; the eigenvalue's error is its square over the gap
+    if (host[2 * j - 1] <= 1e-7 * theta * std::sqrt(sq)) {
+      lambda = 1.0 / theta;
+      return true;
+    }
+  }
+  return false;
+}
+
 }  // namespace dc2

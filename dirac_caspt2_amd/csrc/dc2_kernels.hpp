@@ -85,6 +85,7 @@ void build_phi_adj(hipStream_t s, int na, int ne, int64_t nf, const int* rank_fu
                    const double* eps_act, int64_t m, int64_t* strings, int64_t nred, const int* tup, cplx* Psi,
                    cplx* Psif);
 void scale_rows(hipStream_t s, int64_t m, int64_t ncol, const double* f, const cplx* in, cplx* out);
+void scale_cols(hipStream_t s, int64_t m, int64_t ncol, const double* f, const cplx* in, cplx* out);
 // block Davidson helpers: diagonal of H, unit start vectors e_rows[j], Ritz residuals
 // R = AX - X diag(theta), diagonal preconditioner T[:, c] = R[:, sel_c] / (theta_sel_c - d)
 void davidson_diag(hipStream_t s, int64_t n, const cplx* H, double* d);
@@ -166,6 +167,17 @@ int64_t cg_max_n();
 int64_t cg_work_bytes(int64_t n, int64_t npert);
 bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const cplx* Y, const double* alpha,
                   void* work, int* host2, double* partial, double* out2, int* iterations = nullptr);
+
+// Li (chol_np(n) squared, leading dimension chol_np(n)) = L^-1 of the Hermitian S = L L^H (upper
+// triangle read), lower triangular with the unit matrix past n; flags[0] is set when S, flags[1]
+// when S - sigma I is not positive definite (two ints of device memory).  work:
+// chol_work_elems(n) complex elements; asynchronous on s.
+int64_t chol_np(int64_t n);
+int64_t chol_work_elems(int64_t n);
+void chol_inverse(hipStream_t s, int64_t n, const cplx* S, int64_t lds, double sigma, cplx* work, cplx* Li, int* flags);
+// the smallest eigenvalue of S from Li by Lanczos on S^-1 (n <= 2048); false when it did not
+// converge.  work: 4 n + 256 complex elements; host: 512 doubles of page-locked memory.
+bool chol_lambda_min(hipStream_t s, int64_t n, const cplx* Li, cplx* work, double* host, double& lambda);
 
 // ---------------------------------------------------------------- dc2_pt2.hip
 struct Dens {

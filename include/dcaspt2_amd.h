@@ -141,6 +141,13 @@ int dc2_cdiag(dc2_context* ctx, double* c, int32_t n, int32_t* dimm, double* w, 
  * definite or a column did not converge, and out2 is not set */
 int dc2_resolvent_energy(dc2_context* ctx, int32_t n, int64_t npert, const double* b, const double* y,
                          const double* alpha, double* out2, int32_t* iterations);
+/* a metric of whole rank without its eigenvectors: S = L L^H (n x n complex Hermitian, host,
+ * upper triangle read, n <= 2048), linv = L^-1 (lower triangular) and btilde = L^-1 B L^-H, the
+ * counterpart of cdiag + ulambda_s_half + transform (solve_A_subspace.F90:150-200) when every
+ * eigenvalue of S is above sigma.  *whole_rank: 1 when it is (linv, btilde and *lambda_min, the
+ * smallest eigenvalue, are set), 0 when some eigenvalue is not (nothing is set) */
+int dc2_whiten(dc2_context* ctx, int32_t n, const double* s, const double* b, double sigma, double* linv,
+               double* btilde, double* lambda_min, int32_t* whole_rank);
 /* C = alpha op(A) op(B) + beta C on device memory, batched by strides;
  * opA in 'N','T','C'; opB in 'N','R' (conjugate, no transpose),'T','C' */
 int dc2_zgemm(dc2_context* ctx, char opA, char opB, int64_t M, int64_t N, int64_t K, const double* alpha,
