@@ -1084,7 +1084,6 @@ GramMetric gram_eig(dc2_context* c, Lane& L, char X, int64_t n, const cplx* Y, c
   const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
   int64_t* strings = L.l(nm("_strings").c_str(), m);
   cplx* Phi = L.z(nm("_Phi").c_str(), m * n);
-  cplx* G = L.z(nm("_G").c_str(), m * m);
   double* f = L.d(nm("_f").c_str(), m);
   double* lam = L.d(nm("_lam").c_str(), m);
   build_phi(s, na, c->ne, create, c->nfull, c->rank_full.get(), Y, eps_act, m, strings, Phi, f);
@@ -1123,6 +1122,7 @@ GramMetric gram_eig(dc2_context* c, Lane& L, char X, int64_t n, const cplx* Y, c
     g.margin = std::min(g.margin, thr);   // the m - nred eigenvalues of G that vanish identically
     g.dimm = count_retained(L, nred, lt, g.margin);
     const int64_t nd = m - g.dimm;
+    cplx* G = L.z(nm("_G").c_str(), m * m);
     fill_zero(s, G, m * nd);
     if (nd > 0) DC2_HIP(hipMemsetAsync(lam, 0, nd * sizeof(double), s));
     if (g.dimm > 0) {
@@ -1133,6 +1133,7 @@ GramMetric gram_eig(dc2_context* c, Lane& L, char X, int64_t n, const cplx* Y, c
     }
     return g;
   }
+  cplx* G = L.z(nm("_G").c_str(), m * m);
   zherk_upper(s, m, n, Phi, m, G, m);   // Hermitian: the upper tiles only
   check_finite(c, s, "Phi Phi^H", G, m * m);
   zheevd(c, L, (int)m, G, lam, "a determinant-space metric", ras ? EigKind::rank_deficient : EigKind::general);
@@ -1240,10 +1241,10 @@ SolveOut solve_block_gram(dc2_context* c, Lane& L, char X, const GramMetric& g, 
   if (m == 0 || dimm == 0 || npert == 0) return r;
   const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
   const cplx* Phi = L.z(nm("_Phi").c_str(), m * n);
-  cplx* G = L.z(nm("_G").c_str(), m * m);
   const double* f = L.d(nm("_f").c_str(), m);
   const int64_t nd = m - dimm;
-  const cplx* Gk = G + m * nd;
+  cplx* G = g.chol ? nullptr : L.z(nm("_G").c_str(), m * m);   // chol: only B~ and Y are used
+  const cplx* Gk = g.chol ? nullptr : G + m * nd;
   cplx* Y = L.z(nm("_Y").c_str(), dimm * npert);
   if (g.thin) {
     // (U L^-1/2)^H V = L^-1/2 t^H (M M^T)^(-1/2) M V in the thin factor's space (no division
@@ -1334,7 +1335,10 @@ AcRoute ac_route_of(const dc2_context* c, char X) {
     else r.gram = true;
   } else if (c->ac_route == 0) {
     if (X == 'A' && nred < mdet && nred < n) r.reduced = r.phi = true;
-    else r.gram = mdet < n;
+    // C also with more strings than formula rows, when its thin factor is within this library's
+    // eigensolver: 14 spinors with 7 electrons (3003 strings, 2744 rows, 1274 thin) spent 181 of
+    // 205 ms in rocSOLVER on the 2744 x 2744 formula matrices and 13 in the 3-RDM they need
+    else r.gram = mdet < n || (nred <= 2048 && gram_thin(c, X, mdet));
   }
   return r;
 }

@@ -239,7 +239,7 @@ int64_t footprint_bytes(int64_t ni, int64_t na, int64_t ns, int64_t ne) {
   const int64_t dens = 4 * nf * na2 + nf * na2 * na2 + 6 * na3 * na3;
   const int64_t nr = na2 * (na - 1) / 2;   // A and C by their Cholesky factors (5 + 1 matrices each)
   const int64_t ac = 2 * (std::min(mA, na3) * na3 + 2 * std::min(mA, na3) * std::min(mA, na3)) +
-                     na3 * (ni + ns) * 3 + (nr < mA ? 6 * nr * nr : 0);
+                     na3 * (ni + ns) * 3 + (nr < mA ? 6 * nr * nr : 0) + (nr <= 2048 && mC > na3 ? mC * na3 : 0);
   const int64_t other = 8 * (ns + ni) * (ns + ni) + 4 * ns * ns * ni + 4 * ns * ni * ni * na;
   return 2 * (z * (tb + mx + ci + dens + ac + other) + (64ll << 20));
 }

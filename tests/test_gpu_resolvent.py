@@ -80,3 +80,24 @@ def test_energy_against_eigenvectors(metric, lanes, eshift):
         assert abs(a.e2[X] - b.e2[X]) < 1e-11 * scale, X
         assert abs(a.sumc2[X] - b.sumc2[X]) < 1e-11 * scale, X
     assert a.info == b.info
+
+
+def test_thin_c_with_more_strings_than_rows():
+    """14 spinors with 7 electrons: C(14, 6) = 3003 strings against 14^3 = 2744 formula rows and
+    1274 of the thin factor.  The two metrics weight the weakest directions differently by
+    rounding (eps / 1e-8 of them): the 1e-9 Eh of the oracle comparisons."""
+    from dirac_caspt2_amd import synth
+    from gpu_helpers import context_from_synth, say
+    say("thin C, 14 spinors with 7 electrons")
+    sp = synth.generate(synth.SynthSpec(ninact=4, nact=14, nsec=20, nelec=7, seed=20300))
+    out = []
+    for metric in ("auto", "formula"):
+        with context_from_synth(sp) as c:
+            c.set_option("ac_metric", metric)
+            c.casci(2)
+            out.append(c.caspt2(1, 0.0))
+    a, b = out
+    for X in "ABCDEFGH":
+        assert abs(a.e2[X] - b.e2[X]) < 1e-9, X
+        assert abs(a.sumc2[X] - b.sumc2[X]) < 1e-9, X
+    assert a.info == b.info
