@@ -430,7 +430,7 @@ def hetrd_roofline(ctx, ht, steps, workload):
 
 def gemm_accounting(ctx, step, workload, nsteps):
     """Per-launch GEMM accounting (two HIP events per launch; Davidson graphs off) over extra
-    untimed steps: the dominant k_zgemm2 instantiation and the all-GEMM rate."""
+    untimed steps: the dominant k_zgemm instantiation and the all-GEMM rate."""
     ctx.set_profiling(True)
     for _ in range(nsteps):
         step()
@@ -441,7 +441,7 @@ def gemm_accounting(ctx, step, workload, nsteps):
     ctx.set_profiling(False)
     dom_op, dom = max(ops.items(), key=lambda kv: kv[1]["seconds"])
     ach = dom["flops"] / dom["seconds"] / 1e12 if dom["seconds"] > 0 else 0.0
-    return {"kernel": f"k_zgemm2<'{dom_op[0]}','{dom_op[1]}',16,1> (MFMA FP64 complex GEMM)",
+    return {"kernel": f"k_zgemm<'{dom_op[0]}','{dom_op[1]}',...> (MFMA FP64 complex GEMM)",
             "bound": "mfma", "achieved": ach, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
             "frac": ach / PEAK_FP64_TFLOPS, "traffic": measured_traffic(workload, "k_zgemm", dom_op),
             "launches_per_step": dom["launches"] / nsteps,

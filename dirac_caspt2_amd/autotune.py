@@ -1,5 +1,5 @@
 """GEMM autotuner of the library: the distinct MFMA complex-GEMM shapes of a workload are
-recorded while it runs once, every kernel variant (K tile 16/32 x LDS row padding 1/16)
+recorded while it runs once, every kernel variant (columns per workgroup and K tile)
 and split-K factor is timed on each shape (dc2_gemm_tune), and the fastest choice that
 beats the built-in rule is installed in the library's process-wide table, which the GEMM
 dispatch consults for products of exactly that shape.  A table can be saved as JSON and

@@ -130,8 +130,8 @@ void zherk_trailing(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t 
 // C = L B L^H for Hermitian B and lower triangular L (zeros above its diagonal); T: n x n scratch
 void zgemm_congruence(hipStream_t s, int64_t n, const cplx* L, int64_t ldl, const cplx* B, int64_t ldb, cplx* T,
                       cplx* C, int64_t ldc);
-// GEMM tuning table (exact shapes): the MFMA kernel variant (1..4: K tile 16/32 x LDS padding
-// 1/16) and split-K factor (1: none) chosen for (opA, opB, M, N, K, batch) by measurement.
+// GEMM tuning table (exact shapes): the MFMA kernel variant (1..4: 64, 32, 16 or 16 columns per
+// workgroup with K tiles of 8, 16, 16 or 8) and split-K factor (1: none) chosen for (opA, opB, M, N, K, batch) by measurement.
 // gemm_tune times every candidate on scratch operands on stream s and installs the fastest;
 // out: {best variant, best split, best seconds, seconds of the built-in choice}.
 void gemm_tune(hipStream_t s, char opA, char opB, int64_t M, int64_t N, int64_t K, int64_t batch, int reps,

@@ -1,10 +1,8 @@
 // Complex FP64 GEMM on CDNA4 matrix cores (v_mfma_f64_16x16x4f64).
 //
-// One workgroup = 4 wave64s computing a 64x64 complex tile of C; every wave
-// owns a 32x32 sub-tile = 2x2 MFMA tiles of 16x16.  A complex multiply-add is
-// four real MFMAs on separate real/imaginary planes staged in LDS.
-// The LDS row stride (80 doubles) puts the four k-rows read by one wave in
-// disjoint bank halves.
+// One workgroup = 4 wave64s along m, each with 16 rows and up to 64 columns of complex C in
+// 16x16 MFMA tiles; a complex multiply-add is four real MFMAs.  Operands go through
+// double-buffered LDS as complex numbers.
 //
 // Used for: the four one-index integral transforms (module_intra.F90), the
 // RDM contractions (density_matrix.F90), the V contractions and the
@@ -27,234 +25,235 @@ namespace dc2 {
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 namespace {
-constexpr int BM = 64, BN = 64, BK = 16, LDS_STRIDE = 80;
+constexpr int64_t kLd32 = 1ll << 22;   // below it the byte offsets within a tile fit 32 bits (63 ld 16 < 2^32)
+constexpr int BM = 64, BK = 16;   // rows of an output tile; granule of the split-K chunks
 
-template <char OPA>
-__device__ inline cplx loadA(const cplx* __restrict__ A, int64_t lda, int64_t m, int64_t k) {
-  if (OPA == 'N') return A[m + lda * k];
-  cplx v = A[k + lda * m];
-  return OPA == 'C' ? cconj(v) : v;
-}
-
-template <char OPB>
-__device__ inline cplx loadB(const cplx* __restrict__ B, int64_t ldb, int64_t k, int64_t n) {
-  if (OPB == 'N') return B[k + ldb * n];
-  if (OPB == 'R') return cconj(B[k + ldb * n]);
-  cplx v = B[n + ldb * k];
-  return OPB == 'C' ? cconj(v) : v;
-}
-
-// blockIdx.z = batch index * sk + K-split index; split kz covers K in [kz*kchunk, (kz+1)*kchunk)
-// and writes its partial product to C + kz * sC (the split-K workspace) when sk > 1.
-template <char OPA, char OPB>
-__global__ __launch_bounds__(256) void k_zgemm(int64_t M, int64_t N, int64_t Kfull, cplx alpha,
-                                               const cplx* __restrict__ A, int64_t lda, int64_t sA,
-                                               const cplx* __restrict__ B, int64_t ldb, int64_t sB,
-                                               cplx beta, cplx* __restrict__ C, int64_t ldc, int64_t sC, int sk,
-                                               int64_t kchunk) {
-  __shared__ double Ar[BK][LDS_STRIDE], Ai[BK][LDS_STRIDE], Br[BK][LDS_STRIDE], Bi[BK][LDS_STRIDE];
-  const int64_t bz = blockIdx.z / sk, kz = blockIdx.z % sk;
-  A += bz * sA;
-  B += bz * sB;
-  C += (sk > 1 ? bz * sk + kz : bz) * sC;   // split K: partial kz of product bz
-  const int64_t kbeg = kz * kchunk;
-  const int64_t K = (kbeg + kchunk < Kfull) ? kbeg + kchunk : Kfull;   // loop end
-  const int64_t m0 = (int64_t)blockIdx.x * BM, n0 = (int64_t)blockIdx.y * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  d4 accr[2][2], acci[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      accr[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-      acci[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-    }
-
-  for (int64_t k0 = kbeg; k0 < K; k0 += BK) {
-    // stage A (BM x BK) and B (BK x BN) tiles; the index order follows the
-    // contiguous direction of the operand in memory
-#pragma unroll
-    for (int e = tid; e < BM * BK; e += 256) {
-      int mm, kk;
-      if (OPA == 'N') { mm = e % BM; kk = e / BM; }
-      else { kk = e % BK; mm = e / BK; }
-      const int64_t gm = m0 + mm, gk = k0 + kk;
-      cplx v = (gm < M && gk < K) ? loadA<OPA>(A, lda, gm, gk) : mk(0.0, 0.0);
-      Ar[kk][mm] = v.x;
-      Ai[kk][mm] = v.y;
-    }
-#pragma unroll
-    for (int e = tid; e < BN * BK; e += 256) {
-      int nn, kk;
-      if (OPB == 'N' || OPB == 'R') { kk = e % BK; nn = e / BK; }
-      else { nn = e % BN; kk = e / BN; }
-      const int64_t gn = n0 + nn, gk = k0 + kk;
-      cplx v = (gn < N && gk < K) ? loadB<OPB>(B, ldb, gk, gn) : mk(0.0, 0.0);
-      Br[kk][nn] = v.x;
-      Bi[kk][nn] = v.y;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      const int kl = kk + (lane >> 4);
-      double ar[2], ai[2], br[2], bi[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        ar[i] = Ar[kl][wm + 16 * i + (lane & 15)];
-        ai[i] = Ai[kl][wm + 16 * i + (lane & 15)];
-        br[i] = Br[kl][wn + 16 * i + (lane & 15)];
-        bi[i] = Bi[kl][wn + 16 * i + (lane & 15)];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          accr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], br[j], accr[i][j], 0, 0, 0);
-          accr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai[i], bi[j], accr[i][j], 0, 0, 0);
-          acci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], bi[j], acci[i][j], 0, 0, 0);
-          acci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], br[j], acci[i][j], 0, 0, 0);
-        }
-    }
-    __syncthreads();
-  }
-  // D[row][col] of a 16x16 MFMA tile sits in element (row / 4) of lane col + 16 * (row % 4)
-  // (measured on gfx950 with a one-hot probe of __builtin_amdgcn_mfma_f64_16x16x4f64)
-  const bool beta_zero = (beta.x == 0.0 && beta.y == 0.0);
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t row = m0 + wm + 16 * i + (lane >> 4) + 4 * r;
-        const int64_t col = n0 + wn + 16 * j + (lane & 15);
-        if (row < M && col < N) {
-          cplx acc = mk(accr[i][j][r], acci[i][j][r]);
-          cplx out = cmul(alpha, acc);
-          if (!beta_zero) cfma(out, beta, C[row + ldc * col]);
-          C[row + ldc * col] = out;
-        }
-      }
-}
-
-// Software-pipelined variant: the next K tile is fetched from global memory into registers
-// while the current one is multiplied out of LDS, so load latency hides behind the MFMAs.
-// KB: K per tile (16 or 32); PAD: LDS row padding in doubles (bank spread of the
-// transposed-operand stores and of the MFMA operand reads).
-// UPPER: only the tiles that reach the upper triangle (a Hermitian product; the tiles
-// entirely below the diagonal leave at once)
 // tri: zeros the operands are known to have, which end a tile's K loop early: TRI_A op(A) lower
 // triangular (k <= m), TRI_B op(B) upper triangular (k <= n)
 enum { TRI_NONE = 0, TRI_A = 1, TRI_B = 2 };
-template <char OPA, char OPB, int KB, int PAD, bool UPPER = false>
-__global__ __launch_bounds__(256) void k_zgemm2(int64_t M, int64_t N, int64_t Kfull, cplx alpha,
-                                                const cplx* __restrict__ A, int64_t lda, int64_t sA,
-                                                const cplx* __restrict__ B, int64_t ldb, int64_t sB,
-                                                cplx beta, cplx* __restrict__ C, int64_t ldc, int64_t sC, int sk,
-                                                int64_t kchunk, int tri = TRI_NONE) {
-  int64_t mt, nt;
-  xcd_tile(gridDim.x, gridDim.y, blockIdx.x, blockIdx.y, mt, nt);
-  if (UPPER && mt * BM > nt * BN + BN - 1) return;   // uniform
-  constexpr int LS = BM + PAD;               // BM == BN
-  constexpr int NE = BM * KB / 256;          // elements of each operand tile per thread
-  __shared__ double Ar[KB][LS], Ai[KB][LS], Br[KB][LS], Bi[KB][LS];
-  const int64_t bz = blockIdx.z / sk, kz = blockIdx.z % sk;
-  A += bz * sA;
-  B += bz * sB;
-  C += (sk > 1 ? bz * sk + kz : bz) * sC;   // split K: partial kz of product bz
-  const int64_t kbeg = kz * kchunk;
-  int64_t kend = (kbeg + kchunk < Kfull) ? kbeg + kchunk : Kfull;
-  if (tri == TRI_A && kend > (mt + 1) * BM) kend = (mt + 1) * BM;
-  if (tri == TRI_B && kend > (nt + 1) * BN) kend = (nt + 1) * BN;
-  const int64_t m0 = mt * BM, n0 = nt * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  d4 accr[2][2], acci[2][2];
+// k_zgemm: one workgroup = 4 waves along m, each with FN fragments of 16 x 16 (a tile of 64 x
+// 16 FN), K in tiles of KB through double-buffered LDS, one workgroup barrier per K tile.
+//
+// What bounds it: the FP64 matrix units, and every vector instruction beside them (at 0.9
+// others per product the units were busy 84% of the time, at 0.24-0.49 94-96%).  So the loop
+// over full K tiles has no branch and no edge test: it runs in rounds of two tiles (constant
+// LDS offsets), offsets are formed once, rows and columns past the edges are read from the
+// last valid one (their outputs are never stored), and the partial K tile at the end has its
+// own code, zeroed in both operands and multiplied up to its last group of four.  A column
+// tile at the edge multiplies only the fragments that hold columns (zg_loop exists for every
+// count).  The next tile's loads are issued before the current one is multiplied, and stored to
+// the other buffer after it.  __launch_bounds__(256, 2): with the whole register file to itself
+// the compiler kept the accumulators in AGPRs and moved all of them to VGPRs and back per tile.
+//
+// Measured against the kernel it replaces (64 x 64 tiles, single-buffered planes): 252000 x 280
+// x 280 'T','N' 3170 -> 2250 us (70 TF/s), 41984 x 164 x 164 238 -> 153, 2352000 x 30 x 30
+// 870 -> 523, 322752 x 14 x 14 72 -> 26 (5.6 TB/s), 1274^3 'C','N' 410 -> 300, 2048^3 1190 -> 970.
+template <char OPA, char OPB, int FN, int KB>
+struct ZgTile {
+  static constexpr int TM = BM, TN = 16 * FN;
+  static constexpr bool AK = OPA != 'N', BKc = OPB == 'N' || OPB == 'R';   // contiguous along k
+  static constexpr int NA = TM * KB / 256, NB = (TN * KB + 255) / 256;
+  // rows of LDS padded by one element: 2.8 conflict cycles per LDS instruction, against 17 with
+  // none, 5 with two and 10 with four (counters, 'T','N')
+  static constexpr int LA = TM + 1, LB = TN + 1;
+};
+
+// the part of the kernel that depends on the number F of fragments with valid columns
+template <char OPA, char OPB, int FN, int KB, int F, class OFF>
+__device__ __forceinline__ void zg_loop(const cplx* __restrict__ At, const cplx* __restrict__ Bt, int64_t lda, int64_t ldb,
+                                        int mrem, int nrem, int ktot, cplx* __restrict__ As, cplx* __restrict__ Bs,
+                                        d4 (&accr)[FN], d4 (&acci)[FN]) {
+  using T = ZgTile<OPA, OPB, FN, KB>;
+  constexpr int TM = T::TM, TN = T::TN, NA = T::NA, NB = T::NB, LA = T::LA, LB = T::LB;
+  constexpr bool AK = T::AK, BKc = T::BKc;
+  const int tid = threadIdx.x, lane = tid & 63, wm = (tid >> 6) * 16;
+  const int64_t stepA = AK ? KB : lda * KB, stepB = BKc ? KB : ldb * KB;
+  cplx ra[NA], rb[NB];
+  OFF oa[NA], ob[NB];   // byte offsets within a tile
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      accr[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-      acci[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-    }
-  cplx ra[NE], rb[NE];
-  auto gload = [&](int64_t k0) {
-#pragma unroll
-    for (int r = 0; r < NE; ++r) {
-      const int e = tid + 256 * r;
-      int mm, kk, nn, kb;
-      if (OPA == 'N') { mm = e % BM; kk = e / BM; } else { kk = e % KB; mm = e / KB; }
-      if (OPB == 'N' || OPB == 'R') { kb = e % KB; nn = e / KB; } else { nn = e % BN; kb = e / BN; }
-      const int64_t gm = m0 + mm, gk = k0 + kk, gn = n0 + nn, gkb = k0 + kb;
-      ra[r] = (gm < M && gk < kend) ? loadA<OPA>(A, lda, gm, gk) : mk(0.0, 0.0);
-      rb[r] = (gn < N && gkb < kend) ? loadB<OPB>(B, ldb, gkb, gn) : mk(0.0, 0.0);
-    }
-  };
-  auto sstore = [&]() {
-#pragma unroll
-    for (int r = 0; r < NE; ++r) {
-      const int e = tid + 256 * r;
-      int mm, kk, nn, kb;
-      if (OPA == 'N') { mm = e % BM; kk = e / BM; } else { kk = e % KB; mm = e / KB; }
-      if (OPB == 'N' || OPB == 'R') { kb = e % KB; nn = e / KB; } else { nn = e % BN; kb = e / BN; }
-      Ar[kk][mm] = ra[r].x;
-      Ai[kk][mm] = ra[r].y;
-      Br[kb][nn] = rb[r].x;
-      Bi[kb][nn] = rb[r].y;
-    }
-  };
-  if (kbeg < kend) {
-    gload(kbeg);
-    sstore();
+  for (int r = 0; r < NA; ++r) {
+    const int e = tid + 256 * r, mm = AK ? e / KB : e % TM, kk = AK ? e % KB : e / TM;
+    const int m = mm < mrem ? mm : mrem - 1;
+    oa[r] = (OFF)(16 * (AK ? lda * m + kk : m + lda * kk));
   }
-  __syncthreads();
-  for (int64_t k0 = kbeg; k0 < kend; k0 += KB) {
-    const bool more = k0 + KB < kend;
-    if (more) gload(k0 + KB);
 #pragma unroll
-    for (int kk = 0; kk < KB; kk += 4) {
-      const int kl = kk + (lane >> 4);
-      double ar[2], ai[2], br[2], bi[2];
+  for (int r = 0; r < NB; ++r) {
+    const int e = tid + 256 * r, nn = BKc ? e / KB : e % TN, kk = (BKc ? e % KB : e / TN) % KB;
+    const int n = nn < nrem ? nn : nrem - 1;
+    ob[r] = (OFF)(16 * (BKc ? ldb * n + kk : n + ldb * kk));
+  }
+  auto at = [](const cplx* p, OFF o) {
+    return *reinterpret_cast<const cplx*>(reinterpret_cast<const char*>(p) + o);
+  };
+  auto gload = [&]() {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        ar[i] = Ar[kl][wm + 16 * i + (lane & 15)];
-        ai[i] = Ai[kl][wm + 16 * i + (lane & 15)];
-        br[i] = Br[kl][wn + 16 * i + (lane & 15)];
-        bi[i] = Bi[kl][wn + 16 * i + (lane & 15)];
-      }
+    for (int r = 0; r < NA; ++r) ra[r] = at(At, oa[r]);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int r = 0; r < NB; ++r) rb[r] = at(Bt, ob[r]);
+  };
+  // the last, partial tile: read up to its last k, zero past it
+  auto gload_part = [&](int krem) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          accr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], br[j], accr[i][j], 0, 0, 0);
-          accr[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai[i], bi[j], accr[i][j], 0, 0, 0);
-          acci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i], bi[j], acci[i][j], 0, 0, 0);
-          acci[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[i], br[j], acci[i][j], 0, 0, 0);
-        }
+    for (int r = 0; r < NA; ++r) {
+      const int e = tid + 256 * r, kk = AK ? e % KB : e / TM;
+      ra[r] = at(At, kk < krem ? oa[r] : oa[r] - (OFF)(16 * (AK ? 1 : lda) * (kk - krem + 1)));
+      if (kk >= krem) ra[r] = mk(0.0, 0.0);
     }
+#pragma unroll
+    for (int r = 0; r < NB; ++r) {
+      const int e = tid + 256 * r, kk = (BKc ? e % KB : e / TN) % KB;
+      rb[r] = at(Bt, kk < krem ? ob[r] : ob[r] - (OFF)(16 * (BKc ? 1 : ldb) * (kk - krem + 1)));
+      if (kk >= krem) rb[r] = mk(0.0, 0.0);
+    }
+  };
+  // LDS positions of this thread's elements and fragments in buffer 0 (bytes; the other buffer
+  // is AB / BB further on)
+  constexpr int AB = KB * LA, BB = KB * LB;
+  auto sstore = [&](int buf) {
+    cplx* as = As + buf * AB;
+    cplx* bs = Bs + buf * BB;
+#pragma unroll
+    for (int r = 0; r < NA; ++r) {
+      const int e = tid + 256 * r, mm = AK ? e / KB : e % TM, kk = AK ? e % KB : e / TM;
+      as[kk * LA + mm] = OPA == 'C' ? cconj(ra[r]) : ra[r];
+    }
+#pragma unroll
+    for (int r = 0; r < NB; ++r) {
+      const int e = tid + 256 * r, nn = BKc ? e / KB : e % TN, kk = BKc ? e % KB : e / TN;
+      if (TN * KB % 256 == 0 || e < TN * KB) bs[kk * LB + nn] = (OPB == 'R' || OPB == 'C') ? cconj(rb[r]) : rb[r];
+    }
+  };
+  const cplx* as0 = As + (lane >> 4) * LA + wm + (lane & 15);
+  const cplx* bs0 = Bs + (lane >> 4) * LB + (lane & 15);
+  auto mul4 = [&](int buf, int kk) {   // four k of the tile in buffer buf
+    cplx b[F];
+    const cplx a = as0[buf * AB + kk * LA];
+#pragma unroll
+    for (int j = 0; j < F; ++j) b[j] = bs0[buf * BB + kk * LB + 16 * j];
+    // the transposed fragment (rows n), so that a lane's column index runs along m: the stores
+    // of C write 16 consecutive elements; dependent products are 2 F apart
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      accr[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j].x, a.x, accr[j], 0, 0, 0);
+      acci[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j].y, a.x, acci[j], 0, 0, 0);
+    }
+    const double na = -a.y;
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      accr[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j].y, na, accr[j], 0, 0, 0);
+      acci[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j].x, a.y, acci[j], 0, 0, 0);
+    }
+  };
+  auto mul = [&](int buf) {
+#pragma unroll
+    for (int kk = 0; kk < KB; kk += 4) mul4(buf, kk);
+  };
+  const int nfull = ktot / KB, rem = ktot - nfull * KB;
+  if (nfull > 0) {
+    gload();
+    sstore(0);
     __syncthreads();
-    if (more) {
-      sstore();
+    // two tiles per round, so that the buffer is a constant and the loop has no branches
+    int t = 1;
+    for (; t + 1 < nfull; t += 2) {
+      At += stepA;
+      Bt += stepB;
+      gload();
+      mul(0);
+      sstore(1);
+      __syncthreads();
+      At += stepA;
+      Bt += stepB;
+      gload();
+      mul(1);
+      sstore(0);
       __syncthreads();
     }
+    const bool odd = t < nfull;
+    if (odd) {
+      At += stepA;
+      Bt += stepB;
+      gload();
+      mul(0);
+      sstore(1);
+      __syncthreads();
+    }
+    // the last full tile, in buffer odd
+    if (rem > 0) {
+      At += stepA;
+      Bt += stepB;
+      gload_part(rem);
+    }
+    mul(odd);
+    if (rem > 0) {
+      sstore(!odd);
+      __syncthreads();
+      for (int kk = 0; kk < rem; kk += 4) mul4(!odd, kk);
+    }
+  } else if (rem > 0) {
+    gload_part(rem);
+    sstore(0);
+    __syncthreads();
+    for (int kk = 0; kk < rem; kk += 4) mul4(0, kk);
   }
+}
+
+// blockIdx.z = batch index * sk + K-split index; split kz covers K in [kz*kchunk, (kz+1)*kchunk)
+// and writes its partial product to C + kz * sC (the split-K workspace) when sk > 1.  UPPER:
+// only the tiles that reach the upper triangle (a Hermitian product; the others leave at
+// once).  OFF: offsets within a tile, 32 bits where the leading dimensions allow it.
+template <char OPA, char OPB, int FN, int KB, bool UPPER = false, class OFF = uint32_t>
+__global__ __launch_bounds__(256, 2) void k_zgemm(int64_t M, int64_t N, int64_t Kfull, cplx alpha,
+                                                  const cplx* __restrict__ A, int64_t lda, int64_t sA,
+                                                  const cplx* __restrict__ B, int64_t ldb, int64_t sB,
+                                                  cplx beta, cplx* __restrict__ C, int64_t ldc, int64_t sC, int sk,
+                                                  int64_t kchunk, int tri) {
+  using T = ZgTile<OPA, OPB, FN, KB>;
+  constexpr int TM = T::TM, TN = T::TN;
+  int64_t mt, nt;
+  xcd_tile(gridDim.x, gridDim.y, blockIdx.x, blockIdx.y, mt, nt);
+  if (UPPER && mt * TM > nt * TN + TN - 1) return;   // uniform
+  __shared__ cplx As[2 * KB * T::LA], Bs[2 * KB * T::LB];
+  const int64_t bz = blockIdx.z / sk, kz = blockIdx.z % sk;
+  C += (sk > 1 ? bz * sk + kz : bz) * sC;
+  const int64_t kbeg = kz * kchunk;
+  int64_t kend = (kbeg + kchunk < Kfull) ? kbeg + kchunk : Kfull;
+  if (tri == TRI_A && kend > (mt + 1) * TM) kend = (mt + 1) * TM;
+  if (tri == TRI_B && kend > (nt + 1) * TN) kend = (nt + 1) * TN;
+  const int64_t m0 = mt * TM, n0 = nt * TN;
+  const int mrem = (int)(M - m0 < TM ? M - m0 : TM), nrem = (int)(N - n0 < TN ? N - n0 : TN);
+  const cplx* At = A + bz * sA + (T::AK ? lda * m0 + kbeg : m0 + lda * kbeg);
+  const cplx* Bt = B + bz * sB + (T::BKc ? ldb * n0 + kbeg : n0 + ldb * kbeg);
+  d4 accr[FN], acci[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    accr[j] = d4{0.0, 0.0, 0.0, 0.0};
+    acci[j] = d4{0.0, 0.0, 0.0, 0.0};
+  }
+  const int f = (nrem + 15) / 16, ktot = (int)(kend - kbeg);   // uniform
+  if (f == FN) zg_loop<OPA, OPB, FN, KB, FN, OFF>(At, Bt, lda, ldb, mrem, nrem, ktot, As, Bs, accr, acci);
+  else if (FN > 1 && f == 1) zg_loop<OPA, OPB, FN, KB, 1, OFF>(At, Bt, lda, ldb, mrem, nrem, ktot, As, Bs, accr, acci);
+  else if (FN > 2 && f == 2)
+    zg_loop<OPA, OPB, FN, KB, (FN > 2 ? 2 : 1), OFF>(At, Bt, lda, ldb, mrem, nrem, ktot, As, Bs, accr, acci);
+  else if (FN > 3 && f == 3)
+    zg_loop<OPA, OPB, FN, KB, (FN > 3 ? 3 : 1), OFF>(At, Bt, lda, ldb, mrem, nrem, ktot, As, Bs, accr, acci);
+  // D[row][col] of a 16x16 MFMA tile sits in element (row / 4) of lane col + 16 * (row % 4)
+  // (measured on gfx950 with a one-hot probe of the builtin); rows are n here
+  const int lane = threadIdx.x & 63, wm = (threadIdx.x >> 6) * 16;
   const bool beta_zero = (beta.x == 0.0 && beta.y == 0.0);
+  const int64_t row = m0 + wm + (lane & 15);
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < FN; ++j)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t row = m0 + wm + 16 * i + (lane >> 4) + 4 * r;
-        const int64_t col = n0 + wn + 16 * j + (lane & 15);
-        if (row < M && col < N) {
-          cplx acc = mk(accr[i][j][r], acci[i][j][r]);
-          cplx out = cmul(alpha, acc);
-          if (!beta_zero) cfma(out, beta, C[row + ldc * col]);
-          C[row + ldc * col] = out;
-        }
+    for (int r = 0; r < 4; ++r) {
+      const int64_t col = n0 + 16 * j + (lane >> 4) + 4 * r;
+      if (row < M && col < N) {
+        const cplx acc = mk(accr[j][r], acci[j][r]);
+        cplx out = cmul(alpha, acc);
+        if (!beta_zero) cfma(out, beta, C[row + ldc * col]);
+        C[row + ldc * col] = out;
       }
+    }
 }
 
 // ---- shapes with too few output tiles for the MFMA kernel (the block Davidson of the CI
@@ -511,11 +510,29 @@ cplx* splitk_workspace(hipStream_t s, size_t n) {
 }
 
 GemmStats* g_stats = nullptr;
-// kernel variant: 0 k_zgemm, 1..4 k_zgemm2 with (KB, PAD) = (16,1), (16,16), (32,1), (32,16).
-// Default 1: measured fastest on every shape of the path (e.g. 61 vs 46 TF/s on 2048^3).
+// The variants of k_zgemm: 1 FN 4, KB 8; 2 FN 2, KB 16; 3 FN 1, KB 16; 4 FN 1, KB 8
+struct Variant {
+  int fn, kb;
+};
+constexpr Variant kVariants[5] = {{0, 0}, {4, 8}, {2, 16}, {1, 16}, {1, 8}};
+
+// The variant of a product by its sizes.  FN 4 keeps the matrix units busiest (A is read once
+// per 64 columns) and needs at most 64 columns or more than four tiles per compute unit to do so;
+// short of that the narrower tiles spread the product over more workgroups (1274 x 280 x 1274:
+// 76 us with FN 1, 114 with FN 4; 2048^3: 968 with FN 2, 1010 with FN 4).  At most 32 columns
+// take the tile they fill, and K <= 8 the shorter K tile (600000 x 8 x 8: 24 us against 33).
+int pick_variant(int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const int64_t mt = cdiv(M, BM) * batch;
+  if (N <= 16) return K <= 8 ? 4 : 3;
+  if (N <= 32) return mt >= 256 ? 2 : 3;
+  if (N <= 64 ? mt >= 256 : mt * cdiv(N, 64) > 1024) return 1;
+  return mt * cdiv(N, 32) > 1024 ? 2 : 3;
+}
+
+// DC2_GEMM_VARIANT: 1..4 that variant for every product, 0 no kernels for skinny shapes
 int g_variant = [] {
   const char* v = std::getenv("DC2_GEMM_VARIANT");
-  return v ? std::atoi(v) : 1;
+  return v ? std::atoi(v) : -1;
 }();
 std::mutex g_stats_mu;
 thread_local int g_tag = 0;
@@ -620,19 +637,9 @@ void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, cplx alpha, const cp
     record(false);
     return;
   }
-  // split K over workgroups when the output has few tiles and K is long
-  const int64_t tiles = (int64_t)cdiv(M, BM) * cdiv(N, BN) * batch;
-  int sk = 1;
-  int64_t kchunk = K;
-  if (tiles < 128 && K >= 256) {
-    int64_t want = std::min<int64_t>(K / 128, (256 + tiles - 1) / tiles);
-    want = std::max<int64_t>(2, std::min<int64_t>(want, 64));
-    kchunk = ((K + want - 1) / want + BK - 1) / BK * BK;
-    sk = (int)((K + kchunk - 1) / kchunk);
-  }
-  int variant = g_variant;
+  int variant = g_variant >= 1 && g_variant <= 4 ? g_variant : pick_variant(M, N, K, batch);
   TuneChoice tc{0, 0};
-  int want_split = 0;   // 0: the rule above
+  int want_split = 0;   // 0: the rule below
   if (force_variant > 0) {
     variant = force_variant;
     want_split = force_split;
@@ -640,19 +647,25 @@ void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, cplx alpha, const cp
     variant = tc.variant;
     want_split = tc.split;
   }
-  if (want_split > 0) {
-    sk = 1;
-    kchunk = K;
-    if (want_split > 1) {
-      kchunk = ((K + want_split - 1) / want_split + BK - 1) / BK * BK;
-      sk = (int)((K + kchunk - 1) / kchunk);
-    }
+  if (cdiv(N, 16 * kVariants[variant].fn) >= 65536) variant = 1;   // the grid's second dimension
+  // split K over workgroups when the output has few tiles and K is long (1274 x 280 x 1274: 360
+  // tiles, 92 us unsplit, 76 in three)
+  const int64_t tn = 16 * kVariants[variant].fn;
+  const int64_t tiles = (int64_t)cdiv(M, BM) * cdiv(N, tn) * batch;
+  int sk = 1;
+  int64_t kchunk = K;
+  if (want_split == 0 && tiles < 512 && K >= 256) {
+    want_split = (int)std::min<int64_t>(K / 128, (1024 + tiles - 1) / tiles);
+    want_split = std::max(2, std::min(want_split, 64));
+  }
+  if (want_split > 1) {
+    kchunk = ((K + want_split - 1) / want_split + BK - 1) / BK * BK;
+    sk = (int)((K + kchunk - 1) / kchunk);
   }
   if (batch * sk >= 65536 || g_no_ws) {   // one grid dimension holds batch x split
     sk = 1;
     kchunk = K;
   }
-  dim3 grid(cdiv(M, BM), cdiv(N, BN), (unsigned)(batch * sk));
   cplx* Cw = C;
   int64_t ldw = ldc, sw = sC;
   cplx a1 = alpha, b1 = beta;
@@ -663,26 +676,26 @@ void launch(hipStream_t s, int64_t M, int64_t N, int64_t K, cplx alpha, const cp
     a1 = mk(1.0, 0.0);
     b1 = mk(0.0, 0.0);
   }
-  switch (variant) {
-    case 1:
-      hipLaunchKernelGGL((k_zgemm2<OPA, OPB, 16, 1>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB, b1,
-                         Cw, ldw, sw, sk, kchunk, (int)TRI_NONE);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_zgemm2<OPA, OPB, 16, 16>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB,
-                         b1, Cw, ldw, sw, sk, kchunk, (int)TRI_NONE);
-      break;
-    case 3:
-      hipLaunchKernelGGL((k_zgemm2<OPA, OPB, 32, 1>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB, b1,
-                         Cw, ldw, sw, sk, kchunk, (int)TRI_NONE);
-      break;
-    case 4:
-      hipLaunchKernelGGL((k_zgemm2<OPA, OPB, 32, 16>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB,
-                         b1, Cw, ldw, sw, sk, kchunk, (int)TRI_NONE);
-      break;
-    default:
-      hipLaunchKernelGGL((k_zgemm<OPA, OPB>), grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB, b1, Cw,
-                         ldw, sw, sk, kchunk);
+  DC2_CHECK(cdiv(N, tn) < 65536, 1, "zgemm: matrix too large for the grid");
+  const dim3 grid(cdiv(M, BM), cdiv(N, tn), (unsigned)(batch * sk));
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, M, N, K, a1, A, lda, sA, B, ldb, sB, b1, Cw, ldw, sw, sk, kchunk,
+                       (int)TRI_NONE);
+  };
+  if (lda < kLd32 && ldb < kLd32) {
+    switch (variant) {
+      case 1: go(k_zgemm<OPA, OPB, 4, 8>); break;
+      case 2: go(k_zgemm<OPA, OPB, 2, 16>); break;
+      case 3: go(k_zgemm<OPA, OPB, 1, 16>); break;
+      default: go(k_zgemm<OPA, OPB, 1, 8>); break;
+    }
+  } else {
+    switch (variant) {
+      case 1: go(k_zgemm<OPA, OPB, 4, 8, false, uint64_t>); break;
+      case 2: go(k_zgemm<OPA, OPB, 2, 16, false, uint64_t>); break;
+      case 3: go(k_zgemm<OPA, OPB, 1, 16, false, uint64_t>); break;
+      default: go(k_zgemm<OPA, OPB, 1, 8, false, uint64_t>); break;
+    }
   }
   if (sk > 1)
     hipLaunchKernelGGL(k_splitk_reduce, dim3(cdiv(M * N, 256), (unsigned)batch), dim3(256), 0, s, M, N, sk, Cw, alpha,
@@ -733,7 +746,7 @@ void zgemm(hipStream_t s, char opA, char opB, int64_t M, int64_t N, int64_t K, c
            int64_t sC, int64_t batch) {
   if (M <= 0 || N <= 0 || batch <= 0) return;
   DC2_CHECK(batch < 65536, 1, "zgemm: batch too large for one grid dimension");
-  DC2_CHECK(cdiv(M, BM) < (1u << 31) && cdiv(N, BN) < 65536, 1, "zgemm: matrix too large for the grid");
+  DC2_CHECK(cdiv(M, BM) < (1u << 31) && cdiv(N, 64) < 65536, 1, "zgemm: matrix too large for the grid");
   dispatch(s, opA, opB, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
 }
 
@@ -755,28 +768,27 @@ void zgemm_herm(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda,
   DC2_CHECK(cdiv(m, BM) < 65536, 1, "zgemm_herm: matrix too large for the grid");
   DC2_CHECK(split >= 0 && split <= 64, 1, "zgemm_herm: split 0..64");
   const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
-  const int64_t T = cdiv(m, BM), tiles = T * (T + 1) / 2;
+  // tiles of 64 x 16: finer along the diagonal and enough workgroups without splitting k far
+  const int64_t T = cdiv(m, BM), Tn = cdiv(m, 16), tiles = T * (Tn + 4) / 2;
+  DC2_CHECK(Tn < 65536, 1, "zgemm_herm: matrix too large for the grid");
   int64_t want = split;
-  if (want == 0 && tiles < 256 && k >= 256) want = std::min<int64_t>(std::min<int64_t>(k / 128, cdiv(1024, tiles)), 12);
+  if (want == 0 && tiles < 1024 && k >= 256) want = std::min<int64_t>(std::min<int64_t>(k / 128, cdiv(2048, tiles)), 12);
   int64_t kchunk = k;
   int sk = 1;
   if (want > 1 && k > 0) {
     kchunk = (cdiv(k, want) + BK - 1) / BK * BK;
     sk = (int)cdiv(k, kchunk);
   }
-  if (sk > 1) {
-    cplx* W = splitk_workspace(s, (size_t)sk * m * m);
-    dim3 grid(T, T, (unsigned)sk);
-    hipLaunchKernelGGL((k_zgemm2<'N', 'C', 16, 1, true>), grid, dim3(256), 0, s, m, m, k, one, A, lda, (int64_t)0, B,
-                       ldb, (int64_t)0, zero, W, m, m * m, sk, kchunk, (int)TRI_NONE);
-    hipLaunchKernelGGL(k_herk_reduce, dim3(cdiv(m * m, 256)), dim3(256), 0, s, m, sk, W, C, ldc);
-    DC2_HIP(hipGetLastError());
-    return;
-  }
-  dim3 grid(T, T, 1);
-  hipLaunchKernelGGL((k_zgemm2<'N', 'C', 16, 1, true>), grid, dim3(256), 0, s, m, m, k, one, A, lda, (int64_t)0, B,
-                     ldb, (int64_t)0, zero, C, ldc, (int64_t)0, 1, k, (int)TRI_NONE);
-  hipLaunchKernelGGL(k_lower_from_upper, dim3(cdiv(m * m, 256)), dim3(256), 0, s, m, C, ldc);
+  cplx* W = sk > 1 ? splitk_workspace(s, (size_t)sk * m * m) : C;
+  const dim3 grid(T, Tn, (unsigned)sk);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, m, m, k, one, A, lda, (int64_t)0, B, ldb, (int64_t)0, zero, W,
+                       sk > 1 ? m : ldc, m * m, sk, kchunk, (int)TRI_NONE);
+  };
+  if (lda < kLd32 && ldb < kLd32) go(k_zgemm<'N', 'C', 1, 16, true>);
+  else go(k_zgemm<'N', 'C', 1, 16, true, uint64_t>);
+  if (sk > 1) hipLaunchKernelGGL(k_herk_reduce, dim3(cdiv(m * m, 256)), dim3(256), 0, s, m, sk, W, C, ldc);
+  else hipLaunchKernelGGL(k_lower_from_upper, dim3(cdiv(m * m, 256)), dim3(256), 0, s, m, C, ldc);
   DC2_HIP(hipGetLastError());
 }
 
@@ -785,10 +797,10 @@ void zgemm_herm(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda,
 void zherk_trailing(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda, int64_t sA, cplx* C, int64_t ldc,
                     int64_t sC, int64_t batch) {
   if (m <= 0) return;
-  const int64_t T = cdiv(m, BM);
-  DC2_CHECK(T < 65536 && batch < 65536, 1, "zherk_trailing: matrix too large for the grid");
-  dim3 grid(T, T, (unsigned)batch);
-  hipLaunchKernelGGL((k_zgemm2<'C', 'N', 16, 1, true>), grid, dim3(256), 0, s, m, m, k, mk(-1.0, 0.0), A, lda, sA, A,
+  const int64_t T = cdiv(m, BM), Tn = cdiv(m, 32);
+  DC2_CHECK(Tn < 65536 && batch < 65536 && lda < kLd32, 1, "zherk_trailing: matrix too large");
+  dim3 grid(T, Tn, (unsigned)batch);
+  hipLaunchKernelGGL((k_zgemm<'C', 'N', 2, 16, true>), grid, dim3(256), 0, s, m, m, k, mk(-1.0, 0.0), A, lda, sA, A,
                      lda, sA, mk(1.0, 0.0), C, ldc, sC, 1, k, (int)TRI_NONE);
   DC2_HIP(hipGetLastError());
 }
@@ -799,13 +811,13 @@ void zherk_trailing(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t 
 void zgemm_congruence(hipStream_t s, int64_t n, const cplx* L, int64_t ldl, const cplx* B, int64_t ldb, cplx* T,
                       cplx* C, int64_t ldc) {
   if (n <= 0) return;
-  const int64_t t = cdiv(n, BM);
-  DC2_CHECK(t < 65536, 1, "zgemm_congruence: matrix too large for the grid");
+  const int64_t t = cdiv(n, BM), tn = cdiv(n, 16);
+  DC2_CHECK(tn < 65536 && ldl < kLd32 && ldb < kLd32, 1, "zgemm_congruence: matrix too large");
   const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
-  dim3 grid(t, t, 1);
-  hipLaunchKernelGGL((k_zgemm2<'N', 'N', 16, 1>), grid, dim3(256), 0, s, n, n, n, one, L, ldl, (int64_t)0, B, ldb,
+  dim3 grid(t, tn, 1);
+  hipLaunchKernelGGL((k_zgemm<'N', 'N', 1, 16>), grid, dim3(256), 0, s, n, n, n, one, L, ldl, (int64_t)0, B, ldb,
                      (int64_t)0, zero, T, n, (int64_t)0, 1, n, (int)TRI_A);
-  hipLaunchKernelGGL((k_zgemm2<'N', 'C', 16, 1, true>), grid, dim3(256), 0, s, n, n, n, one, T, n, (int64_t)0, L, ldl,
+  hipLaunchKernelGGL((k_zgemm<'N', 'C', 1, 16, true>), grid, dim3(256), 0, s, n, n, n, one, T, n, (int64_t)0, L, ldl,
                      (int64_t)0, zero, C, ldc, (int64_t)0, 1, n, (int)TRI_B);
   hipLaunchKernelGGL(k_lower_from_upper, dim3(cdiv(n * n, 256)), dim3(256), 0, s, n, C, ldc);
   DC2_HIP(hipGetLastError());
@@ -891,15 +903,17 @@ void gemm_tune(hipStream_t s, char opA, char opB, int64_t M, int64_t N, int64_t 
   }
   const double t_builtin = time(0, 1);
   if (had) gemm_set_choice(opA, opB, M, N, K, batch, prev.variant, prev.split);
-  const int64_t tiles = (int64_t)cdiv(M, BM) * cdiv(N, BN) * batch;
   double best = INFINITY;
   int bv = 1, bs = 1;
-  for (int v = 1; v <= 4; ++v)
+  for (int v = 1; v <= 4; ++v) {
+    const int64_t tiles = (int64_t)cdiv(M, BM) * cdiv(N, 16 * kVariants[v].fn) * batch;
+    if (cdiv(N, 16 * kVariants[v].fn) >= 65536) continue;
     for (int sp : {1, 2, 4, 8, 16, 32}) {
       if (sp > 1 && (K < 2 * BK * sp || tiles * sp > 4096 || batch * sp >= 65536)) continue;
       const double t = time(v, sp);
       if (t < best) { best = t; bv = v; bs = sp; }
     }
+  }
   DC2_HIP(hipEventDestroy(e0));
   DC2_HIP(hipEventDestroy(e1));
   DC2_HIP(hipStreamSynchronize(s));   // the scratch operands are freed next
