@@ -967,9 +967,9 @@ bool chol_whiten(dc2_context* c, Lane& L, char X, int64_t n, const cplx* S, cons
   auto nm = [X](const char* b) { return std::string(1, X) + b; };
   const int64_t np = chol_np(n);
   cplx* Li = L.z(nm("_hLi").c_str(), np * np);
-  cplx* work = L.z(nm("_hW").c_str(), chol_work_elems(n));
+  cplx* work = L.z(nm("_hW").c_str(), chol_work_elems(n, 2));
   cplx* bc1 = L.z(nm("_bc1").c_str(), n * n);
-  int* flags = L.i(nm("_hflag").c_str(), 2);
+  int* flags = L.i(nm("_hflag").c_str(), 3);
   set_gemm_tag(4);
   chol_inverse(s, n, S, n, thr, work, Li, flags);
   zgemm_congruence(s, n, Li, np, B, n, work, bc1, n);
@@ -1050,6 +1050,7 @@ struct GramMetric {
   bool cg = false;        // or (cg) B~ itself in X_bc1
   bool thin = false;      // C through its thin factor: T's eigenvectors in X_Tthin, t L^-1/2 in X_TSthin
   bool chol = false;      // thin, T's inverse Cholesky factor in X_hLi instead, B~ in X_bc1
+  bool defl = false;      // not thin: the cut directions in X_Gd, L^-1 of G + Gd Gd^H in X_hLi
   int64_t m = 0, dimm = 0;
   double margin = INFINITY;
   double seconds = 0.0;   // time spent on the lane before the subspace itself ran
@@ -1064,6 +1065,111 @@ bool gram_thin(const dc2_context* c, char X, int64_t m) {
   // the blocks of M M^T have the eigenvalue 2 + kappa (na - 1) along sigma: invertible only
   const double kappa = (double)(na - 2 * (ne - 1)) / ((double)(ne - 1) * (ne - 1));
   return nred < m && m - nred > e2_schur_max_dropped() && 2.0 + kappa * (na - 1) > 1e-6;
+}
+
+// Whether the determinant-space metric goes without its eigendecomposition (gram_deflate): where
+// the compressed resolvent takes E2 (at most e2_schur_max_dropped() directions cut).  Not with RAS
+// limits, which cut more directions as a rule.
+bool deflate_route(const dc2_context* c, char X, int64_t m) {
+  return chol_route(c, X, m) && c->schur && !gram_thin(c, X, m);
+}
+
+// The metric G (m x m, in X_G, kept) without its eigendecomposition.  The compressed resolvent
+// needs the cut eigenvectors Gd (eigenvalues below the threshold, a few) and the inverse of G on
+// the others only.  One batch of three factorisations: G - 2 thr (positive definite: nothing is
+// cut, and nothing lies near the threshold), G itself, and G + delta for the subspace iteration
+// that gives the cut eigenvectors otherwise; then G' = G + Gd Gd^H, which moves the cut
+// eigenvalues to 1, is factorised beside G' - thr, whose positive definiteness shows that Gd holds
+// all of them.  False (the caller diagonalises G): an eigenvalue within 1e-3 of the threshold,
+// more cut directions than the compressed resolvent takes, or more than LOW_P eigenvalues so
+// small that the iteration would not separate the lowest ones.
+// At 192 spinors (792 x 792, 4 to 8 directions cut) this takes 2.5 ms where tridiagonalisation,
+// divide and conquer, back-transformation and the rotation of the eigenvectors took 11.
+bool gram_deflate(dc2_context* c, Lane& L, char X, const cplx* G, GramMetric& g) {
+  const int64_t m = g.m, np = chol_np(m), p = LOW_P;
+  const double thr = 1.0e-8, delta = 1.0e-9;
+  hipStream_t s = L.stream;
+  auto nm = [X](const char* b) { return std::string(1, X) + b; };
+  const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
+  cplx* Li = L.z(nm("_hLi").c_str(), 2 * np * np);
+  cplx* work = L.z(nm("_hW").c_str(), chol_work_elems(m, 3));
+  int* flags = L.i(nm("_hflag").c_str(), 3);
+  const double shifts[3] = {0.0, 2.0 * thr, -delta};
+  int hf[3];
+  set_gemm_tag(4);
+  chol_factor(s, m, G, m, 3, shifts, work, Li, flags);
+  L.download(hf, flags, sizeof(hf));
+  if (!hf[0] && !hf[1]) {
+    chol_invert(s, m, work, 3, 0, Li);
+    set_gemm_tag(0);
+    g.defl = true;
+    g.dimm = m;
+    // the closest eigenvalue is one of the n - m that vanish, or at least a threshold away
+    g.margin = std::min(g.margin, thr);
+    return true;
+  }
+  if (hf[2] || m < 2 * p) {
+    set_gemm_tag(0);
+    return false;
+  }
+  chol_invert(s, m, work, 3, 2, Li + np * np);
+  cplx* Xs = L.z(nm("_lowX").c_str(), m * p);
+  cplx* H = L.z(nm("_lowH").c_str(), p * p);
+  cplx* lw = L.z(nm("_loww").c_str(), low_work_elems(m));
+  std::vector<zc> hH((size_t)p * p), Q((size_t)p * e2_schur_max_dropped());
+  std::vector<double> w(p);
+  const int rmax = e2_schur_max_dropped();
+  low_start(s, m, Xs);
+  int r = 0;
+  bool ok = false;
+  for (int round = 0; round < 2 && !ok; ++round) {
+    low_iterate(s, m, G, Li + np * np, 8, Xs, lw, H, flags);
+    DC2_HIP(hipMemcpyAsync(L.host(p * p * sizeof(zc) + 3 * sizeof(int), 1), H, p * p * sizeof(zc), hipMemcpyDeviceToHost, s));
+    char* hp = reinterpret_cast<char*>(L.host(p * p * sizeof(zc) + 3 * sizeof(int), 1));
+    DC2_HIP(hipMemcpyAsync(hp + p * p * sizeof(zc), flags, 3 * sizeof(int), hipMemcpyDeviceToHost, s));
+    DC2_HIP(hipStreamSynchronize(s));
+    std::memcpy(hH.data(), hp, p * p * sizeof(zc));
+    std::memcpy(hf, hp + p * p * sizeof(zc), sizeof(hf));
+    if (hf[0]) break;
+    for (int j = 0; j < p; ++j) {
+      hH[j + p * j] = hH[j + p * j].real();
+      for (int i = 0; i < j; ++i) hH[j + p * i] = std::conj(hH[i + p * j]);
+    }
+    herm_eig_low((int)p, hH.data(), w.data(), Q.data(), rmax);
+    if (!std::isfinite(w[0]) || !(w[p - 1] > 3.0 * thr)) break;
+    r = 0;
+    while (r < p && w[r] < thr) ++r;
+    if (r < 1 || r > rmax || w[r - 1] > 0.999 * thr || w[r] < 1.001 * thr) break;
+    // what the cut vectors still hold of the directions outside the block falls by this
+    // factor per step
+    const double rate = (w[r - 1] + delta) / (w[p - 1] + delta);
+    ok = std::pow(rate, 8 * (round + 1)) < 1e-13;
+  }
+  if (ok) {
+    cplx* Gd = L.z(nm("_Gd").c_str(), m * r);
+    cplx* Qd = L.z(nm("_lowQ").c_str(), p * r);
+    zc* hq = reinterpret_cast<zc*>(L.host(p * r * sizeof(zc), 1));
+    std::copy(Q.begin(), Q.begin() + p * r, hq);
+    DC2_HIP(hipMemcpyAsync(Qd, hq, p * r * sizeof(zc), hipMemcpyHostToDevice, s));
+    zgemm(s, 'N', 'N', m, r, p, one, Xs, m, 0, Qd, p, 0, zero, Gd, m, 0, 1);
+    cplx* Gp = L.z(nm("_Gp").c_str(), m * m);
+    DC2_HIP(hipMemcpyAsync(Gp, G, m * m * sizeof(cplx), hipMemcpyDeviceToDevice, s));
+    zgemm(s, 'N', 'C', m, m, r, one, Gd, m, 0, Gd, m, 0, one, Gp, m, 0, 1);
+    const double sh[2] = {0.0, thr};
+    chol_factor(s, m, Gp, m, 2, sh, work, Li, flags);
+    chol_invert(s, m, work, 2, 0, Li);
+    L.download(hf, flags, sizeof(hf));
+    ok = !hf[0] && !hf[1];
+  }
+  set_gemm_tag(0);
+  if (c->debug)
+    std::fprintf(stderr, "dc2: %c metric (m=%lld): %d directions cut, %s; block's eigenvalues %.2e .. %.2e\n", X,
+                 (long long)m, r, ok ? "deflated" : "not deflated", w[0], w[p - 1]);
+  if (!ok) return false;
+  g.defl = true;
+  g.dimm = m - r;
+  for (int i = 0; i < p; ++i) g.margin = std::min(g.margin, std::fabs(w[i] - thr));
+  return true;
 }
 
 // Phi from the E_uv|0> vectors Y of the CASCI state in one orbital basis, G = Phi Phi^H,
@@ -1136,6 +1242,7 @@ GramMetric gram_eig(dc2_context* c, Lane& L, char X, int64_t n, const cplx* Y, c
   cplx* G = L.z(nm("_G").c_str(), m * m);
   zherk_upper(s, m, n, Phi, m, G, m);   // Hermitian: the upper tiles only
   check_finite(c, s, "Phi Phi^H", G, m * m);
+  if (deflate_route(c, X, m) && gram_deflate(c, L, X, G, g)) return g;
   zheevd(c, L, (int)m, G, lam, "a determinant-space metric", ras ? EigKind::rank_deficient : EigKind::general);
   g.dimm = count_retained(L, m, lam, g.margin);
   return g;
@@ -1181,7 +1288,7 @@ void gram_rotated_parts(dc2_context* c, Lane& L, char X, int64_t n, const GramMe
   if (!phi_current)
     build_phi(s, c->na, c->ne, X == 'A', c->nfull, c->rank_full.get(), c->Y1.get(), c->eps.get() + c->ni, m,
               L.l(nm("_strings").c_str(), m), L.z(nm("_Phi").c_str(), m * n), L.d(nm("_f").c_str(), m));
-  if (g.dimm > 0 && !g.thin)
+  if (g.dimm > 0 && !g.thin && !g.defl)
     scale_cols_tail(s, m, g.dimm, L.z(nm("_G").c_str(), m * m), L.d(nm("_lam").c_str(), m),
                     L.z(nm("_GL").c_str(), m * g.dimm), true);
 }
@@ -1243,6 +1350,43 @@ SolveOut solve_block_gram(dc2_context* c, Lane& L, char X, const GramMetric& g, 
   const cplx* Phi = L.z(nm("_Phi").c_str(), m * n);
   const double* f = L.d(nm("_f").c_str(), m);
   const int64_t nd = m - dimm;
+  if (g.defl) {
+    // z = G^+ Phi V without G's eigenvectors: the cut directions projected out, L^-H L^-1
+    const int64_t np = chol_np(m);
+    const int rd = (int)nd;
+    const cplx* Li = L.z(nm("_hLi").c_str(), np * np);
+    cplx* P = L.z(nm("_P").c_str(), m * npert);
+    cplx* T = L.z(nm("_T").c_str(), m * npert);
+    cplx* Z = L.z(nm("_Z").c_str(), m * npert);
+    const cplx* Gd = rd ? L.z(nm("_Gd").c_str(), m * rd) : nullptr;
+    cplx* Cd = rd ? L.z(nm("_Cd").c_str(), rd * npert) : nullptr;
+    auto project = [&](cplx* x) {
+      if (!rd) return;
+      zgemm(s, 'C', 'N', rd, npert, m, one, Gd, m, 0, x, m, 0, zero, Cd, rd, 0, 1);
+      zgemm(s, 'N', 'N', m, npert, rd, mk(-1.0, 0.0), Gd, m, 0, Cd, rd, 0, one, x, m, 0, 1);
+    };
+    set_gemm_tag(4);
+    zgemm(s, 'N', 'N', m, npert, n, one, Phi, m, 0, V, n, 0, zero, P, m, 0, 1);
+    project(P);
+    zgemm(s, 'N', 'N', m, npert, m, one, Li, np, 0, P, m, 0, zero, T, m, 0, 1);
+    zgemm(s, 'C', 'N', m, npert, m, one, Li, np, 0, T, m, 0, zero, Z, m, 0, 1);
+    project(Z);
+    set_gemm_tag(0);
+    double* partial = L.d("partial", 2 * npert);
+    double* out2 = L.d("out2", 2);
+    e2_schur(s, m, rd, npert, Gd, Z, f, alpha, partial, out2);
+    read_out2(L, out2, r);
+    if (std::isfinite(r.e2) && std::isfinite(r.sumc2)) return r;
+    // a singular compressed system: the eigendecomposition after all
+    GramMetric full = g;
+    full.defl = false;
+    cplx* Gm = L.z(nm("_G").c_str(), m * m);
+    double* lam = L.d(nm("_lam").c_str(), m);
+    zheevd(c, L, (int)m, Gm, lam, "a determinant-space metric");
+    full.dimm = count_retained(L, m, lam, full.margin);
+    if (full.dimm > 0) scale_cols_tail(s, m, full.dimm, Gm, lam, L.z(nm("_GL").c_str(), m * full.dimm), true);
+    return solve_block_gram(c, L, X, full, n, npert, V, alpha);
+  }
   cplx* G = g.chol ? nullptr : L.z(nm("_G").c_str(), m * m);   // chol: only B~ and Y are used
   const cplx* Gk = g.chol ? nullptr : G + m * nd;
   cplx* Y = L.z(nm("_Y").c_str(), dimm * npert);
@@ -1753,6 +1897,9 @@ void run_caspt2(dc2_context* c, int selectroot, double eshift, double* e2, doubl
         if (!ras)
           for (int k : plan[w]) {
             if (!gram_k(k) || gram_thin(c, kSub[k], binom_host(na, c->ne - 1))) continue;
+            // without its eigenvectors the metric takes less time than the rotated state does
+            // to arrive, and is formed from that
+            if (deflate_route(c, kSub[k], binom_host(na, k == 0 ? c->ne + 1 : c->ne - 1))) continue;
             Timer tm(Lw.stream);
             prep[k].g = gram_eig(c, Lw, kSub[k], n3, c->Y1o.get(), zeros_act);
             prep[k].seconds = tm.stop();

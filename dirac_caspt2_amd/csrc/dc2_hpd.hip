@@ -257,24 +257,26 @@ bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const
 
 namespace {
 
-constexpr int CH_NB = 64, CH_LS = CH_NB + 1;
+constexpr int CH_NB = LOW_P, CH_LS = CH_NB + 1;   // 64: the Gram matrix of low_iterate is one block
 
-// W[b] (np x np): S in the leading n x n corner, less sigma_b on the diagonal (sigma_0 = 0), the
-// unit matrix below it
-__global__ __launch_bounds__(256) void k_chol_pack(int n, int np, const cplx* __restrict__ S, int64_t lds, double sigma,
-                                                   cplx* __restrict__ W) {
+struct Shifts {
+  double v[3];
+};
+
+// W[b] (np x np), b < nmat: S - shift_b I in the leading n x n corner, the unit matrix below it
+__global__ __launch_bounds__(256) void k_chol_pack(int n, int np, const cplx* __restrict__ S, int64_t lds, int nmat,
+                                                   Shifts shift, cplx* __restrict__ W) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (t >= (int64_t)np * np) return;
   const int i = (int)(t % np), j = (int)(t / np);
-  cplx v = mk(i == j ? 1.0 : 0.0, 0.0);
-  if (i < n && j < n) v = S[i + lds * j];
-  W[t] = v;
-  if (i == j && i < n) v.x -= sigma;
-  W[(int64_t)np * np + t] = v;
+  const bool in = i < n && j < n;
+  const cplx v = in ? S[i + lds * j] : mk(i == j ? 1.0 : 0.0, 0.0);
+  for (int b = 0; b < nmat; ++b)
+    W[(int64_t)np * np * b + t] = mk(in && i == j ? v.x - shift.v[b] : v.x, v.y);
 }
 
-// Step kb: block row kb of U = L^H from W, and (workgroup 0 of each matrix) the inverse of its
-// diagonal block into Li.  flag[b] is set when a pivot of matrix b is not positive.
+// Step kb: block row kb of U = L^H from W, and (workgroup 0 of matrices 0 and 2) the inverse of
+// its diagonal block into Li[0] and Li[1].  flag[b] is set when a pivot of matrix b is not positive.
 __global__ __launch_bounds__(256) void k_chol_step(int np, int kb, const cplx* __restrict__ W, cplx* __restrict__ U,
                                                    cplx* __restrict__ Li, int* __restrict__ flag) {
   __shared__ cplx rowb[2][CH_NB], colb[2][CH_NB];
@@ -382,7 +384,7 @@ __global__ __launch_bounds__(256) void k_chol_step(int np, int kb, const cplx* _
       const cplx v = i > j ? cscale(a[x][y], s) : mk(i == j ? s : 0.0, 0.0);
       Ar[j][i] = v.x;   // [k][m]
       Ai[j][i] = v.y;
-      if (blockIdx.x == 0 && b == 0) Li[(k0 + i) + (int64_t)np * (k0 + j)] = v;
+      if (blockIdx.x == 0 && b != 1) Li[nn * (b >> 1) + (k0 + i) + (int64_t)np * (k0 + j)] = v;
     }
   }
   __syncthreads();
@@ -500,40 +502,116 @@ __global__ void k_lanczos_start(int n, cplx* __restrict__ v) {
 }  // namespace
 
 int64_t chol_np(int64_t n) { return (n + CH_NB - 1) / CH_NB * CH_NB; }
-int64_t chol_work_elems(int64_t n) { return 4 * chol_np(n) * chol_np(n); }
+int64_t chol_work_elems(int64_t n, int nmat) { return 2 * nmat * chol_np(n) * chol_np(n); }
 
-void chol_inverse(hipStream_t s, int64_t n, const cplx* S, int64_t lds, double sigma, cplx* work, cplx* Li, int* flags) {
+void chol_factor(hipStream_t s, int64_t n, const cplx* S, int64_t lds, int nmat, const double* shifts, cplx* work,
+                 cplx* Li, int* flags) {
   const int64_t np = chol_np(n), nn = np * np;
-  DC2_CHECK(n >= 1 && n <= 4096, 1, "chol_inverse: n must be in 1..4096");
+  DC2_CHECK(n >= 1 && n <= 4096 && nmat >= 1 && nmat <= 3, 1, "chol_factor: n must be in 1..4096");
   const int nb = (int)(np / CH_NB);
   cplx* W = work;
-  cplx* U = W + 2 * nn;
-  const cplx one = mk(1.0, 0.0), mone = mk(-1.0, 0.0), zero = mk(0.0, 0.0);
-  DC2_HIP(hipMemsetAsync(flags, 0, 2 * sizeof(int), s));
-  hipLaunchKernelGGL(k_chol_pack, dim3(cdiv(nn, 256)), dim3(256), 0, s, (int)n, (int)np, S, lds, sigma, W);
-  fill_zero(s, Li, nn);
+  cplx* U = W + nmat * nn;
+  Shifts sh{{0.0, 0.0, 0.0}};
+  for (int b = 0; b < nmat; ++b) sh.v[b] = shifts[b];
+  DC2_HIP(hipMemsetAsync(flags, 0, 3 * sizeof(int), s));
+  hipLaunchKernelGGL(k_chol_pack, dim3(cdiv(nn, 256)), dim3(256), 0, s, (int)n, (int)np, S, lds, nmat, sh, W);
+  fill_zero(s, Li, nmat == 3 ? 2 * nn : nn);
   for (int kb = 0; kb < nb; ++kb) {
-    hipLaunchKernelGGL(k_chol_step, dim3(nb - kb, 2), dim3(256), 0, s, (int)np, kb, W, U, Li, flags);
+    hipLaunchKernelGGL(k_chol_step, dim3(nb - kb, nmat), dim3(256), 0, s, (int)np, kb, W, U, Li, flags);
     const int64_t k0 = (int64_t)kb * CH_NB, k1 = k0 + CH_NB;
-    zherk_trailing(s, np - k1, CH_NB, U + k0 + np * k1, np, nn, W + k1 + np * k1, np, nn, 2);
+    zherk_trailing(s, np - k1, CH_NB, U + k0 + np * k1, np, nn, W + k1 + np * k1, np, nn, nmat);
   }
   DC2_HIP(hipGetLastError());
-  // merges of neighbouring blocks (sizes in units of CH_NB): blocks of b, the last one shorter;
-  // T (the first half of W) holds Z U12^H
-  for (int64_t b = 1; b < nb; b *= 2) {
-    const int64_t pairs = nb / (2 * b), step = 2 * b * CH_NB, h = b * CH_NB;
+}
+
+void chol_invert(hipStream_t s, int64_t n, cplx* work, int nmat, int b, cplx* Li) {
+  const int64_t np = chol_np(n), nn = np * np;
+  const int nb = (int)(np / CH_NB);
+  cplx* W = work;
+  const cplx* U = work + nmat * nn + nn * b;
+  const cplx one = mk(1.0, 0.0), mone = mk(-1.0, 0.0), zero = mk(0.0, 0.0);
+  // merges of neighbouring blocks (sizes in units of CH_NB): blocks of c, the last one shorter;
+  // T (in W, which the factorisation no longer needs) holds Z U12^H
+  for (int64_t c = 1; c < nb; c *= 2) {
+    const int64_t pairs = nb / (2 * c), step = 2 * c * CH_NB, h = c * CH_NB;
     if (pairs > 0) {
       zgemm(s, 'N', 'C', h, h, h, one, Li + h + np * h, np, step * (np + 1), U + np * h, np, step * (np + 1), zero, W, h,
             h * h, pairs);
       zgemm(s, 'N', 'N', h, h, h, mone, W, h, h * h, Li, np, step * (np + 1), zero, Li + h, np, step * (np + 1), pairs);
     }
-    const int64_t rest = nb - 2 * b * pairs;   // a full block and a shorter one remain
-    if (rest > b) {
-      const int64_t o = pairs * step, t = (rest - b) * CH_NB;
+    const int64_t rest = nb - 2 * c * pairs;   // a full block and a shorter one remain
+    if (rest > c) {
+      const int64_t o = pairs * step, t = (rest - c) * CH_NB;
       zgemm(s, 'N', 'C', t, h, t, one, Li + (o + h) * (np + 1), np, 0, U + o + np * (o + h), np, 0, zero, W, t, 0, 1);
       zgemm(s, 'N', 'N', t, h, h, mone, W, t, 0, Li + o * (np + 1), np, 0, zero, Li + (o + h) + np * o, np, 0, 1);
     }
   }
+}
+
+void chol_inverse(hipStream_t s, int64_t n, const cplx* S, int64_t lds, double sigma, cplx* work, cplx* Li, int* flags) {
+  const double shifts[2] = {0.0, sigma};
+  chol_factor(s, n, S, lds, 2, shifts, work, Li, flags);
+  chol_invert(s, n, work, 2, 0, Li);
+}
+
+// ------------------------------------------------------------------ the lowest eigenvectors
+//
+// Subspace iteration with (G + delta)^-1 = L^-H L^-1 on LOW_P columns: two products with the
+// explicit inverse factor and an orthonormalisation by the Cholesky factor of the columns'
+// 64 x 64 Gram matrix per step.
+
+namespace {
+
+// start columns: unit-modulus entries of an integer hash
+__global__ void k_low_start(int64_t count, int n, cplx* __restrict__ x) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= count) return;
+  uint64_t z = 0x9E3779B97F4A7C15ull * (uint64_t)(i + 1);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  double sn, cs;
+  sincospi(2.0 * (double)(z >> 11) * 0x1.0p-53, &sn, &cs);
+  const double s = 1.0 / sqrt((double)n);
+  x[i] = mk(cs * s, sn * s);
+}
+
+}  // namespace
+
+int64_t low_work_elems(int64_t n) { return 2 * n * LOW_P + 2 * 3 * LOW_P * LOW_P + 64; }
+
+// X <- X L^-H with X^H X = L L^H, twice (the Gram matrix of the iterated columns is far from 1)
+static void low_orth(hipStream_t s, int64_t n, cplx* X, cplx* Y, cplx* small, int* flags, int passes) {
+  const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
+  const int64_t p = LOW_P, pp = p * p;
+  cplx *Gm = small, *U = small + pp, *Li = small + 2 * pp;
+  for (int q = 0; q < passes; ++q) {
+    zgemm(s, 'C', 'N', p, p, n, one, X, n, 0, X, n, 0, zero, Gm, p, 0, 1);
+    hipLaunchKernelGGL(k_chol_step, dim3(1, 1), dim3(256), 0, s, (int)p, 0, Gm, U, Li, flags);
+    zgemm(s, 'N', 'C', n, p, p, one, X, n, 0, Li, p, 0, zero, Y, n, 0, 1);
+    DC2_HIP(hipMemcpyAsync(X, Y, n * p * sizeof(cplx), hipMemcpyDeviceToDevice, s));
+  }
+}
+
+void low_start(hipStream_t s, int64_t n, cplx* X) {
+  hipLaunchKernelGGL(k_low_start, dim3(cdiv(n * LOW_P, 256)), dim3(256), 0, s, n * LOW_P, (int)n, X);
+  DC2_HIP(hipGetLastError());
+}
+
+void low_iterate(hipStream_t s, int64_t n, const cplx* G, const cplx* Li, int steps, cplx* X, cplx* work, cplx* H,
+                 int* flags) {
+  const int64_t np = chol_np(n), p = LOW_P;
+  const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
+  cplx *Y = work, *Z = Y + n * p, *small = Z + n * p;
+  DC2_HIP(hipMemsetAsync(flags, 0, 3 * sizeof(int), s));
+  for (int t = 0; t < steps; ++t) {
+    zgemm(s, 'N', 'N', n, p, n, one, Li, np, 0, X, n, 0, zero, Y, n, 0, 1);
+    zgemm(s, 'C', 'N', n, p, n, one, Li, np, 0, Y, n, 0, zero, X, n, 0, 1);
+    low_orth(s, n, X, Y, small, flags, t + 1 < steps ? 1 : 3);
+  }
+  zgemm(s, 'N', 'N', n, p, n, one, G, n, 0, X, n, 0, zero, Y, n, 0, 1);
+  zgemm(s, 'C', 'N', p, p, n, one, X, n, 0, Y, n, 0, zero, H, p, 0, 1);
+  DC2_HIP(hipGetLastError());
 }
 
 bool chol_lambda_min(hipStream_t s, int64_t n, const cplx* Li, cplx* work, double* host, double& lambda) {

@@ -168,13 +168,26 @@ int64_t cg_work_bytes(int64_t n, int64_t npert);
 bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const cplx* Y, const double* alpha,
                   void* work, int* host2, double* partial, double* out2, int* iterations = nullptr);
 
-// Li (chol_np(n) squared, leading dimension chol_np(n)) = L^-1 of the Hermitian S = L L^H (upper
-// triangle read), lower triangular with the unit matrix past n; flags[0] is set when S, flags[1]
-// when S - sigma I is not positive definite (two ints of device memory).  work:
-// chol_work_elems(n) complex elements; asynchronous on s.
+// The Cholesky factors of S - shift_b I = L L^H (n x n, upper triangle read) for nmat <= 3 shifts
+// side by side: U = L^H in work and the diagonal blocks of L^-1 of matrices 0 and 2 in Li[0],
+// Li[1] (chol_np(n) squared each, leading dimension chol_np(n), the unit matrix past n);
+// flags[b] is set when matrix b is not positive definite (three ints of device memory).
+// chol_invert completes L^-1 of matrix b in its Li.  work: chol_work_elems(n, nmat) complex
+// elements; asynchronous on s.  chol_inverse: both for the shifts {0, sigma}, L^-1 of the first.
 int64_t chol_np(int64_t n);
-int64_t chol_work_elems(int64_t n);
+int64_t chol_work_elems(int64_t n, int nmat);
+void chol_factor(hipStream_t s, int64_t n, const cplx* S, int64_t lds, int nmat, const double* shifts, cplx* work,
+                 cplx* Li, int* flags);
+void chol_invert(hipStream_t s, int64_t n, cplx* work, int nmat, int b, cplx* Li);
 void chol_inverse(hipStream_t s, int64_t n, const cplx* S, int64_t lds, double sigma, cplx* work, cplx* Li, int* flags);
+// Orthonormal approximations X (n x LOW_P) of the lowest eigenvectors of G by subspace iteration
+// with Li of G + delta I, and H = X^H G X (LOW_P x LOW_P); work: low_work_elems(n) complex
+// elements, flags as above (set: the columns became dependent)
+constexpr int LOW_P = 64;
+int64_t low_work_elems(int64_t n);
+void low_start(hipStream_t s, int64_t n, cplx* X);
+void low_iterate(hipStream_t s, int64_t n, const cplx* G, const cplx* Li, int steps, cplx* X, cplx* work, cplx* H,
+                 int* flags);
 // the smallest eigenvalue of S from Li by Lanczos on S^-1 (n <= 2048); false when it did not
 // converge.  work: 4 n + 256 complex elements; host: 512 doubles of page-locked memory.
 bool chol_lambda_min(hipStream_t s, int64_t n, const cplx* Li, cplx* work, double* host, double& lambda);
