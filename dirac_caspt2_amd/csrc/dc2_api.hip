@@ -175,7 +175,9 @@ struct dc2_context {
   // rank-deficient nact^3 S matrices), else 0 QR (zheev), 1 D&C, 2 D&C + Jacobi, 3 Jacobi
   int eig_method = -1;
   int lane_plan = -1;        // 4 lanes: 0 D alone on lane 3, 1 D with B and F (their S/B solves
-                             // run while the transforms do), -1 1 from 256 secondary spinors
+                             // run while the transforms do), 2 B on A's lane and F on C's,
+                             // -1: 2 where A's and C's lanes are short, else 1 from 256 secondary
+                             // spinors
   bool no_thin = false;      // option "c_thin" 0: C's metric always as the m x m Gram matrix
   bool early_v = true;       // option "early_v": V of A and C on lane 3 once their blocks exist
   int ac_route = 0;          // A/C metric: 0 automatic, 1 RDM formulas (nact^3), 2 determinant space
@@ -1830,16 +1832,23 @@ void run_caspt2(dc2_context* c, int selectroot, double eshift, double* e2, doubl
   // S/B eigensolves then run beside the integral transforms instead of after them on the
   // library stream (324 spinors, 280 secondary: 90.1 against 92.7 ms per energy; 192
   // spinors, 164 secondary: 16.2 against 16.1 ms, where F on lane 3 made that lane the longest)
-  const bool bf_on_d = c->lane_plan == 1 || (c->lane_plan < 0 && ns >= 256);
+  // B on A's lane and F on C's where those are short, their metrics going without an
+  // eigendecomposition: 192 spinors, four S and B~ eigensolves of 66 rows took 5.8 ms on the
+  // library stream after the transforms (14.0 -> 12.0 ms per energy; 324 spinors, where they
+  // stood in front of D: 34.8 -> 30.4; 238 spinors with 5 active electrons 11.2 -> 9.5)
+  const bool ras = c->ras[0] + c->ras[1] + c->ras[2] != 0;
+  const bool light = !ras && c->eig_method < 0;
+  const bool bf_on_ac = c->lane_plan == 2 || (c->lane_plan < 0 && light);
+  const bool bf_on_d = !bf_on_ac && (c->lane_plan == 1 || (c->lane_plan < 0 && ns >= 256));
   std::vector<std::vector<int>> plan(std::max(1, std::min(c->nlanes, 4)));
   for (int k = 0; k < 8; ++k) {
     if (!do_sub[k]) continue;
     int lane = 0;
     if (plan.size() >= 2 && (k == 0 || k == 2)) lane = k == 0 ? 1 : std::min<int>(2, (int)plan.size() - 1);
     if (plan.size() >= 4 && (k == 3 || (bf_on_d && (k == 1 || k == 5)))) lane = 3;
+    if (plan.size() >= 4 && bf_on_ac && (k == 1 || k == 5)) lane = k == 1 ? 1 : 2;
     plan[lane].push_back(k);
   }
-  const bool ras = c->ras[0] + c->ras[1] + c->ras[2] != 0;
   hipEvent_t y1o_ready = nullptr, rot_ready = nullptr, dens_ready = nullptr, ready = nullptr;
   DC2_HIP(hipEventCreateWithFlags(&y1o_ready, hipEventDisableTiming));
   DC2_HIP(hipEventCreateWithFlags(&rot_ready, hipEventDisableTiming));
@@ -2856,7 +2865,7 @@ int dc2_set_option(dc2_context* c, const char* key, int64_t value) {
       DC2_CHECK(value == 0 || value == 1, 1, "early_v must be 0 or 1");
       c->early_v = value != 0;
     } else if (k == "lane_plan") {
-      DC2_CHECK(value >= -1 && value <= 1, 1, "lane_plan must be -1, 0 or 1");
+      DC2_CHECK(value >= -1 && value <= 2, 1, "lane_plan must be -1, 0, 1 or 2");
       c->lane_plan = (int)value;
     } else if (k == "lanes") {
       DC2_CHECK(value >= 1 && value <= 4, 1, "lanes must be 1..4");

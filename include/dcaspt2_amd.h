@@ -215,8 +215,9 @@ int dc2_get_gemm_op_stats(dc2_context* ctx, char opA, char opB, double* out);
  *                  determinant-space factorisation;
  *   "lanes":       1..4 concurrent streams (each with a host thread) for the subspace
  *                  solves (default 4: A, C, D and the rest; 3: A, C and the rest);
- *   "lane_plan":   with 4 lanes, -1 (default) B and F on D's lane from 256 secondary spinors,
- *                  0 never, 1 always;
+ *   "lane_plan":   with 4 lanes, 0 B and F on the library stream, 1 on D's lane, 2 B on A's
+ *                  lane and F on C's, -1 (default) 2 without RAS limits and with the automatic
+ *                  eigensolver choice, else 1 from 256 secondary spinors;
  *   "early_v":     1 (default) with 4 lanes, V of A and C formed on D's lane as soon as their
  *                  transformed blocks exist (the A and C lanes use it after their eigensolves),
  *                  0 on their own lanes;
