@@ -486,6 +486,89 @@ __global__ __launch_bounds__(LZ_T) void k_lanczos(int n, int j, const cplx* __re
   }
 }
 
+// Steps j0 .. j1-1 of the same iteration in one workgroup for n <= LZS_N: L^-1 stays in this
+// compute unit's reach (L2), a step is two triangular matrix-vector products and two sums.
+// Thread (row r, part q) of LZS_P = 1024 / LZS_N sums the columns k = q mod LZS_P of row r for
+// L^-1 v; a wave per column sums over rows for L^-H t.  5 us a step at n = 196 against 25 for
+// four launches.
+constexpr int LZS_N = 256, LZS_P = 1024 / LZS_N;
+__global__ __launch_bounds__(1024) void k_lanczos_small(int n, int np, int j0, int j1, const cplx* __restrict__ Li,
+                                                        cplx* __restrict__ vg, cplx* __restrict__ voldg,
+                                                        double* __restrict__ ab) {
+  __shared__ cplx v[LZS_N], vold[LZS_N], t[LZS_N], w[LZS_N], part[LZS_P][LZS_N];
+  __shared__ double red[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  auto sum = [&](double x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    __syncthreads();
+    if (lane == 0) red[wave] = x;
+    __syncthreads();
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) s += red[q];
+    return s;
+  };
+  if (tid < n) {
+    v[tid] = vg[tid];
+    vold[tid] = j0 > 0 ? voldg[tid] : mk(0.0, 0.0);
+  }
+  double bo = j0 > 0 ? ab[2 * (j0 - 1) + 1] : 0.0;
+  __syncthreads();
+  for (int j = j0; j < j1; ++j) {
+    const int r = tid % LZS_N, q = tid / LZS_N;
+    cplx acc = mk(0.0, 0.0);
+    if (r < n)
+      for (int k = q; k <= r; k += LZS_P) cfma(acc, Li[r + (int64_t)np * k], v[k]);
+    part[q][r] = acc;
+    __syncthreads();
+    if (tid < n) {
+      cplx s = part[0][tid];
+#pragma unroll
+      for (int u = 1; u < LZS_P; ++u) s = cadd(s, part[u][tid]);
+      t[tid] = s;
+    }
+    __syncthreads();
+    for (int k = wave; k < n; k += 16) {   // w_k = sum_{i >= k} conj(Li_ik) t_i
+      cplx a = mk(0.0, 0.0);
+#pragma unroll
+      for (int u = 0; u < LZS_N / 64; ++u) {
+        const int i = lane + 64 * u;
+        if (i >= k && i < n) cfma(a, cconj(Li[i + (int64_t)np * k]), t[i]);
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        a.x += __shfl_xor(a.x, o, 64);
+        a.y += __shfl_xor(a.y, o, 64);
+      }
+      if (lane == 0) w[k] = a;
+    }
+    __syncthreads();
+    cplx x = mk(0.0, 0.0), y = mk(0.0, 0.0);
+    if (tid < n) {
+      x = v[tid];
+      y = mk(w[tid].x - bo * vold[tid].x, w[tid].y - bo * vold[tid].y);
+    }
+    const double a = sum(x.x * y.x + x.y * y.y);
+    y = mk(y.x - a * x.x, y.y - a * x.y);
+    const double b = sqrt(sum(cabs2(y))), ib = b > 0.0 ? 1.0 / b : 0.0;
+    if (tid < n) {
+      vold[tid] = x;
+      v[tid] = cscale(y, ib);
+    }
+    if (tid == 0) {
+      ab[2 * j] = a;
+      ab[2 * j + 1] = b;
+    }
+    bo = b;
+    __syncthreads();
+  }
+  if (tid < n) {
+    vg[tid] = v[tid];
+    voldg[tid] = vold[tid];
+  }
+}
+
 // a start vector with a part along every direction: unit-modulus entries of an integer hash
 __global__ void k_lanczos_start(int n, cplx* __restrict__ v) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -624,6 +707,10 @@ bool chol_lambda_min(hipStream_t s, int64_t n, const cplx* Li, cplx* work, doubl
   const int steps = (int)std::min<int64_t>(n, LZ_STEPS);
   for (int j = 0, seen = 0; j < steps;) {
     const int stop = std::min(steps, j + 32);
+    if (n <= LZS_N) {
+      hipLaunchKernelGGL(k_lanczos_small, dim3(1), dim3(1024), 0, s, (int)n, (int)np, j, stop, Li, v, vold, ab);
+      j = stop;
+    }
     for (; j < stop; ++j) {
       zgemm(s, 'N', 'N', n, 1, n, one, Li, np, 0, v, n, 0, zero, t, n, 0, 1);
       zgemm(s, 'C', 'N', n, 1, n, one, Li, np, 0, t, n, 0, zero, w, n, 0, 1);
