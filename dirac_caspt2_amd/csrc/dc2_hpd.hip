@@ -329,19 +329,21 @@ __global__ __launch_bounds__(256) void k_chol_step(int np, int kb, const cplx* _
       const double ip = 1.0 / piv;
       cplx rw[4];
 #pragma unroll
-      for (int y = 0; y < 4; ++y) {
-        rw[y] = rowb[par][c + 16 * y];
-        if (c + 16 * y == j) rw[y] = mk(1.0, 0.0);   // a_ij - m 1 after a_ij is dropped below: -m
-      }
+      for (int y = 0; y < 4; ++y) rw[y] = rowb[par][c + 16 * y];
+      // column j itself lies in the registers y = xj of the threads c = jr: a_ij is dropped and
+      // -m takes its place (0 - m 1)
+      const bool own = c == jr;
+      if (own) rw[xj] = mk(1.0, 0.0);
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
+      for (int x = xj; x < 4; ++x) {   // rows below 16 xj are done
         const int i = r + 16 * x;
         if (i > j) {
           const cplx m = cscale(colb[par][i], ip);
+          if (own) a[x][xj] = mk(0.0, 0.0);
 #pragma unroll
           for (int y = 0; y < 4; ++y) {
-            cplx v = c + 16 * y == j ? mk(0.0, 0.0) : a[x][y];
-            a[x][y] = csub(v, cmul(m, rw[y]));
+            a[x][y].x = fma(-m.x, rw[y].x, fma(m.y, rw[y].y, a[x][y].x));
+            a[x][y].y = fma(-m.x, rw[y].y, fma(-m.y, rw[y].x, a[x][y].y));
           }
         }
       }
@@ -518,8 +520,19 @@ __global__ __launch_bounds__(1024) void k_lanczos_small(int n, int np, int j0, i
   for (int j = j0; j < j1; ++j) {
     const int r = tid % LZS_N, q = tid / LZS_N;
     cplx acc = mk(0.0, 0.0);
-    if (r < n)
-      for (int k = q; k <= r; k += LZS_P) cfma(acc, Li[r + (int64_t)np * k], v[k]);
+    if (r < n) {
+      // eight loads in flight (past the diagonal L^-1 holds zeros; np >= n columns)
+      for (int k0 = q; k0 <= r; k0 += 8 * LZS_P) {
+        cplx l[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int k = k0 + u * LZS_P;
+          l[u] = k <= r ? Li[r + (int64_t)np * k] : mk(0.0, 0.0);
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) cfma(acc, l[u], v[min(k0 + u * LZS_P, LZS_N - 1)]);
+      }
+    }
     part[q][r] = acc;
     __syncthreads();
     if (tid < n) {
@@ -529,19 +542,35 @@ __global__ __launch_bounds__(1024) void k_lanczos_small(int n, int np, int j0, i
       t[tid] = s;
     }
     __syncthreads();
-    for (int k = wave; k < n; k += 16) {   // w_k = sum_{i >= k} conj(Li_ik) t_i
-      cplx a = mk(0.0, 0.0);
+    for (int k0 = wave; k0 < n; k0 += 64) {   // w_k = sum_{i >= k} conj(Li_ik) t_i, four columns at a time
+      cplx a[4];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) a[h] = mk(0.0, 0.0);
 #pragma unroll
       for (int u = 0; u < LZS_N / 64; ++u) {
         const int i = lane + 64 * u;
-        if (i >= k && i < n) cfma(a, cconj(Li[i + (int64_t)np * k]), t[i]);
+        if (64 * u >= n) break;   // uniform
+        cplx l[4];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const int k = k0 + 16 * h;
+          l[h] = (k < n && i >= k && i < n) ? Li[i + (int64_t)np * k] : mk(0.0, 0.0);
+        }
+        const cplx ti = i < n ? t[i] : mk(0.0, 0.0);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) cfma(a[h], cconj(l[h]), ti);
       }
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        a.x += __shfl_xor(a.x, o, 64);
-        a.y += __shfl_xor(a.y, o, 64);
-      }
-      if (lane == 0) w[k] = a;
+      for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          a[h].x += __shfl_xor(a[h].x, o, 64);
+          a[h].y += __shfl_xor(a[h].y, o, 64);
+        }
+      if (lane == 0)
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          if (k0 + 16 * h < n) w[k0 + 16 * h] = a[h];
     }
     __syncthreads();
     cplx x = mk(0.0, 0.0), y = mk(0.0, 0.0);
@@ -706,7 +735,7 @@ bool chol_lambda_min(hipStream_t s, int64_t n, const cplx* Li, cplx* work, doubl
   hipLaunchKernelGGL(k_lanczos_start, dim3(cdiv(n, 256)), dim3(256), 0, s, (int)n, v);
   const int steps = (int)std::min<int64_t>(n, LZ_STEPS);
   for (int j = 0, seen = 0; j < steps;) {
-    const int stop = std::min(steps, j + 32);
+    const int stop = std::min(steps, j + (j == 0 ? 24 : 16));
     if (n <= LZS_N) {
       hipLaunchKernelGGL(k_lanczos_small, dim3(1), dim3(1024), 0, s, (int)n, (int)np, j, stop, Li, v, vold, ab);
       j = stop;
