@@ -3,7 +3,7 @@
 // of this library instead of the context's grow-only scratch, for callers that cannot
 // allocate device memory (code under HIP graph capture, tight serving loops).
 //
-// The array `scratch` has a fixed size of 64 MiB on every device the entry point runs on,
+// The array `scratch` has a fixed size of 64 MiB (and the padding of the slices) on every device the entry point runs on,
 // held until the process ends.  Its device address is looked up once per device
 // (hipGetSymbolAddress with that device current, on the entry point's first call there);
 // host code never passes the array's name to a kernel, only that address.  All calls on
@@ -28,7 +28,10 @@ namespace {
 constexpr int64_t kScratchBytes = 64ll << 20;
 constexpr int kMaxDevices = 64;
 
-__device__ __align__(256) int8_t scratch[kScratchBytes];
+// The products taken are those whose digits fit the documented size; the slices are stored in
+// blocks of 16 rows and columns, at most 3 x 15 more of them in all.
+constexpr int64_t kPadBytes = 8 * 3 * 15 * 2 * 4096;
+__device__ __align__(256) int8_t scratch[kScratchBytes + kPadBytes + 512];
 
 std::mutex g_scratch_mu;
 int8_t* g_scratch_ptr[kMaxDevices] = {};   // address of `scratch` on each device
@@ -57,7 +60,8 @@ extern "C" int dc2_zgemm_split_noalloc(dc2_context* c, int32_t slices, char opB,
     DC2_CHECK(slices >= 3 && slices <= 8, 1, "dc2_zgemm_split_noalloc: slices must be in 3..8");
     DC2_CHECK(lda >= K && ldb >= K && ldc >= std::max<int64_t>(M, 1), 1, "leading dimension too small");
     const int64_t wb = (zgemm_ozaki_work_bytes(slices, M, N, K) + 255) / 256 * 256;
-    const int64_t need = wb + (M + N) * (int64_t)sizeof(int);
+    const int64_t digits = (int64_t)slices * (M + 2 * N) * 64 * ((K + 31) / 32);
+    const int64_t need = (digits + 255) / 256 * 256 + (M + N) * (int64_t)sizeof(int);
     DC2_CHECK(need <= kScratchBytes, 1,
               "dc2_zgemm_split_noalloc: the product needs " + std::to_string(need) +
                   " bytes of scratch, more than the fixed " + std::to_string(kScratchBytes) +
