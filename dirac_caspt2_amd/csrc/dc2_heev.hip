@@ -1,7 +1,7 @@
 // Hermitian eigensolver for 3 <= n <= 2048 (the matrix its upper triangle defines, as
 // rocSOLVER's fill_upper): Householder tridiagonalisation in one persistent
 // kernel, divide and conquer on the real tridiagonal (this library's, dc2_tridc.hip, or
-// rocSOLVER dstedc), back-transformation with one wave per eigenvector.
+// rocSOLVER dstedc), back-transformation in blocks of reflectors (16 lanes per eigenvector below n = 256).
 //
 // Tridiagonalisation (k_hetrd).  Step k (k = 0 .. n-3) applies the reflector
 // H_k = I - tau_k v_k v_k^H, v_k supported on rows k+1 .. n-1, to the trailing block
@@ -16,7 +16,7 @@
 // Layout: workgroup w of nwg owns the columns j = w + nwg * l (l = wave + 8 c, c < CPW), held
 // in registers for the whole reduction; lane L of a wave holds rows L + 64 s.  Per step:
 //   (a) every workgroup forms p_j for its columns (a wave reduction per column) and a partial
-//       of Re(v^H p); the owner of column k+1 publishes that column as it stands;
+//       of Re(v^H p); the owner of column k+1 has published it at the end of step k-1;
 //   -- one grid barrier --
 //   (b) every workgroup reads p, the partials and column k+1, updates its columns, applies
 //       the same update to its copy of column k+1 and derives reflector k+1 from it.
@@ -244,6 +244,22 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
   // the loads of the owned columns complete here, once, rather than being waited for again
   // before every store that might use them
   __builtin_amdgcn_s_waitcnt(0);
+  // the owner of column k+1 publishes it for step k as soon as it is up to date: its stores
+  // complete behind the reflector and the products, not between them and the barrier (half of
+  // NC by the parity of k; the step before last has been read by all, see the barrier)
+  auto publish = [&](int k) {
+    cplx* NC = w.NC + (int64_t)(k & 1) * n;
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+      if (col[c] == k + 1) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          const int i = lane + 64 * s;
+          if (i > k && i < n) st_coherent(NC + i, a[c][s]);
+        }
+      }
+  };
+  publish(0);
   reflector(n, 0, x2, sc, sv, redn, &s_tau, &s_delta, d, sub, tau, delta, Vh);
   for (int k = 0; k <= n - 3; ++k) {
     const int par = k & 1;
@@ -273,16 +289,6 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
       }
       if (lane == 0) red[wave] = part;
     }
-    // the owner publishes column k+1
-#pragma unroll
-    for (int c = 0; c < CPW; ++c)
-      if (col[c] == k + 1) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          const int i = lane + 64 * s;
-          if (i > k && i < n) st_coherent(NC + i, a[c][s]);
-        }
-      }
     if (!grid_sync(w.bar, k, w.err, t != 0.0 ? Sp + wg : nullptr, red, n, sv, Vh)) return;
     // (b) one round of coherent loads: column k+1, p and the partials (nwg <= 256, one per
     // thread, summed in the same order in every workgroup); q = p - K v is formed where used.
@@ -337,6 +343,7 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
           }
         }
       }
+      if (k < n - 3) publish(k + 1);
       // column k+1 updated by the rows this thread loaded, and its part of the next norm
       const cplx cq1 = cconj(qat(k + 1)), cv1 = cconj(sv[k + 1]);
       for (int i = k + 1 + threadIdx.x; i < n; i += HT_THREADS) {
@@ -347,6 +354,7 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
         if (i > k + 1) x2 += cabs2(x);
       }
     } else {
+      if (k < n - 3) publish(k + 1);
       for (int i = k + 1 + threadIdx.x; i < n; i += HT_THREADS)
         if (i > k + 1) x2 += cabs2(sc[i]);
     }
@@ -383,56 +391,70 @@ __global__ void k_tri_prep(int n, const cplx* __restrict__ sub, double* __restri
   if (Z && t < (int64_t)n * n) Z[t] = (t % (n + 1) == 0) ? 1.0 : 0.0;
 }
 
-// X[:, c] = H_0 H_1 ... H_{n-3} (delta .* Z[:, c]); one wave per column, 8 columns per
-// workgroup; the reflectors are staged through LDS in chunks of BT_CH (coalesced loads)
-constexpr int BT_CH = 8;
+// sums over each row of 16 lanes, the same value in all 16 (DPP: no trip through LDS)
+template <int CTRL>
+__device__ inline double dpp_add(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+  return x + __hiloint2double(hi, lo);
+}
+__device__ inline cplx row16_sum(cplx x) {
+  x = mk(dpp_add<0xB1>(x.x), dpp_add<0xB1>(x.y));     // quad_perm 1,0,3,2
+  x = mk(dpp_add<0x4E>(x.x), dpp_add<0x4E>(x.y));     // quad_perm 2,3,0,1
+  x = mk(dpp_add<0x141>(x.x), dpp_add<0x141>(x.y));   // row_half_mirror
+  return mk(dpp_add<0x140>(x.x), dpp_add<0x140>(x.y));   // row_mirror
+}
+
+// X[:, c] = H_0 H_1 ... H_{n-3} (delta .* Z[:, c]), n <= 16 S: 16 lanes per column (lane r holds
+// the rows r + 16 s), 16 columns per workgroup of four waves; the reflectors are staged through
+// LDS 64 KB at a time.  A serial chain of n - 2 dot products: with 16 lanes
+// their sums stay inside DPP rows and four columns share each LDS read (n = 93: 42 us
+// against 72 with a wave per column, whose sums took six trips through LDS)
 template <int S>
-__global__ __launch_bounds__(512) void k_hetrd_back(int n, const double* __restrict__ Z, const cplx* __restrict__ delta,
+__global__ __launch_bounds__(256) void k_hetrd_back(int n, const double* __restrict__ Z, const cplx* __restrict__ delta,
                                                    const double* __restrict__ tau, const cplx* __restrict__ Vh,
                                                    cplx* __restrict__ X, int64_t ldx) {
-  __shared__ cplx vs[BT_CH][64 * S];
-  __shared__ double ts[BT_CH];
-  const int lane = threadIdx.x & 63;
-  const int c = blockIdx.x * 8 + (threadIdx.x >> 6);
-  const bool active = c < n;   // every wave takes part in the chunk loads
+  constexpr int CH = 4096 / (16 * S);   // reflectors in 64 KB
+  __shared__ cplx vs[CH][16 * S];
+  __shared__ double ts[CH];
+  const int r = threadIdx.x & 15, c = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const bool active = c < n;   // every lane takes part in the chunk loads and the sums
   cplx x[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int i = lane + 64 * s;
+    const int i = r + 16 * s;
     x[s] = (active && i < n) ? cscale(delta[i], Z[i + (int64_t)n * c]) : mk(0.0, 0.0);
   }
-  for (int k0 = n - 3; k0 >= 0; k0 -= BT_CH) {
-    const int nk = min(BT_CH, k0 + 1);   // reflectors k0, k0-1, ..., k0-nk+1
+  for (int k0 = n - 3; k0 >= 0; k0 -= CH) {
+    const int nk = min(CH, k0 + 1);   // reflectors k0, k0-1, ..., k0-nk+1
     __syncthreads();
-    for (int idx = threadIdx.x; idx < nk * n; idx += 512) {
-      const int kk = idx / n, i = idx - kk * n, k = k0 - kk;
-      vs[kk][i] = i > k ? Vh[i + (int64_t)n * k] : mk(0.0, 0.0);
+    for (int idx = threadIdx.x; idx < nk * 16 * S; idx += 256) {
+      const int kk = idx / (16 * S), i = idx % (16 * S), k = k0 - kk;
+      vs[kk][i] = i > k && i < n ? Vh[i + (int64_t)n * k] : mk(0.0, 0.0);
     }
     if (threadIdx.x < nk) ts[threadIdx.x] = tau[k0 - threadIdx.x];
     __syncthreads();
-    if (!active) continue;
     for (int kk = 0; kk < nk; ++kk) {
       const double t = ts[kk];
       if (t == 0.0) continue;
-      cplx dot = mk(0.0, 0.0);
+      cplx v[S], dot = mk(0.0, 0.0), dot1 = mk(0.0, 0.0);
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        const int i = lane + 64 * s;
-        if (i < n) cfma(dot, cconj(vs[kk][i]), x[s]);
-      }
-      dot = wave_sum(dot);
-      const cplx f = mk(t * dot.x, t * dot.y);
+      for (int s = 0; s < S; ++s) v[s] = vs[kk][r + 16 * s];
 #pragma unroll
-      for (int s = 0; s < S; ++s) {
-        const int i = lane + 64 * s;
-        if (i < n) x[s] = csub(x[s], cmul(vs[kk][i], f));
+      for (int s = 0; s < S; s += 2) {
+        cfma(dot, cconj(v[s]), x[s]);
+        cfma(dot1, cconj(v[s + 1]), x[s + 1]);
       }
+      dot = row16_sum(mk(dot.x + dot1.x, dot.y + dot1.y));
+      const cplx f = mk(-t * dot.x, -t * dot.y);
+#pragma unroll
+      for (int s = 0; s < S; ++s) cfma(x[s], v[s], f);
     }
   }
   if (!active) return;
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    const int i = lane + 64 * s;
+    const int i = r + 16 * s;
     if (i < n) X[i + ldx * c] = x[s];
   }
 }
@@ -455,32 +477,30 @@ __global__ void k_dz(int n, const double* __restrict__ Z, const cplx* __restrict
 }
 
 // T of every panel from its Gram matrix G = V^H V (nb x nb per panel, column-major) and tau;
-// one workgroup of BT_NB threads per panel with G and T in LDS, thread i owns row i of T.
+// one workgroup per panel with G and T in LDS, four threads per row of T, which share its dot
+// products (a serial chain of 64 columns: 49 us; one thread per row 123).
 // Reflectors past nrefl (and those with tau = 0) give zero columns.
-__global__ __launch_bounds__(BT_NB) void k_wy_t(int nrefl, const double* __restrict__ tau,
-                                                const cplx* __restrict__ G, cplx* __restrict__ T) {
+__global__ __launch_bounds__(4 * BT_NB) void k_wy_t(int nrefl, const double* __restrict__ tau,
+                                                    const cplx* __restrict__ G, cplx* __restrict__ T) {
   __shared__ cplx gs[BT_NB][BT_NB + 1], ts[BT_NB][BT_NB + 1];   // [column][row]
-  const int p = blockIdx.x, i = threadIdx.x, a = p * BT_NB;
+  const int p = blockIdx.x, i = threadIdx.x >> 2, q = threadIdx.x & 3, a = p * BT_NB;
   const cplx* g = G + (int64_t)BT_NB * BT_NB * p;
-  for (int j = 0; j < BT_NB; ++j) gs[j][i] = g[i + BT_NB * j];
+  for (int e = threadIdx.x; e < BT_NB * BT_NB; e += 4 * BT_NB) gs[e / BT_NB][e % BT_NB] = g[e];
   __syncthreads();
   for (int j = 0; j < BT_NB; ++j) {
     const double tj = a + j < nrefl ? tau[a + j] : 0.0;
     // T[i][j] = -tau_j sum_{l=i}^{j-1} T[i][l] G[l][j] (i < j), tau_j (i = j), 0 (i > j);
     // column j reads only columns l < j, written in earlier steps
-    cplx v = mk(0.0, 0.0);
-    if (i < j && tj != 0.0) {
-      cplx acc = mk(0.0, 0.0);
-      for (int l = i; l < j; ++l) cfma(acc, ts[l][i], gs[j][l]);
-      v = mk(-tj * acc.x, -tj * acc.y);
-    } else if (i == j) {
-      v = mk(tj, 0.0);
-    }
-    ts[j][i] = v;
+    cplx acc = mk(0.0, 0.0);
+    if (tj != 0.0)
+      for (int l = i + q; l < j; l += 4) cfma(acc, ts[l][i], gs[j][l]);
+    acc = mk(dpp_add<0xB1>(acc.x), dpp_add<0xB1>(acc.y));
+    acc = mk(dpp_add<0x4E>(acc.x), dpp_add<0x4E>(acc.y));
+    if (q == 0) ts[j][i] = i < j ? mk(-tj * acc.x, -tj * acc.y) : i == j ? mk(tj, 0.0) : mk(0.0, 0.0);
     __syncthreads();
   }
   cplx* t = T + (int64_t)BT_NB * BT_NB * p;
-  for (int j = 0; j < BT_NB; ++j) t[i + BT_NB * j] = ts[j][i];
+  for (int e = threadIdx.x; e < BT_NB * BT_NB; e += 4 * BT_NB) t[e] = ts[e / BT_NB][e % BT_NB];
 }
 
 // T of a merged panel: its four panels' T on the diagonal blocks (the rest zero)
@@ -510,7 +530,7 @@ void back_blocked(hipStream_t s, int n, const double* Z, const cplx* delta, cons
   // reflector are zero, so are their T columns)
   zgemm(s, 'C', 'N', BT_NB, BT_NB, n, one, Vh, n, (int64_t)n * BT_NB, Vh, n, (int64_t)n * BT_NB, zero, G, BT_NB,
         (int64_t)BT_NB * BT_NB, np);
-  hipLaunchKernelGGL(k_wy_t, dim3(np), dim3(BT_NB), 0, s, nrefl, tau, G, T);
+  hipLaunchKernelGGL(k_wy_t, dim3(np), dim3(4 * BT_NB), 0, s, nrefl, tau, G, T);
   zgemm(s, 'C', 'N', BT_SB, BT_SB, n, one, Vh, n, (int64_t)n * BT_SB, Vh, n, (int64_t)n * BT_SB, zero, GS, ld, sq,
         nps);
   hipLaunchKernelGGL(k_ts_diag, dim3(4 * 16, nps), dim3(256), 0, s, T, TS);
@@ -581,7 +601,7 @@ hipError_t launch_hetrd(hipStream_t s, int nwg, int n, const cplx* A, int64_t ld
 template <int S>
 void launch_back(hipStream_t s, int n, const double* Z, const cplx* delta, const double* tau, const cplx* Vh, cplx* X,
                  int64_t ldx) {
-  hipLaunchKernelGGL((k_hetrd_back<S>), dim3(cdiv(n, 8)), dim3(512), 0, s, n, Z, delta, tau, Vh, X, ldx);
+  hipLaunchKernelGGL((k_hetrd_back<S>), dim3(cdiv(n, 16)), dim3(256), 0, s, n, Z, delta, tau, Vh, X, ldx);
 }
 
 // device time of every tridiagonalisation, by matrix size (HIP events around the launch)
@@ -728,10 +748,9 @@ bool heev_native(hipStream_t s, rocblas_handle h, int n, cplx* A, int64_t lda, d
     DC2_HIP(hipGetLastError());
     return true;
   }
-  if (n <= 128) launch_back<2>(s, n, Z, delta, tau, Vh, A, lda);
-  else if (n <= 256) launch_back<4>(s, n, Z, delta, tau, Vh, A, lda);
-  else if (n <= 512) launch_back<8>(s, n, Z, delta, tau, Vh, A, lda);
-  else if (n <= 768) launch_back<12>(s, n, Z, delta, tau, Vh, A, lda);
+  // below BT_BLOCKED_MIN
+  if (n <= 64) launch_back<4>(s, n, Z, delta, tau, Vh, A, lda);
+  else if (n <= 128) launch_back<8>(s, n, Z, delta, tau, Vh, A, lda);
   else launch_back<16>(s, n, Z, delta, tau, Vh, A, lda);
   DC2_HIP(hipGetLastError());
   return true;

@@ -189,8 +189,11 @@ __global__ __launch_bounds__(256) void k_dc_deflate(int n, int depth, const doub
                                                     const double* __restrict__ Din, const double* __restrict__ Q,
                                                     DcWork w) {
   __shared__ double sd[DC_NMAX], sz[DC_NMAX];
-  __shared__ int srt[DC_NMAX];
+  __shared__ int srt[DC_NMAX], prv[DC_NMAX];
+  __shared__ unsigned char gone[DC_NMAX];   // 1: small, 2: rotated away
   __shared__ double red[2][256];
+  __shared__ int sci[256], scf[256];
+  __shared__ unsigned long long pairs[DC_NMAX / 64];
   const int j = blockIdx.x, tid = threadIdx.x;
   const int a = node_lo(n, depth, j), m = node_lo(n, depth + 1, 2 * j + 1), c = node_lo(n, depth, j + 1);
   const int N = c - a, n1 = m - a, n2 = c - m;
@@ -276,76 +279,121 @@ __global__ __launch_bounds__(256) void k_dc_deflate(int n, int depth, const doub
     }
   }
   __syncthreads();
-  if (tid != 0) return;
-  // the serial scan; the next entry's loads are issued one iteration ahead, and the test for
-  // a close pair, |(d_j - d_p) c s| <= tol with c s = -z_j z_p / (z_j^2 + z_p^2), is made
-  // without a square root or division (those are needed only for a rotation)
-  int K = 0, nf = 0, nr = 0, pj = -1;
-  double pd = 0.0, pz = 0.0;
-  int jn = srt[0];
-  double dn = sd[0], zn = sz[0];
-  for (int k = 0; k < N; ++k) {
-    const int jj = jn;
-    const double dj = dn, zj = zn;
-    if (k + 1 < N) {
-      jn = srt[k + 1];
-      dn = sd[k + 1];
-      zn = sz[k + 1];
-    }
-    if (rho * fabs(zj) <= tol) {
-      w.dfd[a + nf] = dj;
-      w.dfc[a + nf] = jj;
-      ++nf;
-      continue;
-    }
-    if (pj < 0) {
-      pj = jj;
-      pd = dj;
-      pz = zj;
-      continue;
-    }
+  // Per sorted entry, in parallel: small (rho |z| <= tol, an eigenpair as it stands), prv (the
+  // entry before it that is not), and whether the rotation with that one is negligible as both
+  // stand: |(d_j - d_p) c s| <= tol with c s = -z_j z_p / (z_j^2 + z_p^2), without a square root
+  // or division (those are needed only for a rotation).  A rotation changes the entry that the
+  // next test meets, so one thread follows each chain of rotations from its first pair; between
+  // chains nothing is serial (a scan of every entry by one thread, 0.2 us an entry: 0.57 ms
+  // over the merges at n = 1274, now 0.065).
+  const int lane = tid & 63, wave = tid >> 6;
+  const int per = (N + 255) / 256, k0 = tid * per, k1 = min(N, k0 + per);
+  int last = -1;
+  for (int k = k0; k < k1; ++k)
+    if (!(rho * fabs(sz[k]) <= tol)) last = k;
+  sci[tid] = last;
+  __syncthreads();
+  for (int s = 1; s < 256; s <<= 1) {   // inclusive running maximum
+    const int o = tid >= s ? sci[tid - s] : -1;
+    __syncthreads();
+    sci[tid] = max(sci[tid], o);
+    __syncthreads();
+  }
+  last = tid > 0 ? sci[tid - 1] : -1;
+  for (int k = k0; k < k1; ++k) {
+    const bool sm = rho * fabs(sz[k]) <= tol;
+    prv[k] = sm ? -2 : last;
+    gone[k] = sm;
+    if (!sm) last = k;
+  }
+  __syncthreads();
+  auto close = [&](double dj, double zj, double pd, double pz) {
     const double z2 = zj * zj + pz * pz;
-    const bool scaled_ok = z2 > 1e-280 && z2 < 1e280;   // else the exact form below
-    bool close;
-    if (scaled_ok) {
-      close = fabs((dj - pd) * zj * pz) <= tol * z2;
-    } else {
-      const double t0 = dc_hyp(zj, pz);
-      close = fabs((dj - pd) * (zj / t0) * (pz / t0)) <= tol;
+    if (z2 > 1e-280 && z2 < 1e280) return fabs((dj - pd) * zj * pz) <= tol * z2;
+    const double t0 = dc_hyp(zj, pz);   // the exact form
+    return fabs((dj - pd) * (zj / t0) * (pz / t0)) <= tol;
+  };
+  for (int b = wave; b * 64 < N; b += 4) {
+    const int k = 64 * b + lane;
+    const bool f = k < N && prv[k] >= 0 && close(sd[k], sz[k], sd[max(prv[min(k, N - 1)], 0)], sz[max(prv[min(k, N - 1)], 0)]);
+    const unsigned long long m64 = __ballot(f);
+    if (lane == 0) pairs[b] = m64;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int nr = 0, done = -1;   // entries up to done have been met by a chain
+    for (int b = 0; b * 64 < N; ++b) {
+      unsigned long long m64 = pairs[b];
+      while (m64) {
+        int k = 64 * b + __ffsll(m64) - 1;
+        m64 &= m64 - 1;
+        if (k <= done) continue;
+        int p = prv[k];
+        double pd = sd[p], pz = sz[p];
+        while (true) {   // rotate p and k; the first is an eigenpair, the second goes on
+          const double dj = sd[k], zj = sz[k];
+          const double t = dc_hyp(zj, pz);
+          const double cs = zj / t, sn = -pz / t;
+          w.rp[a + nr] = srt[p];
+          w.rq[a + nr] = srt[k];
+          w.rc[a + nr] = cs;
+          w.rs[a + nr] = sn;
+          ++nr;
+          sd[p] = pd * cs * cs + dj * sn * sn;
+          gone[p] = 2;
+          prv[k] = -3 - p;   // p is deflated where the scan reaches k
+          pd = pd * sn * sn + dj * cs * cs;
+          pz = t;
+          sd[k] = pd;
+          sz[k] = pz;
+          p = k;
+          do ++k;
+          while (k < N && prv[k] == -2);
+          done = k;
+          if (k >= N || !close(sd[k], sz[k], pd, pz)) break;
+        }
+      }
     }
-    if (close) {
-      const double t = dc_hyp(zj, pz);
-      const double cs = zj / t, sn = -pz / t;
-      w.rp[a + nr] = pj;
-      w.rq[a + nr] = jj;
-      w.rc[a + nr] = cs;
-      w.rs[a + nr] = sn;
-      ++nr;
-      w.dfd[a + nf] = pd * cs * cs + dj * sn * sn;
-      w.dfc[a + nf] = pj;
+    w.cnt[3 * j + 2] = nr;
+  }
+  __syncthreads();
+  // the kept entries in order; the deflated ones in the order in which the scan meets them (a
+  // rotated one with its partner)
+  int nk = 0, nf = 0;
+  for (int k = k0; k < k1; ++k) {
+    nk += gone[k] == 0;
+    nf += gone[k] == 1 || prv[k] <= -3;
+  }
+  sci[tid] = nk;
+  scf[tid] = nf;
+  __syncthreads();
+  for (int s = 1; s < 256; s <<= 1) {   // inclusive sums
+    const int o = tid >= s ? sci[tid - s] : 0, of = tid >= s ? scf[tid - s] : 0;
+    __syncthreads();
+    sci[tid] += o;
+    scf[tid] += of;
+    __syncthreads();
+  }
+  nk = sci[tid] - nk;
+  nf = scf[tid] - nf;
+  for (int k = k0; k < k1; ++k) {
+    if (gone[k] == 0) {
+      w.ndd[a + nk] = sd[k];
+      w.ndz[a + nk] = sz[k];
+      w.ndc[a + nk] = srt[k];
+      ++nk;
+    }
+    const int f = gone[k] == 1 ? k : prv[k] <= -3 ? -3 - prv[k] : -1;
+    if (f >= 0) {
+      w.dfd[a + nf] = sd[f];
+      w.dfc[a + nf] = srt[f];
       ++nf;
-      pd = pd * sn * sn + dj * cs * cs;
-      pz = t;
-      pj = jj;
-    } else {
-      w.ndd[a + K] = pd;
-      w.ndz[a + K] = pz;
-      w.ndc[a + K] = pj;
-      ++K;
-      pj = jj;
-      pd = dj;
-      pz = zj;
     }
   }
-  if (pj >= 0) {
-    w.ndd[a + K] = pd;
-    w.ndz[a + K] = pz;
-    w.ndc[a + K] = pj;
-    ++K;
+  if (tid == 255) {
+    w.cnt[3 * j] = sci[255];
+    w.cnt[3 * j + 1] = scf[255];
   }
-  w.cnt[3 * j] = K;
-  w.cnt[3 * j + 1] = nf;
-  w.cnt[3 * j + 2] = nr;
 }
 
 // ------------------------------------------------------------------ rotations
@@ -353,11 +401,11 @@ __global__ __launch_bounds__(256) void k_dc_deflate(int n, int depth, const doub
 // off-diagonal blocks of Q), then applies the deflation rotations in order.  A rotation's
 // first column is the previous rotation's second one or a column not touched before, so the
 // chain is carried in a register.
-__global__ __launch_bounds__(256) void k_dc_rotate(int n, int depth, double* __restrict__ Q, DcWork w) {
+__device__ void dc_rotate(int n, int depth, int bx, double* __restrict__ Q, const DcWork& w) {
   const int j = blockIdx.y;
   const int a = node_lo(n, depth, j), m = node_lo(n, depth + 1, 2 * j + 1), c = node_lo(n, depth, j + 1);
   if (!(a < m && m < c)) return;
-  const int r = a + blockIdx.x * 256 + threadIdx.x;
+  const int r = a + bx * 256 + threadIdx.x;
   if (r >= c) return;
   double* row = Q + r;
   const int z0 = r < m ? m : a, z1 = r < m ? c : m;
@@ -378,10 +426,16 @@ __global__ __launch_bounds__(256) void k_dc_rotate(int n, int depth, double* __r
 }
 
 // ------------------------------------------------------------------ secular equation
-// One wave per root; the node's non-deflated (d, z) in LDS.
-__global__ __launch_bounds__(256) void k_dc_secular(int n, int depth, const double* __restrict__ e, DcWork w,
-                                                    int* __restrict__ info, int report) {
+// One wave per root; the node's non-deflated (d, z) in LDS.  The blocks from nsec on rotate
+// (independent work: one launch less per merge, 4-5 us).
+__global__ __launch_bounds__(256) void k_dc_secular(int n, int depth, const double* __restrict__ e,
+                                                    double* __restrict__ Q, DcWork w, int* __restrict__ info,
+                                                    int report, int nsec) {
   __shared__ double ld[DC_NMAX], lz[DC_NMAX];
+  if ((int)blockIdx.x >= nsec) {
+    dc_rotate(n, depth, blockIdx.x - nsec, Q, w);
+    return;
+  }
   const int j = blockIdx.y;
   const int K = w.cnt[3 * j];
   if (blockIdx.x * 4 >= K) return;
@@ -476,25 +530,46 @@ __global__ __launch_bounds__(256) void k_dc_secular(int n, int depth, const doub
   }
 }
 
-// ------------------------------------------------------------------ zhat
-// One wave per entry i: zhat_i^2 = (lambda_i - d_i) / rho * prod_{j != i} (lambda_j - d_i) / (d_j - d_i).
-__global__ __launch_bounds__(256) void k_dc_zhat(int n, int depth, const double* __restrict__ e, DcWork w) {
-  __shared__ double ld[DC_NMAX], lt[DC_NMAX];
+// ------------------------------------------------------------------ zhat, order
+// One wave per entry i of the node: its rank among the node's new eigenvalues (ties by entry
+// index), the eigenvalue stored at that rank, and for a non-deflated one
+// zhat_i^2 = (lambda_i - d_i) / rho * prod_{j != i} (lambda_j - d_i) / (d_j - d_i).
+__global__ __launch_bounds__(256) void k_dc_zhat(int n, int depth, const double* __restrict__ e,
+                                                 double* __restrict__ Dout, DcWork w) {
+  __shared__ double ld[DC_NMAX], lt[DC_NMAX], v[DC_NMAX];
   __shared__ int lo_[DC_NMAX];
   const int j = blockIdx.y;
+  const int a = node_lo(n, depth, j), m = node_lo(n, depth + 1, 2 * j + 1), N = node_lo(n, depth, j + 1) - a;
+  if ((int)blockIdx.x * 4 >= N) return;
   const int K = w.cnt[3 * j];
-  if (blockIdx.x * 4 >= K) return;
-  const int a = node_lo(n, depth, j), m = node_lo(n, depth + 1, 2 * j + 1);
-  const double rho = 2.0 * fabs(e[m - 1]);
-  for (int i = threadIdx.x; i < K; i += 256) {
-    ld[i] = w.ndd[a + i];
-    lt[i] = w.tau[a + i];
-    lo_[i] = w.org[a + i];
+  for (int i = threadIdx.x; i < N; i += 256) {
+    if (i < K) {
+      const int o = w.org[a + i];
+      ld[i] = w.ndd[a + i];
+      lt[i] = w.tau[a + i];
+      lo_[i] = o;
+      v[i] = w.ndd[a + o] + w.tau[a + i];
+    } else {
+      v[i] = w.dfd[a + i - K];
+    }
   }
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= N) return;
+  const double x = v[i];
+  int r = 0;
+  for (int f0 = 0; f0 < N; f0 += 64) {
+    const int f = f0 + lane;
+    const double y = f < N ? v[f] : 0.0;
+    r += __popcll(__ballot(f < N && (y < x || (y == x && f < i))));
+  }
+  if (lane == 0) {
+    Dout[a + r] = x;
+    w.pos[a + i] = r;
+  }
   if (i >= K) return;
+  const double rho = 2.0 * fabs(e[m - 1]);
   const double di = ld[i];
   double p = 1.0;
   for (int q = lane; q < K; q += 64) {
@@ -503,30 +578,6 @@ __global__ __launch_bounds__(256) void k_dc_zhat(int n, int depth, const double*
   }
   p = wave_prod(p) * (((ld[lo_[i]] - di) + lt[i]) / rho);
   if (lane == 0) w.zh[a + i] = copysign(sqrt(fmax(p, 0.0)), w.ndz[a + i]);
-}
-
-// ------------------------------------------------------------------ order
-// Thread per entry of the node: its rank among the node's new eigenvalues (ties by entry
-// index), the eigenvalue stored at that rank.
-__global__ __launch_bounds__(256) void k_dc_order(int n, int depth, double* __restrict__ Dout, DcWork w) {
-  __shared__ double v[DC_NMAX];
-  const int j = blockIdx.y;
-  const int a = node_lo(n, depth, j), c = node_lo(n, depth, j + 1), N = c - a;
-  if (blockIdx.x * 256 >= N) return;
-  const int K = w.cnt[3 * j];
-  for (int q = threadIdx.x; q < N; q += 256)
-    v[q] = q < K ? w.ndd[a + w.org[a + q]] + w.tau[a + q] : w.dfd[a + q - K];
-  __syncthreads();
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  if (q >= N) return;
-  const double x = v[q];
-  int r = 0;
-  for (int f = 0; f < N; ++f) {
-    const double y = v[f];
-    r += (y < x) || (y == x && f < q);
-  }
-  Dout[a + r] = x;
-  w.pos[a + q] = r;
 }
 
 // ------------------------------------------------------------------ eigenvectors of the update
@@ -559,54 +610,70 @@ __global__ __launch_bounds__(256) void k_dc_vec(int n, int depth, double* __rest
 // ------------------------------------------------------------------ new eigenvectors
 // Zout[a + r, a + pos[j]] = sum_i Q[a + r, a + ndc[i]] V[i, j]: 64 x 64 output tiles, four
 // waves of 2 x 2 16x16 FP64 MFMA tiles (v_mfma_f64_16x16x4f64), K in steps of 16 through LDS.
+// The next K step's elements are loaded into registers while this one's are multiplied (all
+// merges at n = 1274: 0.54 -> 0.31 ms, against loads between two barriers).  blockIdx.y = ntile:
+// the deflated columns of the rotated Q to their places, 64 rows.
 constexpr int DG_LDS = 80;
 __global__ __launch_bounds__(256) void k_dc_gemm(int n, int depth, const double* __restrict__ Q,
-                                                 const double* __restrict__ W, double* __restrict__ Zout, DcWork w) {
-  __shared__ double As[16][DG_LDS], Bs[16][DG_LDS];
-  __shared__ int cols[16];
+                                                 const double* __restrict__ W, double* __restrict__ Zout, DcWork w,
+                                                 int ntile) {
+  __shared__ double As[2][16][DG_LDS], Bs[2][16][DG_LDS];
+  __shared__ int cols[DC_NMAX];
   const int j = blockIdx.z;
   const int a = node_lo(n, depth, j), c = node_lo(n, depth, j + 1), N = c - a;
   const int K = w.cnt[3 * j];
   const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-  if (m0 >= N || n0 >= K) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if ((int)blockIdx.y == ntile) {
+    const int nf = w.cnt[3 * j + 1], r = m0 + lane;
+    if (r < N)
+      for (int f = wave; f < nf; f += 4)
+        Zout[a + r + (int64_t)n * (a + w.pos[a + K + f])] = Q[a + r + (int64_t)n * (a + w.dfc[a + f])];
+    return;
+  }
+  if (m0 >= N || n0 >= K) return;
   const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+  for (int k = tid; k < K; k += 256) cols[k] = w.ndc[a + k];
+  __syncthreads();
   d4 acc[2][2];
 #pragma unroll
   for (int x = 0; x < 2; ++x)
 #pragma unroll
     for (int y = 0; y < 2; ++y) acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
   const double* Wn = W + a + (int64_t)n * a;
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    if (tid < 16) cols[tid] = k0 + tid < K ? w.ndc[a + k0 + tid] : 0;
-    __syncthreads();
+  double ra[4], rb[4];
+  auto load = [&](int k0) {
 #pragma unroll
-    for (int e4 = tid; e4 < 64 * 16; e4 += 256) {
-      const int mm = e4 & 63, kk = e4 >> 6;
-      const int r = m0 + mm;
-      As[kk][mm] = (r < N && k0 + kk < K) ? Q[(a + r) + (int64_t)n * (a + cols[kk])] : 0.0;
+    for (int u = 0; u < 4; ++u) {
+      const int kk = k0 + wave + 4 * u, r = m0 + lane;
+      ra[u] = (r < N && kk < K) ? Q[(a + r) + (int64_t)n * (a + cols[kk])] : 0.0;
+      const int kb = k0 + (tid & 15), nn = n0 + (tid >> 4) + 16 * u;
+      rb[u] = (kb < K && nn < K) ? Wn[kb + (int64_t)n * nn] : 0.0;
     }
+  };
+  load(0);
+  for (int k0 = 0, buf = 0; k0 < K; k0 += 16, buf ^= 1) {
 #pragma unroll
-    for (int e4 = tid; e4 < 64 * 16; e4 += 256) {
-      const int kk = e4 & 15, nn = e4 >> 4;
-      Bs[kk][nn] = (k0 + kk < K && n0 + nn < K) ? Wn[(k0 + kk) + (int64_t)n * (n0 + nn)] : 0.0;
+    for (int u = 0; u < 4; ++u) {
+      As[buf][wave + 4 * u][lane] = ra[u];
+      Bs[buf][tid & 15][(tid >> 4) + 16 * u] = rb[u];
     }
-    __syncthreads();
+    __syncthreads();   // one barrier a step: the other half is written after it was last read
+    if (k0 + 16 < K) load(k0 + 16);
 #pragma unroll
     for (int kk = 0; kk < 16; kk += 4) {
       const int kl = kk + (lane >> 4);
       double av[2], bv[2];
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
-        av[x] = As[kl][wm + 16 * x + (lane & 15)];
-        bv[x] = Bs[kl][wn + 16 * x + (lane & 15)];
+        av[x] = As[buf][kl][wm + 16 * x + (lane & 15)];
+        bv[x] = Bs[buf][kl][wn + 16 * x + (lane & 15)];
       }
 #pragma unroll
       for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[x], bv[y], acc[x][y], 0, 0, 0);
     }
-    __syncthreads();
   }
   // element r of lane L of a 16x16 tile holds row (L >> 4) + 4 r, column L & 15
 #pragma unroll
@@ -622,18 +689,6 @@ __global__ __launch_bounds__(256) void k_dc_gemm(int n, int depth, const double*
         if (row < N) out[row] = acc[x][y][r];
       }
     }
-}
-
-// deflated columns of the rotated Q to their places: one workgroup per deflated entry
-__global__ __launch_bounds__(256) void k_dc_copydef(int n, int depth, const double* __restrict__ Q,
-                                                    double* __restrict__ Zout, DcWork w) {
-  const int j = blockIdx.y, f = blockIdx.x;
-  if (f >= w.cnt[3 * j + 1]) return;
-  const int a = node_lo(n, depth, j), c = node_lo(n, depth, j + 1), N = c - a;
-  const int K = w.cnt[3 * j];
-  const double* src = Q + a + (int64_t)n * (a + w.dfc[a + f]);
-  double* dst = Zout + a + (int64_t)n * (a + w.pos[a + K + f]);
-  for (int r = threadIdx.x; r < N; r += 256) dst[r] = src[r];
 }
 
 int leaf_depth(int n) {
@@ -690,15 +745,13 @@ void tri_dc(hipStream_t s, int n, double* w, const double* e, double* Z, void* w
     double* Dout = Dbuf[q ^ 1];
     double* Zout = Zbuf[q ^ 1];
     hipLaunchKernelGGL(k_dc_deflate, dim3(nodes), dim3(256), 0, s, n, depth, e, Din, Q, dw);
-    hipLaunchKernelGGL(k_dc_rotate, dim3(cdiv(nmax, 256), nodes), dim3(256), 0, s, n, depth, Q, dw);
-    hipLaunchKernelGGL(k_dc_secular, dim3(cdiv(nmax, 4), nodes), dim3(256), 0, s, n, depth, e, dw, info_dev,
-                       (int)report);
-    hipLaunchKernelGGL(k_dc_zhat, dim3(cdiv(nmax, 4), nodes), dim3(256), 0, s, n, depth, e, dw);
-    hipLaunchKernelGGL(k_dc_order, dim3(cdiv(nmax, 256), nodes), dim3(256), 0, s, n, depth, Dout, dw);
+    const int nsec = (int)cdiv(nmax, 4);
+    hipLaunchKernelGGL(k_dc_secular, dim3(nsec + cdiv(nmax, 256), nodes), dim3(256), 0, s, n, depth, e, Q, dw,
+                       info_dev, (int)report, nsec);
+    hipLaunchKernelGGL(k_dc_zhat, dim3(nsec, nodes), dim3(256), 0, s, n, depth, e, Dout, dw);
     hipLaunchKernelGGL(k_dc_vec, dim3(cdiv(nmax, 4), nodes), dim3(256), 0, s, n, depth, W, dw);
-    hipLaunchKernelGGL(k_dc_gemm, dim3(cdiv(nmax, 64), cdiv(nmax, 64), nodes), dim3(256), 0, s, n, depth, Q, W,
-                       Zout, dw);
-    hipLaunchKernelGGL(k_dc_copydef, dim3(nmax, nodes), dim3(256), 0, s, n, depth, Q, Zout, dw);
+    const int nt = (int)cdiv(nmax, 64);
+    hipLaunchKernelGGL(k_dc_gemm, dim3(nt, nt + 1, nodes), dim3(256), 0, s, n, depth, Q, W, Zout, dw, nt);
     q ^= 1;
   }
   DC2_HIP(hipGetLastError());
