@@ -30,6 +30,33 @@ __host__ __device__ inline void cfma(cplx& a, cplx b, cplx c) {
   a.y = fma(b.x, c.y, fma(b.y, c.x, a.y));
 }
 
+// Sums over a wave (wave_add) and over each of its rows of 16 lanes (row_add), the same value in
+// every lane, all 64 lanes active.  By DPP moves and scalar reads of one lane per row: no trip
+// through LDS, which __shfl_xor takes six times (a sum's latency in the serial chains of the
+// tridiagonalisation and of Lanczos).
+template <int CTRL>
+__device__ inline double dpp_add(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+  return x + __hiloint2double(hi, lo);
+}
+__device__ inline double row_add(double x) {
+  x = dpp_add<0xB1>(x);           // quad_perm 1,0,3,2
+  x = dpp_add<0x4E>(x);           // quad_perm 2,3,0,1
+  x = dpp_add<0x141>(x);          // row_half_mirror
+  return dpp_add<0x140>(x);       // row_mirror
+}
+__device__ inline cplx row_add(cplx x) { return mk(row_add(x.x), row_add(x.y)); }
+__device__ inline double lane_value(double x, int l) {   // l uniform
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                          __builtin_amdgcn_readlane(__double2loint(x), l));
+}
+__device__ inline double wave_add(double x) {
+  x = row_add(x);
+  return (lane_value(x, 0) + lane_value(x, 16)) + (lane_value(x, 32) + lane_value(x, 48));
+}
+__device__ inline cplx wave_add(cplx x) { return mk(wave_add(x.x), wave_add(x.y)); }
+
 // XCD-aware tile order of a 2D grid of Mt x Nt output tiles (blockIdx.x over Mt, .y over Nt):
 // workgroups are dealt to the 8 XCDs in turn by their linear id, so the i-th workgroup an XCD
 // receives takes tile i of that XCD's contiguous share of the tiles in n-fastest order.  The

@@ -141,26 +141,12 @@ __device__ bool grid_sync(unsigned* bar, int k, int* err, double* part_dst, cons
   return ok != 0;
 }
 
-__device__ inline cplx wave_sum(cplx x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    x.x += __shfl_xor(x.x, o, 64);
-    x.y += __shfl_xor(x.y, o, 64);
-  }
-  return x;
-}
-__device__ inline double wave_sum(double x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-  return x;
-}
-
 // sum over the workgroup of one double per thread (same order in every workgroup), with one
 // workgroup barrier, which also publishes the LDS stores made before the call.  red must not
 // be read by another call between this one and the next workgroup barrier: the two sums of
 // a step use red slots of their own.
 __device__ double block_sum(double x, double* red) {
-  x = wave_sum(x);
+  x = wave_add(x);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) red[wave] = x;
   __syncthreads();
@@ -281,7 +267,7 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
           const int i = lane + 64 * s;
           if (i > k && i < n) cfma(acc, cconj(a[c][s]), sv[i]);
         }
-        acc = wave_sum(acc);
+        acc = wave_add(acc);
         const cplx pj = mk(t * acc.x, t * acc.y);
         if (lane == 0) st_coherent(P + j, pj);
         const cplx vj = sv[j];
@@ -391,20 +377,6 @@ __global__ void k_tri_prep(int n, const cplx* __restrict__ sub, double* __restri
   if (Z && t < (int64_t)n * n) Z[t] = (t % (n + 1) == 0) ? 1.0 : 0.0;
 }
 
-// sums over each row of 16 lanes, the same value in all 16 (DPP: no trip through LDS)
-template <int CTRL>
-__device__ inline double dpp_add(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
-  return x + __hiloint2double(hi, lo);
-}
-__device__ inline cplx row16_sum(cplx x) {
-  x = mk(dpp_add<0xB1>(x.x), dpp_add<0xB1>(x.y));     // quad_perm 1,0,3,2
-  x = mk(dpp_add<0x4E>(x.x), dpp_add<0x4E>(x.y));     // quad_perm 2,3,0,1
-  x = mk(dpp_add<0x141>(x.x), dpp_add<0x141>(x.y));   // row_half_mirror
-  return mk(dpp_add<0x140>(x.x), dpp_add<0x140>(x.y));   // row_mirror
-}
-
 // X[:, c] = H_0 H_1 ... H_{n-3} (delta .* Z[:, c]), n <= 16 S: 16 lanes per column (lane r holds
 // the rows r + 16 s), 16 columns per workgroup of four waves; the reflectors are staged through
 // LDS 64 KB at a time.  A serial chain of n - 2 dot products: with 16 lanes
@@ -445,7 +417,7 @@ __global__ __launch_bounds__(256) void k_hetrd_back(int n, const double* __restr
         cfma(dot, cconj(v[s]), x[s]);
         cfma(dot1, cconj(v[s + 1]), x[s + 1]);
       }
-      dot = row16_sum(mk(dot.x + dot1.x, dot.y + dot1.y));
+      dot = row_add(mk(dot.x + dot1.x, dot.y + dot1.y));
       const cplx f = mk(-t * dot.x, -t * dot.y);
 #pragma unroll
       for (int s = 0; s < S; ++s) cfma(x[s], v[s], f);

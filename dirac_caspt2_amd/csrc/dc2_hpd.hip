@@ -21,11 +21,8 @@ enum { CG_ACTIVE = 0, CG_DONE = 1, CG_BAD = 2 };
 
 // sums over the workgroup of two doubles, the same in every thread (fixed order)
 __device__ inline void cg_sum2(double& a, double& b, double* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    a += __shfl_xor(a, o, 64);
-    b += __shfl_xor(b, o, 64);
-  }
+  a = wave_add(a);
+  b = wave_add(b);
   __syncthreads();   // red may still be read from the sum before
   if ((threadIdx.x & 63) == 0) {
     red[2 * (threadIdx.x >> 6)] = a;
@@ -440,8 +437,7 @@ __global__ __launch_bounds__(LZ_T) void k_lanczos(int n, int j, const cplx* __re
                                                   cplx* __restrict__ vold, double* __restrict__ ab) {
   __shared__ double red[16];
   auto sum = [&](double x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    x = wave_add(x);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
     __syncthreads();
@@ -501,8 +497,7 @@ __global__ __launch_bounds__(1024) void k_lanczos_small(int n, int np, int j0, i
   __shared__ double red[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   auto sum = [&](double x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+    x = wave_add(x);
     __syncthreads();
     if (lane == 0) red[wave] = x;
     __syncthreads();
@@ -561,12 +556,7 @@ __global__ __launch_bounds__(1024) void k_lanczos_small(int n, int np, int j0, i
         for (int h = 0; h < 4; ++h) cfma(a[h], cconj(l[h]), ti);
       }
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          a[h].x += __shfl_xor(a[h].x, o, 64);
-          a[h].y += __shfl_xor(a[h].y, o, 64);
-        }
+      for (int h = 0; h < 4; ++h) a[h] = wave_add(a[h]);
       if (lane == 0)
 #pragma unroll
         for (int h = 0; h < 4; ++h)

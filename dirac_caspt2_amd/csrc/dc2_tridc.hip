@@ -53,13 +53,6 @@ __device__ inline double dc_hyp(double a, double b) {
   return m * sqrt(x * x + y * y);
 }
 
-// sum over the wave, the same value in every lane (lane 0's, so that every lane takes the
-// same branches)
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return __shfl(v, 0, 64);
-}
 __device__ inline double wave_prod(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v *= __shfl_xor(v, o, 64);
@@ -455,7 +448,7 @@ __global__ __launch_bounds__(256) void k_dc_secular(int n, int depth, const doub
     const double mid = 0.5 * (ld[jr + 1] - ld[jr]);
     double s = 0.0;
     for (int i = lane; i < K; i += 64) s += lz[i] * lz[i] / ((ld[i] - ld[jr]) - mid);
-    s = wave_sum(s);
+    s = wave_add(s);
     if (1.0 + rho * s >= 0.0) {
       o = jr;
       lo = 0.0;
@@ -470,7 +463,7 @@ __global__ __launch_bounds__(256) void k_dc_secular(int n, int depth, const doub
     for (int i = lane; i < K; i += 64) s += lz[i] * lz[i];
     o = jr;
     lo = 0.0;
-    hi = rho * wave_sum(s);
+    hi = rho * wave_add(s);
   }
   const double dorg = ld[o], zo2 = lz[o] * lz[o];
   double t = 0.5 * (lo + hi);
@@ -486,9 +479,9 @@ __global__ __launch_bounds__(256) void k_dc_secular(int n, int depth, const doub
       s2 += q * dl * r;
       sa += fabs(q);
     }
-    s1 = wave_sum(s1);
-    s2 = wave_sum(s2);
-    sa = wave_sum(sa);
+    s1 = wave_add(s1);
+    s2 = wave_add(s2);
+    sa = wave_add(sa);
     const double F = t * (1.0 + rho * s1) - rho * zo2;
     // converged once F is within the rounding error of its own evaluation (the stopping rule
     // of LAPACK's dlaed4): close to a pole, 1 + rho s1 can cancel to a few digits, and no
@@ -602,7 +595,7 @@ __global__ __launch_bounds__(256) void k_dc_vec(int n, int depth, double* __rest
     const double v = lzh[i] / ((ld[i] - dorg) - t);
     s += v * v;
   }
-  const double inv = 1.0 / sqrt(wave_sum(s));
+  const double inv = 1.0 / sqrt(wave_add(s));
   double* col = W + a + (int64_t)n * (a + jr);
   for (int i = lane; i < K; i += 64) col[i] = lzh[i] / ((ld[i] - dorg) - t) * inv;
 }
