@@ -77,101 +77,94 @@ struct DcWork {
 };
 
 // ------------------------------------------------------------------ leaves
-// One wave per leaf: lane r < N owns row r of the leaf's eigenvectors (LDS, column-major).
-// The scalar QL recurrence is executed by every lane on the shared d/e (identical values),
-// so that no lane waits for another.
+// One wave per leaf: lane r < N owns row r of the leaf's eigenvectors (LDS, column-major) and
+// holds d_r, e_r.  The scalar QL recurrence is executed by every lane on values read from one
+// lane, so that no lane waits for another; a rotation's columns are carried in a register and
+// loaded one ahead.  A serial chain of about 200 rotations (a square root and a division each):
+// with d and e in LDS every rotation also waited for its loads (n = 93: 87 -> 66 us).
 __global__ __launch_bounds__(64) void k_dc_leaf(int n, int depth, const double* __restrict__ din,
                                                 const double* __restrict__ e, double* __restrict__ Dout,
                                                 double* __restrict__ Zout, int* __restrict__ info) {
-  __shared__ double sd[DC_LEAF], se[DC_LEAF], Zl[DC_LEAF * DC_LEAF];
+  __shared__ double Zl[DC_LEAF * DC_LEAF];
   const int j = blockIdx.x, lane = threadIdx.x;
   const int a = node_lo(n, depth, j), c = node_lo(n, depth, j + 1), N = c - a;
   if (N <= 0) return;
-  if (lane < N) {
-    double d = din[a + lane];
+  const bool own = lane < N;
+  double d = 0.0, ev = 0.0;
+  if (own) {
+    d = din[a + lane];
     if (lane == 0 && a > 0) d -= fabs(e[a - 1]);        // tears at the leaf's two ends
     if (lane == N - 1 && c < n) d -= fabs(e[c - 1]);
-    sd[lane] = d;
-    se[lane] = lane < N - 1 ? e[a + lane] : 0.0;
+    ev = lane < N - 1 ? e[a + lane] : 0.0;
     for (int col = 0; col < N; ++col) Zl[col * DC_LEAF + lane] = col == lane ? 1.0 : 0.0;
   }
-  __syncthreads();
-  const bool own = lane < N;
   bool ok = true;
   double tst1 = 0.0;
   for (int l = 0; l < N && ok; ++l) {
-    int iter = 0, m;
-    tst1 = fmax(tst1, fabs(sd[l]) + fabs(se[l]));
-    do {
-      for (m = l; m + 1 < N; ++m)
-        if (fabs(se[m]) <= 2.0 * DC_EPS * tst1) break;
-      if (m != l) {
-        if (++iter > 90) {
-          ok = false;
+    int iter = 0;
+    tst1 = fmax(tst1, fabs(lane_value(d, l)) + fabs(lane_value(ev, l)));
+    while (true) {
+      const unsigned long long tiny = __ballot(lane >= l && lane + 1 < N && fabs(ev) <= 2.0 * DC_EPS * tst1);
+      const int m = __builtin_amdgcn_readfirstlane(tiny ? __ffsll(tiny) - 1 : N - 1);
+      if (m == l) break;
+      if (++iter > 90) {
+        ok = false;
+        break;
+      }
+      const double dl = lane_value(d, l), el = lane_value(ev, l);
+      double dn = lane_value(d, m);   // d of the rotation's second row
+      double g = (lane_value(d, l + 1) - dl) / (2.0 * el);
+      double r = dc_hyp(g, 1.0);
+      g = dn - dl + el / (g + (g >= 0.0 ? r : -r));
+      double s = 1.0, cc = 1.0, p = 0.0;
+      bool under = false;
+      double h = own ? Zl[m * DC_LEAF + lane] : 0.0, xn = own ? Zl[(m - 1) * DC_LEAF + lane] : 0.0;
+      int i = m - 1;
+      for (; i >= l; --i) {
+        const double ei = lane_value(ev, i), x = xn;
+        if (own && i > l) xn = Zl[(i - 1) * DC_LEAF + lane];
+        const double f = s * ei, b = cc * ei;
+        r = dc_hyp(f, g);
+        if (lane == i + 1) ev = r;
+        if (r == 0.0) {
+          if (lane == i + 1) d = dn - p;
+          under = true;
           break;
         }
-        double g = (sd[l + 1] - sd[l]) / (2.0 * se[l]);
-        double r = dc_hyp(g, 1.0);
-        g = sd[m] - sd[l] + se[l] / (g + (g >= 0.0 ? r : -r));
-        double s = 1.0, cc = 1.0, p = 0.0;
-        bool under = false;
-        for (int i = m - 1; i >= l; --i) {
-          const double f = s * se[i], b = cc * se[i];
-          r = dc_hyp(f, g);
-          se[i + 1] = r;
-          if (r == 0.0) {
-            sd[i + 1] -= p;
-            se[m] = 0.0;
-            under = true;
-            break;
-          }
-          s = f / r;
-          cc = g / r;
-          g = sd[i + 1] - p;
-          r = (sd[i] - g) * s + 2.0 * cc * b;
-          p = s * r;
-          sd[i + 1] = g + p;
-          g = cc * r - b;
-          if (own) {
-            const double h = Zl[(i + 1) * DC_LEAF + lane], x = Zl[i * DC_LEAF + lane];
-            Zl[(i + 1) * DC_LEAF + lane] = s * x + cc * h;
-            Zl[i * DC_LEAF + lane] = cc * x - s * h;
-          }
-        }
-        if (under) continue;
-        sd[l] -= p;
-        se[l] = g;
-        se[m] = 0.0;
+        s = f / r;
+        cc = g / r;
+        g = dn - p;
+        dn = lane_value(d, i);
+        r = (dn - g) * s + 2.0 * cc * b;
+        p = s * r;
+        if (lane == i + 1) d = g + p;
+        g = cc * r - b;
+        if (own) Zl[(i + 1) * DC_LEAF + lane] = s * x + cc * h;
+        h = cc * x - s * h;
       }
-    } while (m != l);
+      if (own) Zl[(i + 1) * DC_LEAF + lane] = h;   // the last column met: l, or where r vanished
+      if (lane == m) ev = 0.0;
+      if (under) continue;
+      if (lane == l) {
+        d -= p;
+        ev = g;
+      }
+    }
   }
   if (!ok) {
     if (lane == 0) info[0] = 1;
     return;
   }
-  // ascending order (selection sort, columns swapped with their eigenvalues)
-  for (int i = 0; i + 1 < N; ++i) {
-    int k = i;
-    double p = sd[i];
-    for (int q = i + 1; q < N; ++q)
-      if (sd[q] < p) {
-        k = q;
-        p = sd[q];
-      }
-    if (k != i) {
-      const double di = sd[i];
-      sd[k] = di;
-      sd[i] = p;
-      if (own) {
-        const double t = Zl[i * DC_LEAF + lane];
-        Zl[i * DC_LEAF + lane] = Zl[k * DC_LEAF + lane];
-        Zl[k * DC_LEAF + lane] = t;
-      }
-    }
+  // ascending order, ties by column
+  int rank = 0;
+  for (int q = 0; q < N; ++q) {
+    const double y = lane_value(d, q);
+    rank += y < d || (y == d && q < lane);
   }
-  if (own) {
-    Dout[a + lane] = sd[lane];
-    for (int col = 0; col < N; ++col) Zout[(a + lane) + (int64_t)n * (a + col)] = Zl[col * DC_LEAF + lane];
+  if (own) Dout[a + rank] = d;
+  for (int col = 0; col < N; ++col) {
+    const int to = __builtin_amdgcn_readlane(rank, col);
+    if (own) Zout[(a + lane) + (int64_t)n * (a + to)] = Zl[col * DC_LEAF + lane];
   }
 }
 
