@@ -1706,7 +1706,7 @@ void subspace_v(dc2_context* c, Lane& L, int k, double eshift, cplx*& V_out, dou
       case 'F':
         V_F(s, na, ns, d, blk("F"), c->tpairs.get(), c->spairs.get(), V, L.z("F_vscr", V_F_scratch(na, ns)));
         break;
-      case 'G': V_G(s, na, ni, ns, d, blk("G"), c->spairs.get(), V); break;
+      case 'G': V_G(s, na, ni, ns, d, blk("G"), V); break;
     }
     alphas(s, X, ni, na, ns, c->eps.get(), c->e0.get(), eshift, c->ipairs.get(), c->spairs.get(), npert, alpha);
   }

@@ -243,7 +243,7 @@ void V_E(hipStream_t s, int na, int ni, int ns, const Dens& d, const cplx* Eb, c
 int64_t V_F_scratch(int na, int ns);
 void V_F(hipStream_t s, int na, int ns, const Dens& d, const cplx* Fb, const int* tpairs, const int* spairs, cplx* V,
          cplx* scratch);
-void V_G(hipStream_t s, int na, int ni, int ns, const Dens& d, const cplx* Gb, const int* spairs, cplx* V);
+void V_G(hipStream_t s, int na, int ni, int ns, const Dens& d, const cplx* Gb, cplx* V);
 // alpha per perturber of subspace X (solve_X_subspace.F90 'alpha =' lines)
 void alphas(hipStream_t s, char X, int ni, int na, int ns, const double* eps, const double* e0_dev, double eshift,
             const int* ipairs, const int* spairs, int64_t npert, double* alpha);

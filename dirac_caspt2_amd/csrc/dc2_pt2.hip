@@ -338,17 +338,55 @@ __global__ void k_vf_gather(const cplx* __restrict__ C, int ns, const int* sp, i
   V[i] = C[k + ntp * ab];
 }
 
-// V_G(t; a>b, i) (solve_G_subspace.F90:445-462), Gb = (s,i|s,a)
-__global__ void k_V_G(int na, int ni, int ns, DV d, const cplx* Gb, const int* sp, int64_t nsp, cplx* V) {
-  const int t = threadIdx.x % 32 < na ? threadIdx.x % 32 : -1;
-  const int64_t pi = (int64_t)blockIdx.x * (blockDim.x / 32) + threadIdx.x / 32;  // pair*ni + i
-  if (t < 0 || pi >= nsp * ni) return;
+// V_G(t; a>b, i) (solve_G_subspace.F90:445-462), Gb = (s,i|s,a): sum_p D1(t,p) (G(a,i,b,p) -
+// G(b,i,a,p)) over 16 x 16 tiles of (a, b) with a in the tile at or above b's: the element with a
+// and b exchanged comes through LDS, so that both are read along a (a lane group per pair and i
+// read both 16 bytes at a time: 30 x 14 x 280 1.2 ms, of which its 0.79 GB are 0.18).  NT values
+// of t at a time (t0 on); 8 p in flight.  The pairs a > b are
+// ordered by a, then b.
+template <int NT>
+__global__ __launch_bounds__(256) void k_V_G(int na, int ni, int ns, int t0, DV d, const cplx* __restrict__ Gb,
+                                             cplx* __restrict__ V) {
+  constexpr int PC = 8;
+  __shared__ cplx y[PC][16][17];
+  // tile pair x = ta (ta + 1) / 2 + tb, tb <= ta
+  int ta = (int)((sqrt(8.0 * blockIdx.x + 1.0) - 1.0) * 0.5);
+  while (ta * (ta + 1) / 2 > (int)blockIdx.x) --ta;
+  while ((ta + 1) * (ta + 2) / 2 <= (int)blockIdx.x) ++ta;
+  const int tb = blockIdx.x - ta * (ta + 1) / 2, i = blockIdx.y;
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  const int a = 16 * ta + tx, b = 16 * tb + ty;        // this thread's pair
+  const int ra = 16 * tb + tx, rb = 16 * ta + ty;      // the exchanged element it reads for another
   const int64_t S = ns, Ni = ni;
-  const int m = (int)(pi / ni), i = (int)(pi % ni), a = sp[2 * m], b = sp[2 * m + 1];
-  auto Gv = [&](int aa, int ii, int bb, int p) { return Gb[aa + S * (ii + Ni * (bb + S * p))]; };
-  cplx acc = mk(0.0, 0.0);
-  for (int p = 0; p < na; ++p) cfma(acc, d.D1(t, p), csub(Gv(a, i, b, p), Gv(b, i, a, p)));
-  V[t + (int64_t)na * pi] = acc;
+  cplx acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = mk(0.0, 0.0);
+  for (int p0 = 0; p0 < na; p0 += PC) {
+    cplx x[PC];
+#pragma unroll
+    for (int u = 0; u < PC; ++u) {
+      const int p = p0 + u;
+      x[u] = p < na && a < ns && b < ns ? Gb[a + S * (i + Ni * (b + S * p))] : mk(0.0, 0.0);
+      y[u][ty][tx] = p < na && ra < ns && rb < ns ? Gb[ra + S * (i + Ni * (rb + S * p))] : mk(0.0, 0.0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PC; ++u) {
+      const int p = p0 + u;
+      if (p >= na) break;
+      const cplx g = csub(x[u], y[u][tx][ty]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (t0 + t < na) cfma(acc[t], d.D1(t0 + t, p), g);
+    }
+    __syncthreads();
+  }
+  if (!(a > b && a < ns)) return;
+  const int64_t m = (int64_t)a * (a - 1) / 2 + b;
+  cplx* v = V + (int64_t)na * (m * ni + i) + t0;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    if (t0 + t < na) v[t] = acc[t];
 }
 
 __global__ void k_alphas(char X, int ni, int na, int ns, const double* eps, const double* e0p, double eshift,
@@ -643,12 +681,15 @@ void V_F(hipStream_t s, int na, int ns, const Dens& d, const cplx* Fb, const int
   hipLaunchKernelGGL(k_vf_gather, dim3(cdiv(ntp * nsp, 256)), dim3(256), 0, s, C, ns, spairs, ntp, nsp, V);
   DC2_HIP(hipGetLastError());
 }
-void V_G(hipStream_t s, int na, int ni, int ns, const Dens& d, const cplx* Gb, const int* spairs, cplx* V) {
-  const int64_t nsp = (int64_t)ns * (ns - 1) / 2;
-  if (nsp == 0 || ni == 0) return;
+void V_G(hipStream_t s, int na, int ni, int ns, const Dens& d, const cplx* Gb, cplx* V) {
+  if (ns < 2 || ni == 0) return;
+  DC2_CHECK(ni < 65536, 1, "V_G: ninact < 65536");
   DC2_CHECK(na <= 32, 1, "V_G: nact <= 32");
-  const int64_t items = nsp * ni;   // 8 items of 32 lanes per 256-thread block
-  hipLaunchKernelGGL(k_V_G, dim3(cdiv(items, 8)), dim3(256), 0, s, na, ni, ns, dv(d), Gb, spairs, nsp, V);
+  const unsigned T = cdiv(ns, 16);
+  for (int t0 = 0; t0 < na; t0 += 16) {
+    auto k = na - t0 <= 8 ? k_V_G<8> : k_V_G<16>;
+    hipLaunchKernelGGL(k, dim3(T * (T + 1) / 2, ni), dim3(256), 0, s, na, ni, ns, t0, dv(d), Gb, V);
+  }
   DC2_HIP(hipGetLastError());
 }
 void alphas(hipStream_t s, char X, int ni, int na, int ns, const double* eps, const double* e0_dev, double eshift,
