@@ -341,7 +341,7 @@ __global__ void k_vf_gather(const cplx* __restrict__ C, int ns, const int* sp, i
 // V_G(t; a>b, i) (solve_G_subspace.F90:445-462), Gb = (s,i|s,a): sum_p D1(t,p) (G(a,i,b,p) -
 // G(b,i,a,p)) over 16 x 16 tiles of (a, b) with a in the tile at or above b's: the element with a
 // and b exchanged comes through LDS, so that both are read along a (a lane group per pair and i
-// read both 16 bytes at a time: 30 x 14 x 280 1.2 ms, of which its 0.79 GB are 0.18).  NT values
+// read both 16 bytes at a time: 30 x 14 x 280 1.17 ms and 3.4 GB of traffic; now 0.40 ms, 0.8 GB).  NT values
 // of t at a time (t0 on); 8 p in flight.  The pairs a > b are
 // ordered by a, then b.
 template <int NT>
