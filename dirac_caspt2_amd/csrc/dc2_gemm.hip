@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm(int64_t M, int64_t N, int64_t 
   xcd_tile(gridDim.x, gridDim.y, blockIdx.x, blockIdx.y, mt, nt);
   // An XCD gets consecutive row blocks, whose work grows or shrinks along a triangle: the first
   // with the last, the second with the last but one ... evens it out (upper tiles of m = 1274, k
-  // = 3432: FIG1 us, 686 with the rows in order, 33 TF/s)
+  // = 3432: 479 us, 686 with the rows in order)
   if (UPPER || tri != TRI_NONE) mt = (mt & 1) ? gridDim.x - 1 - mt / 2 : mt / 2;
   if (UPPER && mt * TM > nt * TN + TN - 1) return;   // uniform
   __shared__ cplx As[2 * KB * T::LA], Bs[2 * KB * T::LB];
