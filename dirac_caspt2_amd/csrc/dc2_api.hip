@@ -514,8 +514,7 @@ void upload_ints(hipStream_t s, DevBuf<int>& dst, const std::vector<int>& v) {
 // matrix V^H H V is kept on the host and extended by the new block only (after a restart it
 // is diag(theta)); its eigenproblem runs on the host (herm_eig), the orthonormalisation of a
 // block of four on the device (a second round trip to the host for larger blocks), so that
-// an iteration has one host round trip.  A block of four (one root) takes the fused step of
-// davidson4_ritz and davidson4_block.  Writes c->civec (n x nroot) and
+// an iteration has one host round trip.  Writes c->civec (n x nroot) and
 // c->ecas; returns false (no result) when it does not converge, and the caller falls back to
 // the dense eigensolver.
 bool davidson(dc2_context* c, int64_t n, const cplx* H, int nroot) {
@@ -588,28 +587,11 @@ bool davidson(dc2_context* c, int64_t n, const cplx* H, int nroot) {
   // the block orthonormalisation on the device for blocks of four (one root), so that an
   // iteration needs one host round trip; the host's, in a round trip of its own, otherwise
   const bool dev_orth = b == 4;
-  // The whole step of a block of four in nine launches and one download instead of fourteen
-  // launches and two copies: the chain of short launches bounds it, not the 14 MB of H (924
-  // determinants: the whole 192-spinor energy 11.9 -> 10.8 ms, 554: 17.6 -> 16.6 ms).  Past davidson4_max() vectors, a
-  // subspace that only the option asks for, the coefficients leave one workgroup's LDS.
-  const bool four = dev_orth && maxsub <= davidson4_max();
-  double* pn = L.d("dv_pn", davidson4_partials(n));
-  cplx* C2 = L.z("dv_c2", 4 * (int64_t)(maxsub + 4));
-  cplx* Cf = L.z("dv_cf", 4 * (int64_t)(maxsub + 4));
   // the first block's Rayleigh columns
   zgemm(s, 'C', 'N', m, nk, n, one, V, n, 0, W, n, 0, zero, Cn, ldc, 0, 1);
   to_host(Ch, Cn, (size_t)ldc * nk * sizeof(cplx));
-  auto keep = [&](int roots) {
-    c->civec.ensure(n * roots);
-    DC2_HIP(hipMemcpyAsync(c->civec.get(), X, n * roots * sizeof(cplx), hipMemcpyDeviceToDevice, s));
-    DC2_HIP(hipStreamSynchronize(s));
-    c->ecas.assign(theta.begin(), theta.begin() + roots);
-    c->nroots_avail = roots;
-    return true;
-  };
-  bool done = false;   // converged, the newest block still unused
-  for (int it = 1; it <= 200 || done; ++it) {
-    if (!done) c->davidson_iters = it;
+  for (int it = 1; it <= 200; ++it) {
+    c->davidson_iters = it;
     // Rayleigh matrix: the new columns V^H W[:, m-nk:m], downloaded with ldc rows
     for (int j = 0; j < nk; ++j)
       for (int i = 0; i < m; ++i) {
@@ -632,38 +614,13 @@ bool davidson(dc2_context* c, int64_t n, const cplx* H, int nroot) {
     herm_eig_low(m, Tm.data(), theta.data(), Yh.data(), b);   // every theta, the lowest b vectors
     std::copy(Yh.begin(), Yh.begin() + (size_t)m * b, up_y);     // first b Ritz vectors
     std::memcpy(up_y + (size_t)maxsub * b, theta.data(), b * sizeof(double));
-    if (done) {
-      to_dev(Sy, up_y, (size_t)m * nroot * sizeof(cplx));
-      zgemm(s, 'N', 'N', n, nroot, m, one, V, n, 0, Sy, m, 0, zero, X, n, 0, 1);
-      return keep(nroot);
-    }
-    if (!four) to_dev(Sy, up_y, (size_t)maxsub * b * sizeof(cplx) + b * sizeof(double));   // Sy, then theta
+    to_dev(Sy, up_y, (size_t)maxsub * b * sizeof(cplx) + b * sizeof(double));   // Sy, then theta
     const bool restart = m + b > maxsub;
     const int m_in = m;
     // Ritz vectors and residuals, preconditioned corrections (one launch up to 64 subspace
     // vectors), (restart,) two classical Gram-Schmidt passes against V, the Gram matrix of the
     // block and (device_orth) its orthonormal combinations: launches only
-    auto segment4 = [&](int mm, bool rs) {
-      const cplx* yh = reinterpret_cast<const cplx*>(up_y);
-      cplx* Tv = rs ? T : V + n * mm;   // a restart still reads the columns it will write
-      davidson4_ritz(s, n, mm, V, W, yh, reinterpret_cast<const double*>(yh + (size_t)maxsub * b), d, X, AX, Tv, pn);
-      if (rs) {
-        DC2_HIP(hipMemcpyAsync(V, X, n * b * sizeof(cplx), hipMemcpyDeviceToDevice, s));
-        DC2_HIP(hipMemcpyAsync(W, AX, n * b * sizeof(cplx), hipMemcpyDeviceToDevice, s));
-        mm = b;
-        Tv = V + n * mm;
-        DC2_HIP(hipMemcpyAsync(Tv, T, n * b * sizeof(cplx), hipMemcpyDeviceToDevice, s));
-      }
-      zgemm(s, 'C', 'N', mm, b, n, one, V, n, 0, Tv, n, 0, zero, Sm, mm, 0, 1);
-      zgemm(s, 'N', 'N', n, b, mm, mone, V, n, 0, Sm, mm, 0, one, Tv, n, 0, 1);
-      zgemm(s, 'C', 'N', mm + b, b, n, one, V, n, 0, Tv, n, 0, zero, C2, mm + b, 0, 1);
-      davidson4_block(s, n, mm, C2, pn, Cf, RG, nk_dev, V);
-    };
     auto segment = [&](int mm, bool rs) {
-      if (four) {
-        segment4(mm, rs);
-        return;
-      }
       if (mm <= 64) {   // sel is the identity
         davidson_ritz(s, n, b, mm, V, W, Sy, th, d, X, AX, R, T);
       } else {
@@ -693,8 +650,7 @@ bool davidson(dc2_context* c, int64_t n, const cplx* H, int nroot) {
     if (graph_ok) {
       const std::vector<int64_t> key = {n, b, m_in, (int64_t)V, (int64_t)W, (int64_t)X, (int64_t)AX, (int64_t)R,
                                         (int64_t)T, (int64_t)Sy, (int64_t)th, (int64_t)RG, (int64_t)Sm, (int64_t)d,
-                                        (int64_t)sel, (int64_t)s, (int64_t)Sc, (int64_t)nk_dev, (int64_t)dev_orth, (int64_t)four,
-                                        (int64_t)up_y, (int64_t)pn, (int64_t)C2, (int64_t)Cf, (int64_t)maxsub};
+                                        (int64_t)sel, (int64_t)s, (int64_t)Sc, (int64_t)nk_dev, (int64_t)dev_orth};
       auto it = c->dav_graphs.find(key);
       if (it == c->dav_graphs.end()) {   // capture; on any failure the context stops using graphs
         hipGraph_t g = nullptr;
@@ -750,23 +706,25 @@ bool davidson(dc2_context* c, int64_t n, const cplx* H, int nroot) {
     }
     // the next block (b columns, the dropped ones zero) and its Rayleigh columns, then one
     // download of the residual norms, the kept count and V^H W_new; m + b <= maxsub here
-    if (!four) zgemm(s, 'N', 'N', n, b, b, one, T, n, 0, Sc, b, 0, zero, V + n * m, n, 0, 1);
+    zgemm(s, 'N', 'N', n, b, b, one, T, n, 0, Sc, b, 0, zero, V + n * m, n, 0, 1);
     zgemm(s, 'N', 'N', n, b, n, one, H, n, 0, V + n * m, n, 0, zero, W + n * m, n, 0, 1);
     zgemm(s, 'C', 'N', m + b, b, n, one, V, n, 0, W + n * m, n, 0, zero, Cn, m + b, 0, 1);
     to_host(rg, DL, (nrg + 1 + (size_t)(m + b) * b) * sizeof(cplx));
     double worst = 0.0;
     for (int j = 0; j < nroot; ++j) worst = std::max(worst, std::sqrt(std::fabs(rg[j + (size_t)b * j].real())));
-    nk = dev_orth ? *nk_host : kept_host;
-    // The block of this step and its products are there: the vectors from the subspace with it
-    // (30 us) are 2 to 9 times nearer the converged ones than X (554, 924, 3003 determinants)
     if (worst < tol) {
-      done = four && nk > 0;
-      if (!done) return keep(nroot);
+      c->civec.ensure(n * nroot);
+      DC2_HIP(hipMemcpyAsync(c->civec.get(), X, n * nroot * sizeof(cplx), hipMemcpyDeviceToDevice, s));
+      DC2_HIP(hipStreamSynchronize(s));
+      c->ecas.assign(theta.begin(), theta.begin() + nroot);
+      c->nroots_avail = nroot;
+      return true;
     }
     if (restart) {
       for (int j = 0; j < b; ++j)
         for (int i = 0; i < b; ++i) Th[i + (size_t)maxsub * j] = (i == j) ? zc(theta[j], 0.0) : zc(0.0, 0.0);
     }
+    nk = dev_orth ? *nk_host : kept_host;
     if (nk <= 0) return false;
     ldc = m + b;
     m += nk;

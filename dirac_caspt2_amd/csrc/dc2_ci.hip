@@ -817,68 +817,6 @@ __global__ __launch_bounds__(256) void k_ritz_fused(int64_t n, int mm, const cpl
   T[i + n * j] = cscale(r, 1.0 / den);
 }
 
-// The same for a block of four whose corrections go to the columns after V (T = V + n mm), with
-// the Ritz coefficients read from page-locked host memory into LDS (no upload launch) and the
-// squared norms of the residuals and corrections summed per workgroup: pn[8 blk + 2 j + {0, 1}].
-// Latency bound like the whole step (3 MB at 924 determinants and 24 vectors): what counts is
-// that it takes the place of two uploads, two normalisations and a Gram product
-__global__ __launch_bounds__(256) void k_ritz4(int64_t n, int mm, cplx* V, const cplx* __restrict__ W,
-                                               const cplx* __restrict__ Yh, const double* __restrict__ thh,
-                                               const double* __restrict__ d, cplx* __restrict__ X,
-                                               cplx* __restrict__ AX, cplx* T, double* __restrict__ pn) {
-  __shared__ cplx y[64];
-  __shared__ double red[8];
-  __shared__ double th_s;
-  const int j = blockIdx.y, tid = threadIdx.x;
-  if (tid < mm) y[tid] = Yh[(int64_t)mm * j + tid];
-  if (tid == 64) th_s = thh[j];
-  __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * 256 + tid;
-  double nr = 0.0, nt = 0.0;
-  if (i < n) {
-    cplx x = mk(0.0, 0.0), ax = mk(0.0, 0.0);
-    int k = 0;
-    for (; k + 4 <= mm; k += 4) {   // eight loads in flight
-      cplx v[4], w[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        v[u] = V[i + n * (k + u)];
-        w[u] = W[i + n * (k + u)];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        cfma(x, v[u], y[k + u]);
-        cfma(ax, w[u], y[k + u]);
-      }
-    }
-    for (; k < mm; ++k) {
-      cfma(x, V[i + n * k], y[k]);
-      cfma(ax, W[i + n * k], y[k]);
-    }
-    const double th = th_s;
-    const cplx r = csub(ax, cscale(x, th));
-    double den = th - d[i];
-    if (fabs(den) < 1e-8) den = den < 0 ? -1e-8 : 1e-8;
-    const cplx t = cscale(r, 1.0 / den);
-    X[i + n * j] = x;
-    AX[i + n * j] = ax;
-    T[i + n * j] = t;
-    nr = cabs2(r);
-    nt = cabs2(t);
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    nr += __shfl_xor(nr, o, 64);
-    nt += __shfl_xor(nt, o, 64);
-  }
-  if ((tid & 63) == 0) {
-    red[2 * (tid >> 6)] = nr;
-    red[2 * (tid >> 6) + 1] = nt;
-  }
-  __syncthreads();
-  if (tid < 2) pn[8 * (int64_t)blockIdx.x + 2 * j + tid] = red[tid] + red[2 + tid] + red[4 + tid] + red[6 + tid];
-}
-
 // one workgroup per column: T[:, c] /= |T[:, c]| (deterministic tree reduction)
 __global__ __launch_bounds__(256) void k_col_normalize(int64_t n, cplx* T) {
   __shared__ double sh[256];
@@ -1146,11 +1084,10 @@ void davidson_ritz(hipStream_t s, int64_t n, int ncol, int mm, const cplx* V, co
 // Sc = R^-1 on the kept columns, written first, zero columns after them, and the kept count in
 // nk[0].  One thread, every index static.  This is the block orthonormalisation the host did
 // between two round trips, so that an iteration needs one host round trip instead of two.
-// Sc (4 x 4): orthonormal combinations (kept columns first, then zeros) of four columns from
-// their Gram matrix G (column-major, upper triangle read), a column dropped when what is left of
-// it is at most 1e-12 tn[k] (squared norms); returns the kept count
-__device__ int chol4(const cplx* G, const double* tn, cplx* Sc) {
+__global__ __launch_bounds__(64) void k_block_chol4(const cplx* __restrict__ G, cplx* __restrict__ Sc,
+                                                    int* __restrict__ nk) {
   constexpr int B = 4;
+  if (threadIdx.x != 0) return;
   cplx A[B][B], R[B][B];
   bool keep[B];
 #pragma unroll
@@ -1175,7 +1112,7 @@ __device__ int chol4(const cplx* G, const double* tn, cplx* Sc) {
       R[j][k] = x;
       d -= cabs2(x);
     }
-    keep[k] = d > 1e-12 * tn[k];
+    keep[k] = d > 1e-12;
     R[k][k] = mk(keep[k] ? sqrt(d) : 1.0, 0.0);
   }
   // X = R^-1 (upper triangular on the kept indices): X[k][k] = 1/R[k][k],
@@ -1212,100 +1149,7 @@ __device__ int chol4(const cplx* G, const double* tn, cplx* Sc) {
   for (int k = kept; k < B; ++k)
 #pragma unroll
     for (int i = 0; i < B; ++i) Sc[i + B * k] = mk(0.0, 0.0);
-  return kept;
-}
-
-__global__ __launch_bounds__(64) void k_block_chol4(const cplx* __restrict__ G, cplx* __restrict__ Sc,
-                                                    int* __restrict__ nk) {
-  if (threadIdx.x != 0) return;
-  const double one[4] = {1.0, 1.0, 1.0, 1.0};
-  nk[0] = chol4(G, one, Sc);
-}
-
-// After one Gram-Schmidt pass: C2 = [V T']^H T' ((mm + 4) x 4).  The second pass and the
-// orthonormalisation in one set of coefficients Cf: T'' = T' - V C2[0:mm] has the Gram matrix
-// T'^H T' - C2^H C2, and its orthonormal combinations T'' Sc are [V T'] [-C2 Sc; Sc].  tn: the
-// squared norms of the columns before any projection, summed from pn with those of the
-// residuals, which go to the diagonal of RG.
-constexpr int DAV_MM = 60;
-__global__ __launch_bounds__(64) void k_block_coef(int mm, int nblk, const cplx* __restrict__ C2,
-                                                   const double* __restrict__ pn, cplx* __restrict__ Cf,
-                                                   cplx* __restrict__ RG, int* __restrict__ nk) {
-  __shared__ cplx c2[DAV_MM + 4][4], G[16], Sc[16];
-  __shared__ double tn[4];
-  const int l = threadIdx.x, ld = mm + 4;
-  for (int e = l; e < 4 * ld; e += 64) c2[e % ld][e / ld] = C2[e];
-  if (l < 8) {
-    double x = 0.0;
-    for (int b = 0; b < nblk; ++b) x += pn[8 * (int64_t)b + l];
-    if (l & 1) tn[l >> 1] = x;
-    else RG[5 * (l >> 1)] = mk(x, 0.0);
-  }
-  __syncthreads();
-  const int a = (l >> 2) & 3, b = l >> 4, q = l & 3;   // G[a + 4 b], a quarter of the sum each
-  cplx g = mk(0.0, 0.0);
-  for (int k = q; k < mm; k += 4) cfma(g, cconj(c2[k][a]), c2[k][b]);
-#pragma unroll
-  for (int o = 1; o < 4; o <<= 1) {
-    g.x += __shfl_xor(g.x, o, 64);
-    g.y += __shfl_xor(g.y, o, 64);
-  }
-  if (q == 0) G[a + 4 * b] = csub(c2[mm + a][b], g);
-  __syncthreads();
-  if (l == 0) nk[0] = chol4(G, tn, Sc);
-  __syncthreads();
-  for (int e = l; e < 4 * ld; e += 64) {
-    const int k = e % ld, c = e / ld;
-    cplx x = mk(0.0, 0.0);
-    if (k >= mm) {
-      x = Sc[(k - mm) + 4 * c];
-    } else {
-      for (int u = 0; u < 4; ++u) cfma(x, c2[k][u], Sc[u + 4 * c]);
-      x = mk(-x.x, -x.y);
-    }
-    Cf[e] = x;
-  }
-}
-
-// the columns mm .. mm + 3 of V <- [V T'] Cf, T' in their place; thread = row
-__global__ __launch_bounds__(64) void k_new_block(int64_t n, int mm, const cplx* __restrict__ Cf, cplx* V) {
-  __shared__ cplx cf[DAV_MM + 4][4];
-  const int ld = mm + 4;
-  for (int e = threadIdx.x; e < 4 * ld; e += 64) cf[e % ld][e / ld] = Cf[e];
-  __syncthreads();
-  const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (i >= n) return;
-  cplx x[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) x[c] = mk(0.0, 0.0);
-  for (int k = 0; k < ld; k += 4) {
-    cplx v[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = k + u < ld ? V[i + n * (k + u)] : mk(0.0, 0.0);
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (k + u < ld)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) cfma(x[c], v[u], cf[k + u][c]);
-  }
-#pragma unroll
-  for (int c = 0; c < 4; ++c) V[i + n * (mm + c)] = x[c];
-}
-
-int davidson4_max() { return DAV_MM; }
-int64_t davidson4_partials(int64_t n) { return 8 * (int64_t)cdiv(n, 256); }
-
-void davidson4_ritz(hipStream_t s, int64_t n, int mm, cplx* V, const cplx* W, const cplx* Y_host,
-                    const double* theta_host, const double* d, cplx* X, cplx* AX, cplx* T, double* pn) {
-  hipLaunchKernelGGL(k_ritz4, dim3(cdiv(n, 256), 4), dim3(256), 0, s, n, mm, V, W, Y_host, theta_host, d, X, AX, T, pn);
-  DC2_HIP(hipGetLastError());
-}
-
-void davidson4_block(hipStream_t s, int64_t n, int mm, const cplx* C2, const double* pn, cplx* Cf, cplx* RG, int* nk,
-                     cplx* V) {
-  hipLaunchKernelGGL(k_block_coef, dim3(1), dim3(64), 0, s, mm, (int)cdiv(n, 256), C2, pn, Cf, RG, nk);
-  hipLaunchKernelGGL(k_new_block, dim3(cdiv(n, 64)), dim3(64), 0, s, n, mm, Cf, V);
-  DC2_HIP(hipGetLastError());
+  nk[0] = kept;
 }
 
 void davidson_block_orth(hipStream_t s, const cplx* G, cplx* Sc, int* nk) {

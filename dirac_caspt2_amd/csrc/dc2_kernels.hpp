@@ -99,20 +99,6 @@ void davidson_normalize(hipStream_t s, int64_t n, int ncol, cplx* T);
 // R = AX - X diag(theta), T[:, c] = R[:, c] / (theta_c - d) (Y = Sy, mm x ncol)
 void davidson_ritz(hipStream_t s, int64_t n, int ncol, int mm, const cplx* V, const cplx* W, const cplx* Sy,
                    const double* theta, const double* d, cplx* X, cplx* AX, cplx* R, cplx* T);
-// The iteration of a block of four (one root) with fewer launches, mm <= davidson4_max():
-// davidson4_ritz: X, AX, R and T as above with the Ritz coefficients (mm x 4) and theta read from
-// page-locked host memory, T to T, the residuals' and corrections' squared norms to pn
-// (davidson4_partials(n) doubles); davidson4_block: the columns mm .. mm + 3 of V, which hold the
-// corrections T' after one Gram-Schmidt pass, replaced by the next block, from C2 = [V T']^H T'
-// ((mm + 4) x 4): second pass and orthonormalisation at once (dropped columns zero, last); Cf
-// scratch of 4 (mm + 4); the residuals' squared norms to the diagonal of RG (4 x 4), the kept
-// count to nk
-int davidson4_max();
-int64_t davidson4_partials(int64_t n);
-void davidson4_ritz(hipStream_t s, int64_t n, int mm, cplx* V, const cplx* W, const cplx* Y_host,
-                    const double* theta_host, const double* d, cplx* X, cplx* AX, cplx* T, double* pn);
-void davidson4_block(hipStream_t s, int64_t n, int mm, const cplx* C2, const double* pn, cplx* Cf, cplx* RG, int* nk,
-                     cplx* V);
 // orthonormal combinations Sc (4 x 4, kept columns first, then zeros) of a correction block of
 // four columns from its Gram matrix G (4 x 4); the kept count in nk[0]
 void davidson_block_orth(hipStream_t s, const cplx* G, cplx* Sc, int* nk);
