@@ -506,9 +506,11 @@ __global__ __launch_bounds__(1024) void k_lanczos_small(int n, int np, int j0, i
     for (int q = 0; q < 16; ++q) s += red[q];
     return s;
   };
-  if (tid < n) {
-    v[tid] = vg[tid];
-    vold[tid] = j0 > 0 ? voldg[tid] : mk(0.0, 0.0);
+  // all LZS_N entries: the rounds of eight below multiply the ones past n by zeros of L^-1, which
+  // what an earlier workgroup left in LDS (a NaN) would survive
+  if (tid < LZS_N) {
+    v[tid] = tid < n ? vg[tid] : mk(0.0, 0.0);
+    vold[tid] = tid < n && j0 > 0 ? voldg[tid] : mk(0.0, 0.0);
   }
   double bo = j0 > 0 ? ab[2 * (j0 - 1) + 1] : 0.0;
   __syncthreads();
