@@ -2581,8 +2581,12 @@ int dc2_whiten(dc2_context* c, int32_t n, const double* S, const double* b, doub
     const cplx* Li = L.z("W_hLi", np * np);
     double lam = 0.0;
     if (!chol_lambda_min(c->stream, n, Li, L.z("lanczos", 4 * (int64_t)n + 256),
-                         reinterpret_cast<double*>(L.host(512 * sizeof(double), 1)), lam))
-      return;
+                         reinterpret_cast<double*>(L.host(512 * sizeof(double), 1)), lam)) {
+      // many eigenvalues close to the smallest one: Lanczos did not separate it in its steps
+      double* w = L.d("W_w", n);
+      zheevd(c, n, Sd.get(), w, "a metric");
+      L.download(&lam, w, sizeof(double));
+    }
     DC2_HIP(hipMemcpy2DAsync(linv, n * sizeof(cplx), Li, np * sizeof(cplx), n * sizeof(cplx), n, hipMemcpyDeviceToHost,
                              c->stream));
     copy_sync(c, btilde, L.z("W_bc1", nn), nn * sizeof(cplx), hipMemcpyDeviceToHost);
