@@ -981,7 +981,9 @@ bool chol_whiten(dc2_context* c, Lane& L, char X, int64_t n, const cplx* S, cons
   if (c->debug)
     std::fprintf(stderr, "dc2: Cholesky of the %c metric (n=%lld): %s\n", X, (long long)n,
                  hf[0] || hf[1] ? "eigenvalues below the threshold" : "whole rank");
-  return hf[0] == 0 && hf[1] == 0;
+  if (hf[0] || hf[1]) return false;
+  check_finite(c, s, "B~", bc1, n * n);
+  return true;
 }
 
 // with the automatic eigensolver choice, where the resolvents take E2 from B~ (cg_route); not
