@@ -124,7 +124,7 @@ struct Lane {
     for (void* h : pinned)
       if (h) (void)hipHostFree(h);
     if (owned) {
-      if (blas) rocblas_destroy_handle(blas);
+      drop_blas_handle(blas);
       if (stream) {
         release_stream_workspace(stream);
         (void)hipStreamDestroy(stream);
@@ -204,6 +204,7 @@ struct dc2_context {
   // rocSOLVER dstedc
   bool tri_own = true;
   std::map<std::vector<int64_t>, hipGraphExec_t> dav_graphs;
+  hipStream_t capture_stream = nullptr;   // captures happen here, so that a broken one does not stop `stream`
   int64_t graph_launches = 0, graph_captures = 0;
 
   // called from the lane that finished subspace k (0 = A .. 7 = H) with its e2 and sumc2
@@ -620,28 +621,28 @@ bool davidson(dc2_context* c, int64_t n, const cplx* H, int nroot) {
     // Ritz vectors and residuals, preconditioned corrections (one launch up to 64 subspace
     // vectors), (restart,) two classical Gram-Schmidt passes against V, the Gram matrix of the
     // block and (device_orth) its orthonormal combinations: launches only
-    auto segment = [&](int mm, bool rs) {
+    auto segment = [&](hipStream_t q, int mm, bool rs) {
       if (mm <= 64) {   // sel is the identity
-        davidson_ritz(s, n, b, mm, V, W, Sy, th, d, X, AX, R, T);
+        davidson_ritz(q, n, b, mm, V, W, Sy, th, d, X, AX, R, T);
       } else {
-        zgemm(s, 'N', 'N', n, b, mm, one, V, n, 0, Sy, mm, 0, zero, X, n, 0, 1);
-        zgemm(s, 'N', 'N', n, b, mm, one, W, n, 0, Sy, mm, 0, zero, AX, n, 0, 1);
-        davidson_residual(s, n, b, AX, X, th, R);
-        davidson_precond(s, n, b, sel, R, th, d, T);
+        zgemm(q, 'N', 'N', n, b, mm, one, V, n, 0, Sy, mm, 0, zero, X, n, 0, 1);
+        zgemm(q, 'N', 'N', n, b, mm, one, W, n, 0, Sy, mm, 0, zero, AX, n, 0, 1);
+        davidson_residual(q, n, b, AX, X, th, R);
+        davidson_precond(q, n, b, sel, R, th, d, T);
       }
-      zgemm(s, 'C', 'N', b, b, n, one, R, n, 0, R, n, 0, zero, RG, b, 0, 1);   // residual norms
-      davidson_normalize(s, n, b, T);
+      zgemm(q, 'C', 'N', b, b, n, one, R, n, 0, R, n, 0, zero, RG, b, 0, 1);   // residual norms
+      davidson_normalize(q, n, b, T);
       if (rs) {   // thick restart on the b Ritz vectors: V^H H V = diag(theta)
-        DC2_HIP(hipMemcpyAsync(V, X, n * b * sizeof(cplx), hipMemcpyDeviceToDevice, s));
-        DC2_HIP(hipMemcpyAsync(W, AX, n * b * sizeof(cplx), hipMemcpyDeviceToDevice, s));
+        DC2_HIP(hipMemcpyAsync(V, X, n * b * sizeof(cplx), hipMemcpyDeviceToDevice, q));
+        DC2_HIP(hipMemcpyAsync(W, AX, n * b * sizeof(cplx), hipMemcpyDeviceToDevice, q));
         mm = b;
       }
       for (int pass = 0; pass < 2; ++pass) {
-        zgemm(s, 'C', 'N', mm, b, n, one, V, n, 0, T, n, 0, zero, Sm, mm, 0, 1);
-        zgemm(s, 'N', 'N', n, b, mm, mone, V, n, 0, Sm, mm, 0, one, T, n, 0, 1);
+        zgemm(q, 'C', 'N', mm, b, n, one, V, n, 0, T, n, 0, zero, Sm, mm, 0, 1);
+        zgemm(q, 'N', 'N', n, b, mm, mone, V, n, 0, Sm, mm, 0, one, T, n, 0, 1);
       }
-      zgemm(s, 'C', 'N', b, b, n, one, T, n, 0, T, n, 0, zero, RG + (size_t)b * b, b, 0, 1);
-      if (dev_orth) davidson_block_orth(s, RG + (size_t)b * b, Sc, nk_dev);
+      zgemm(q, 'C', 'N', b, b, n, one, T, n, 0, T, n, 0, zero, RG + (size_t)b * b, b, 0, 1);
+      if (dev_orth) davidson_block_orth(q, RG + (size_t)b * b, Sc, nk_dev);
     };
     // Replayed from a captured graph when no restart copy is involved and the launches are
     // not being timed; the captured products run without split-K (their workspace can be
@@ -655,24 +656,34 @@ bool davidson(dc2_context* c, int64_t n, const cplx* H, int nroot) {
       if (it == c->dav_graphs.end()) {   // capture; on any failure the context stops using graphs
         hipGraph_t g = nullptr;
         hipGraphExec_t ge = nullptr;
-        bool ok = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess;
-        if (ok) {
-          set_gemm_no_workspace(true);   // the graph must not hold the grow-only split-K buffer
-          try {
-            segment(m_in, false);
-          } catch (...) {
-            ok = false;
+        bool ok = c->capture_stream != nullptr ||
+                  hipStreamCreateWithFlags(&c->capture_stream, hipStreamNonBlocking) == hipSuccess;
+        hipStream_t cs = c->capture_stream;
+        {
+          std::shared_lock<std::shared_mutex> lk(capture_mutex());
+          ok = ok && hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) == hipSuccess;
+          if (ok) {
+            set_gemm_no_workspace(true);   // the graph must not hold the grow-only split-K buffer
+            try {
+              segment(cs, m_in, false);
+            } catch (...) {
+              ok = false;
+            }
+            set_gemm_no_workspace(false);
+            ok = hipStreamEndCapture(cs, &g) == hipSuccess && ok && g != nullptr;
           }
-          set_gemm_no_workspace(false);
-          ok = hipStreamEndCapture(s, &g) == hipSuccess && ok && g != nullptr;
-          ok = ok && hipGraphInstantiateWithFlags(&ge, g, 0) == hipSuccess;
-          if (g) (void)hipGraphDestroy(g);
         }
+        ok = ok && hipGraphInstantiateWithFlags(&ge, g, 0) == hipSuccess;
+        if (g) (void)hipGraphDestroy(g);
         if (ok) {
           it = c->dav_graphs.emplace(key, ge).first;
           ++c->graph_captures;
         } else {
+          // a capture that another thread's work on the null stream has broken stays with its
+          // stream (HIP refuses its launches from then on, and those of a new stream in its
+          // place): the stream is left as it is
           (void)hipGetLastError();
+          c->capture_stream = nullptr;
           c->graphs = false;
         }
       }
@@ -680,10 +691,10 @@ bool davidson(dc2_context* c, int64_t n, const cplx* H, int nroot) {
         DC2_HIP(hipGraphLaunch(it->second, s));
         ++c->graph_launches;
       } else {
-        segment(m_in, false);
+        segment(s, m_in, false);
       }
     } else {
-      segment(m_in, restart);
+      segment(s, m_in, restart);
     }
     if (restart) m = b;
     int kept_host = 0;
@@ -1747,10 +1758,7 @@ Lane& worker_lane(dc2_context* c, int i) {
     c->lanes.push_back(std::move(L));
   }
   Lane& L = *c->lanes[i - 1];
-  if (!L.blas) {   // streams made at context creation get their handle here
-    DC2_ROCSOLVER(rocblas_create_handle(&L.blas));
-    DC2_ROCSOLVER(rocblas_set_stream(L.blas, L.stream));
-  }
+  if (!L.blas) L.blas = make_blas_handle(L.stream);   // streams made at context creation get their handle here
   return L;
 }
 
@@ -2246,8 +2254,7 @@ int context_create_lanes(int32_t device, int lanes, dc2_context** out) {
       DC2_HIP(hipStreamCreateWithFlags(&L->stream, hipStreamNonBlocking));
       c->lanes.push_back(std::move(L));
     }
-    DC2_ROCSOLVER(rocblas_create_handle(&c->blas));
-    DC2_ROCSOLVER(rocblas_set_stream(c->blas, c->stream));
+    c->blas = make_blas_handle(c->stream);
     c->lane0 = std::make_unique<Lane>();
     c->lane0->stream = c->stream;
     c->lane0->blas = c->blas;
@@ -2282,7 +2289,8 @@ int dc2_context_destroy(dc2_context* ctx) {
     if (ctx->gstats.on) set_gemm_stats(nullptr);
     for (auto& r : ctx->gstats.rec) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
     for (auto& kv : ctx->dav_graphs) (void)hipGraphExecDestroy(kv.second);
-    if (ctx->blas) rocblas_destroy_handle(ctx->blas);
+    drop_blas_handle(ctx->blas);
+    if (ctx->capture_stream) (void)hipStreamDestroy(ctx->capture_stream);
     hipStream_t s = ctx->stream;
     delete ctx;
     if (s) {

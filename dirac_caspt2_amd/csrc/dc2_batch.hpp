@@ -16,12 +16,20 @@
 #include <deque>
 #include <memory>
 #include <mutex>
+#include <shared_mutex>
 #include <thread>
 #include <vector>
 
 #include "dc2_common.hpp"
 
 namespace dc2 {
+
+// A rocBLAS handle on stream s, and its end.  Both work on the null stream, which HIP refuses
+// while any thread captures a graph (the capture is lost as well): they take this lock alone,
+// every capture shares it.
+std::shared_mutex& capture_mutex();
+rocblas_handle make_blas_handle(hipStream_t s);
+void drop_blas_handle(rocblas_handle h);
 
 class EigBatcher {
  public:

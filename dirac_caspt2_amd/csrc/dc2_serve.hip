@@ -39,6 +39,28 @@ void set_last_error(const std::string& msg);   // dc2_api.hip: the message dc2_l
 void set_batcher(dc2_context* c, EigBatcher* b);   // dc2_api.hip: route the context's eigensolves
 int context_create_lanes(int32_t device, int lanes, dc2_context** out);   // dc2_api.hip: with lane streams
 
+std::shared_mutex& capture_mutex() {
+  static std::shared_mutex mu;
+  return mu;
+}
+
+rocblas_handle make_blas_handle(hipStream_t s) {
+  std::lock_guard<std::shared_mutex> lk(capture_mutex());
+  rocblas_handle h = nullptr;
+  if (rocblas_create_handle(&h) != rocblas_status_success) throw Error(3, "rocblas_create_handle failed");
+  if (rocblas_set_stream(h, s) != rocblas_status_success) {
+    rocblas_destroy_handle(h);
+    throw Error(3, "rocblas_set_stream failed");
+  }
+  return h;
+}
+
+void drop_blas_handle(rocblas_handle h) {
+  if (!h) return;
+  std::lock_guard<std::shared_mutex> lk(capture_mutex());
+  rocblas_destroy_handle(h);
+}
+
 // ---------------------------------------------------------------- EigBatcher
 EigBatcher::EigBatcher(int device, int max_batch, double window_s, int executors)
     : device_(device), max_batch_(max_batch), window_(window_s) {
@@ -46,8 +68,7 @@ EigBatcher::EigBatcher(int device, int max_batch, double window_s, int executors
   for (int k = 0; k < executors; ++k) {
     auto x = std::make_unique<Exec>();
     DC2_HIP(hipStreamCreateWithFlags(&x->stream, hipStreamNonBlocking));
-    if (rocblas_create_handle(&x->blas) != rocblas_status_success) throw Error(3, "rocblas_create_handle failed");
-    rocblas_set_stream(x->blas, x->stream);
+    x->blas = make_blas_handle(x->stream);
     execs_.push_back(std::move(x));
   }
   for (auto& x : execs_) x->th = std::thread(&EigBatcher::run, this, x.get());
@@ -66,7 +87,7 @@ EigBatcher::~EigBatcher() {
     x->D.release();
     x->E.release();
     x->info.release();
-    rocblas_destroy_handle(x->blas);
+    drop_blas_handle(x->blas);
     release_stream_workspace(x->stream);
     (void)hipStreamDestroy(x->stream);
   }
