@@ -283,7 +283,11 @@ struct dc2_server {
   std::condition_variable cv_work, cv_done;
   std::vector<std::thread> threads;
   std::string ckpt_dir;   // per-request checkpoint files (empty: off)
-  std::vector<std::pair<std::string, int64_t>> options;   // applied to every slot context
+  // applied to every slot context, in order.  Slots start without Davidson graphs: HIP refuses a
+  // program's work on the null stream while any slot captures, at moments the program does not
+  // choose; and eight slots replaying graphs wait for each other (16 energies of 156 spinors 89 ms,
+  // 75 with direct launches; one context alone takes the same time either way).
+  std::vector<std::pair<std::string, int64_t>> options = {{"graphs", 0}};
   std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
   double now() const { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); }
 };
@@ -485,6 +489,7 @@ int dc2_server_create_batched(int32_t device, int32_t nslots, int64_t mem_budget
       return fail(st, "dc2_server_create: " + msg);
     }
     if (S->batcher) dc2::set_batcher(c, S->batcher.get());
+    for (const auto& o : S->options) (void)dc2_set_option(c, o.first.c_str(), o.second);   // known names and values
     S->slot_ctx.push_back(c);
     S->slot_mol.push_back(nullptr);
     S->held.push_back(0);

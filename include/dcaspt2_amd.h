@@ -225,7 +225,9 @@ int dc2_get_gemm_op_stats(dc2_context* ctx, char opA, char opB, double* out);
  *                  eigenproblem of nact^2 (nact-1)/2 instead of C(nact, nelec-1)) when that is
  *                  smaller and more than 32 directions are cut anyway, 0 never;
  *   "graphs":      1 (default) block-Davidson iterations replayed from captured graphs
- *                  (dc2_get_graph_stats), 0 every launch issued directly;
+ *                  (dc2_get_graph_stats), 0 every launch issued directly (default of a request
+ *                  server's slots).  While a capture runs HIP refuses the process's work on the
+ *                  null stream, in any thread: 0 for a program whose other threads use it;
  *   "schur":       1 (default) E2 of the determinant-space route through the compressed
  *                  resolvent when at most 32 directions are cut, 0 always through the
  *                  eigendecomposition of B~;
