@@ -34,6 +34,7 @@ _SIGS = {
     "dc2_get_ci_vector": (c_int, [P, c_int, P]),
     "dc2_caspt2": (c_int, [P, c_int, c_dbl, P, P, P]),
     "dc2_get_subspace_info": (c_int, [P, P, P]),
+    "dc2_get_routes": (c_int, [P, P]),
     "dc2_get_fock_rotation": (c_int, [P, P, P]),
     "dc2_get_rotated_ci": (c_int, [P, P]),
     "dc2_get_density": (c_int, [P, c_int, P, c_i64]),

@@ -275,6 +275,14 @@ class Caspt2Context:
             margin={X: float(margin[k]) for k, X in enumerate(SUBSPACES)},
             timings=[float(t) for t in tm])
 
+    ROUTES = ("whole_rank", "deflated", "vectors", "cg", "compressed", "b_vectors", "refused")
+
+    def routes(self) -> Dict[str, set]:
+        """dc2_get_routes: per subspace of the last caspt2 the names (ROUTES) of the ways it took."""
+        bits = np.zeros(8, dtype=np.int32)
+        check("dc2_get_routes", self.lib.dc2_get_routes(self.h, _ptr(bits)))
+        return {X: {name for b, name in enumerate(self.ROUTES) if bits[k] >> b & 1} for k, X in enumerate(SUBSPACES)}
+
     def fock_rotation(self):
         n = sum(self.dims[:3])
         eps = np.zeros(n)

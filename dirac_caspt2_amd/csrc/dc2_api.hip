@@ -164,6 +164,7 @@ struct dc2_context {
   DevBuf<int> tpairs, ipairs, spairs;
   int64_t sub_info[4 * DC2_NSUBSPACE] = {0};
   double sub_margin[DC2_NSUBSPACE] = {0};
+  int32_t sub_route[DC2_NSUBSPACE] = {0};
   double timings[12] = {0};
   bool have_pt2 = false;
   // scratch
@@ -855,6 +856,7 @@ void transform(dc2_context* c, const std::string& name) {
 struct SolveOut {
   double e2 = 0, sumc2 = 0, margin = INFINITY;
   int64_t dimm = 0;
+  int route = 0;   // DC2_ROUTE_* bits
 };
 
 // e2 and sumc2 from the two-double result of a reduction on lane L
@@ -890,6 +892,7 @@ bool cg_energy(dc2_context* c, Lane& L, int64_t dimm, int64_t npert, const cplx*
   if (c->debug)
     std::fprintf(stderr, "dc2: conjugate gradients n=%lld, %lld columns: %s, %d iterations\n", (long long)dimm,
                  (long long)npert, ok ? "converged" : "failed", it);
+  r.route |= ok ? DC2_ROUTE_CG : DC2_ROUTE_REFUSED;
   if (ok) read_out2(L, out2, r);
   return ok;
 }
@@ -913,6 +916,7 @@ void finish_block(dc2_context* c, Lane& L, char sub, int64_t dimm, int64_t npert
   double* out2 = L.d("out2", 2);
   e2_reduce(s, dimm, npert, X, wb, alpha, partial, np, out2);
   read_out2(L, out2, r);
+  r.route |= DC2_ROUTE_B_VECTORS;
 }
 
 // count of retained eigenvalues (w >= 1e-8, cutoff.F90:64-69) and the distance of the
@@ -942,9 +946,12 @@ struct BlockPrep {
   bool cg = false;   // X_bc1 holds B~, not its eigenvectors
   bool chol = false; // S^-1/2 is the inverse Cholesky factor in X_hLi, not U L^-1/2 in X_uc
   double margin = INFINITY;
+  int route = 0;
 };
-BlockPrep solve_prep(dc2_context* c, Lane& L, char X, int64_t n, cplx* S, cplx* B, EigKind kind, double scale = 1.0) {
+BlockPrep solve_prep(dc2_context* c, Lane& L, char X, int64_t n, cplx* S, cplx* B, EigKind kind, double scale = 1.0,
+                     int route = 0) {
   BlockPrep p;
+  p.route = route | DC2_ROUTE_VECTORS;   // route: of an attempt without the eigenvectors
   p.n = n;
   if (n == 0) return p;
   hipStream_t s = L.stream;
@@ -1017,8 +1024,9 @@ bool chol_small(const dc2_context* c, char X, int64_t n) {
 bool chol_prep(dc2_context* c, Lane& L, char X, int64_t n, cplx* S, cplx* B, double scale, BlockPrep& p) {
   const double thr = 1.0e-8;
   // a relative 1e-4 above the threshold: closer ones are left to the eigensolver
-  if (!(chol_route(c, X, n) || chol_small(c, X, n)) || !chol_whiten(c, L, X, n, S, B, 1.0001 * thr / scale))
-    return false;
+  if (!(chol_route(c, X, n) || chol_small(c, X, n))) return false;
+  p.route = DC2_ROUTE_REFUSED;
+  if (!chol_whiten(c, L, X, n, S, B, 1.0001 * thr / scale)) return false;
   double lam = 0.0;
   if (!chol_lambda_min(L.stream, n, L.z((std::string(1, X) + "_hLi").c_str(), 1), L.z("lanczos", 4 * n + 256),
                        reinterpret_cast<double*>(L.host(512 * sizeof(double), 1)), lam))
@@ -1027,6 +1035,7 @@ bool chol_prep(dc2_context* c, Lane& L, char X, int64_t n, cplx* S, cplx* B, dou
   p.dimm = n;
   p.margin = std::min(p.margin, std::fabs(scale * lam - thr));
   p.chol = true;
+  p.route = DC2_ROUTE_WHOLE_RANK;
   p.cg = cg_route(c, X, n);
   if (!p.cg)
     zheevd(c, L, (int)n, L.z((std::string(1, X) + "_bc1").c_str(), n * n), L.d((std::string(1, X) + "_wb").c_str(), n),
@@ -1040,6 +1049,7 @@ SolveOut solve_finish(dc2_context* c, Lane& L, char X, const BlockPrep& p, int64
   SolveOut r;
   r.margin = p.margin;
   r.dimm = p.dimm;
+  r.route = p.route;
   if (p.n == 0 || p.dimm == 0 || npert == 0) return r;
   hipStream_t s = L.stream;
   auto nm = [X](const char* b) { return std::string(1, X) + b; };
@@ -1070,6 +1080,7 @@ SolveOut solve_finish(dc2_context* c, Lane& L, char X, const BlockPrep& p, int64
   double* out2 = L.d(nm("_out2").c_str(), 2);
   e2_reduce(s, dimm, npert, Xm, wb, alpha, partial, np, out2);
   read_out2(L, out2, r);
+  r.route |= DC2_ROUTE_B_VECTORS;
   return r;
 }
 
@@ -1082,6 +1093,7 @@ struct GramMetric {
   bool defl = false;      // not thin: the cut directions in X_Gd, L^-1 of G + Gd Gd^H in X_hLi
   int64_t m = 0, dimm = 0;
   double margin = INFINITY;
+  int route = 0;
   double seconds = 0.0;   // time spent on the lane before the subspace itself ran
 };
 
@@ -1250,9 +1262,12 @@ GramMetric gram_eig(dc2_context* c, Lane& L, char X, int64_t n, const cplx* Y, c
         g.chol = g.btilde = g.cg = true;
         g.dimm = nred;
         g.margin = std::min(g.margin, thr);
+        g.route = DC2_ROUTE_WHOLE_RANK;
         return g;
       }
+      g.route = DC2_ROUTE_REFUSED;
     }
+    g.route |= DC2_ROUTE_VECTORS;
     zheevd(c, L, (int)nred, T, lt, "a determinant-space metric", ras ? EigKind::rank_deficient : EigKind::general);
     g.margin = std::min(g.margin, thr);   // the m - nred eigenvalues of G that vanish identically
     g.dimm = count_retained(L, nred, lt, g.margin);
@@ -1271,7 +1286,14 @@ GramMetric gram_eig(dc2_context* c, Lane& L, char X, int64_t n, const cplx* Y, c
   cplx* G = L.z(nm("_G").c_str(), m * m);
   zherk_upper(s, m, n, Phi, m, G, m);   // Hermitian: the upper tiles only
   check_finite(c, s, "Phi Phi^H", G, m * m);
-  if (deflate_route(c, X, m) && gram_deflate(c, L, X, G, g)) return g;
+  if (deflate_route(c, X, m)) {
+    if (gram_deflate(c, L, X, G, g)) {
+      g.route = g.dimm < m ? DC2_ROUTE_DEFLATED : DC2_ROUTE_WHOLE_RANK;
+      return g;
+    }
+    g.route = DC2_ROUTE_REFUSED;
+  }
+  g.route |= DC2_ROUTE_VECTORS;
   zheevd(c, L, (int)m, G, lam, "a determinant-space metric", ras ? EigKind::rank_deficient : EigKind::general);
   g.dimm = count_retained(L, m, lam, g.margin);
   return g;
@@ -1374,6 +1396,7 @@ SolveOut solve_block_gram(dc2_context* c, Lane& L, char X, const GramMetric& g, 
   const int64_t m = g.m, dimm = g.dimm;
   r.margin = g.margin;
   r.dimm = dimm;
+  r.route = g.route;
   if (m == 0 || dimm == 0 || npert == 0) return r;
   const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
   const cplx* Phi = L.z(nm("_Phi").c_str(), m * n);
@@ -1405,10 +1428,14 @@ SolveOut solve_block_gram(dc2_context* c, Lane& L, char X, const GramMetric& g, 
     double* out2 = L.d("out2", 2);
     e2_schur(s, m, rd, npert, Gd, Z, f, alpha, partial, out2);
     read_out2(L, out2, r);
-    if (std::isfinite(r.e2) && std::isfinite(r.sumc2)) return r;
+    if (std::isfinite(r.e2) && std::isfinite(r.sumc2)) {
+      r.route |= DC2_ROUTE_COMPRESSED;
+      return r;
+    }
     // a singular compressed system: the eigendecomposition after all
     GramMetric full = g;
     full.defl = false;
+    full.route |= DC2_ROUTE_REFUSED | DC2_ROUTE_VECTORS;
     cplx* Gm = L.z(nm("_G").c_str(), m * m);
     double* lam = L.d(nm("_lam").c_str(), m);
     zheevd(c, L, (int)m, Gm, lam, "a determinant-space metric");
@@ -1454,7 +1481,11 @@ SolveOut solve_block_gram(dc2_context* c, Lane& L, char X, const GramMetric& g, 
     double* out2 = L.d("out2", 2);
     e2_schur(s, m, (int)nd, npert, G, Z, f, alpha, partial, out2);
     read_out2(L, out2, r);
-    if (std::isfinite(r.e2) && std::isfinite(r.sumc2)) return r;
+    if (std::isfinite(r.e2) && std::isfinite(r.sumc2)) {
+      r.route |= DC2_ROUTE_COMPRESSED;
+      return r;
+    }
+    r.route |= DC2_ROUTE_REFUSED;
     // a singular compressed system: fall through to the eigendecomposition of B~
   }
   if (g.btilde) {   // B~ formed (and diagonalised) before V was known
@@ -1473,6 +1504,7 @@ SolveOut solve_block_gram(dc2_context* c, Lane& L, char X, const GramMetric& g, 
     double* out2 = L.d("out2", 2);
     e2_reduce(s, dimm, npert, Xm, wb, alpha, partial, np, out2);
     read_out2(L, out2, r);
+    r.route |= DC2_ROUTE_B_VECTORS;
     return r;
   }
   cplx* FG = L.z(nm("_FG").c_str(), m * dimm);
@@ -1599,10 +1631,11 @@ SubPrep subspace_prep(dc2_context* c, Lane& L, int k) {
       const bool ras = c->ras[0] + c->ras[1] + c->ras[2] != 0;
       if (!route.phi || nred > mdet || !chol_prep(c, L, X, nred, S, B, 2.0, p.bp))
         p.bp = solve_prep(c, L, X, nred, S, B, nred > mdet || (route.phi && ras) ? EigKind::rank_deficient
-                                                                                 : EigKind::general, 2.0);
+                                                                                 : EigKind::general, 2.0, p.bp.route);
     } else {
       const EigKind kind = (X == 'A' || X == 'C') ? EigKind::rank_deficient : EigKind::general;
-      if (!chol_small(c, X, n) || !chol_prep(c, L, X, n, S, B, 1.0, p.bp)) p.bp = solve_prep(c, L, X, n, S, B, kind);
+      if (!chol_small(c, X, n) || !chol_prep(c, L, X, n, S, B, 1.0, p.bp))
+        p.bp = solve_prep(c, L, X, n, S, B, kind, 1.0, p.bp.route);
     }
   }
   p.seconds = tx.stop();
@@ -1746,6 +1779,7 @@ void run_subspace(dc2_context* c, Lane& L, int k, double eshift, double* e2, dou
   c->sub_info[4 * k + 2] = npert;
   c->sub_info[4 * k + 3] = 1;
   c->sub_margin[k] = r.margin;
+  c->sub_route[k] = r.route;
   c->timings[4 + k] = tx.stop() + prep->seconds;
 }
 
@@ -1819,6 +1853,7 @@ void run_caspt2(dc2_context* c, int selectroot, double eshift, double* e2, doubl
   for (double& t : c->timings) t = (&t == &c->timings[0]) ? t : 0.0;
   std::memset(c->sub_info, 0, sizeof(c->sub_info));
   for (int k = 0; k < DC2_NSUBSPACE; ++k) c->sub_margin[k] = INFINITY;
+  std::memset(c->sub_route, 0, sizeof(c->sub_route));
 
   Timer t1(s);
   // ---- E_pq tables and the CASCI 1-RDM in the original basis
@@ -2474,6 +2509,13 @@ int dc2_get_subspace_info(dc2_context* c, int64_t* info, double* margin) {
     DC2_CHECK(c && c->have_pt2, 1, "no CASPT2 result");
     std::memcpy(info, c->sub_info, sizeof(c->sub_info));
     std::memcpy(margin, c->sub_margin, sizeof(c->sub_margin));
+  });
+}
+
+int dc2_get_routes(dc2_context* c, int32_t* routes) {
+  return guarded([&] {
+    DC2_CHECK(c && c->have_pt2 && routes, 1, "no CASPT2 result");
+    std::memcpy(routes, c->sub_route, sizeof(c->sub_route));
   });
 }
 

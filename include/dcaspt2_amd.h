@@ -97,6 +97,21 @@ int dc2_caspt2(dc2_context* ctx, int32_t selectroot, double eshift, double* e2, 
  * {dimn, dimm, npert, ran}, margin[k] = min |w_S - 1e-8| (distance of the
  * closest S eigenvalue to the linear-dependency threshold). */
 int dc2_get_subspace_info(dc2_context* ctx, int64_t* info, double* margin);
+/* The way each subspace of the last dc2_caspt2 took, routes[8] as sums of DC2_ROUTE_* (0 for H
+ * and for subspaces that were skipped): its metric by the Cholesky factor of a matrix of whole
+ * rank, by a factor with the few cut directions deflated, or by its eigenvectors; E2 by conjugate
+ * gradients, by the compressed resolvent, or by the eigenvectors of B~; and whether a way without
+ * eigenvectors was tried and refused.  For tests and for reading timings. */
+enum {
+  DC2_ROUTE_WHOLE_RANK = 1,
+  DC2_ROUTE_DEFLATED = 2,
+  DC2_ROUTE_VECTORS = 4,
+  DC2_ROUTE_CG = 8,
+  DC2_ROUTE_COMPRESSED = 16,
+  DC2_ROUTE_B_VECTORS = 32,
+  DC2_ROUTE_REFUSED = 64
+};
+int dc2_get_routes(dc2_context* ctx, int32_t* routes);
 /* orbital energies after fockdiag (nmo doubles) and the rotation U (nmo x nmo complex) */
 int dc2_get_fock_rotation(dc2_context* ctx, double* eps, double* U);
 /* rotated CI vector of the last dc2_caspt2 (ndet complex) */
