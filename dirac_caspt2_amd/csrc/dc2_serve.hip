@@ -243,9 +243,11 @@ int64_t binom(int n, int k) {
 // device bytes one request holds while it runs (besides the molecule's resident blocks):
 // transformed blocks + transform scratch, CI matrix and LU copy, E_pq tables and images,
 // density tensors, the A/C metric work and the V matrices, doubled to cover what the sum
-// leaves out (lane scratch, split-precision slices, solver workspaces): measured, one
-// context with four lanes held 2.2 GB at 192 spinors (sum 1.3 GB) and 8.8 GB at 324
-// spinors (sum 7.7 GB)
+// leaves out (lane scratch, split-precision slices, the Cholesky factors of A and C, solver
+// workspaces): measured after one energy, a slot with four lanes holds 1.8 GB at 192 spinors and
+// 7.2 GB at 324 (sums 1.3 and 7.7 GB), 1.9 and 7.5 GB where the metrics of a weakly correlated
+// state are factorised and then diagonalised after all; the largest share of the doubled sum over
+// 8 to 16 active and 20 to 280 secondary spinors is 0.81 (238 spinors with 5 active electrons)
 int64_t footprint_bytes(int64_t ni, int64_t na, int64_t ns, int64_t ne) {
   const int64_t z = 16;
   const int64_t blocks[] = {na * ni * na * na, na * ni * ni * ni, na * ni * na * ni, ns * na * na * na,
@@ -255,12 +257,11 @@ int64_t footprint_bytes(int64_t ni, int64_t na, int64_t ns, int64_t ne) {
   int64_t tb = 0, mx = 0;
   for (int64_t b : blocks) { tb += b; mx = b > mx ? b : mx; }
   const int64_t nf = binom((int)na, (int)ne), na2 = na * na, na3 = na2 * na;
-  const int64_t mA = binom((int)na, (int)ne + 1), mC = binom((int)na, (int)ne - 1);
+  const int64_t mA = binom((int)na, (int)ne + 1);
   const int64_t ci = 3 * nf * nf;
   const int64_t dens = 4 * nf * na2 + nf * na2 * na2 + 6 * na3 * na3;
-  const int64_t nr = na2 * (na - 1) / 2;   // A and C by their Cholesky factors (5 + 1 matrices each)
   const int64_t ac = 2 * (std::min(mA, na3) * na3 + 2 * std::min(mA, na3) * std::min(mA, na3)) +
-                     na3 * (ni + ns) * 3 + (nr < mA ? 6 * nr * nr : 0) + (nr <= 2048 && mC > na3 ? mC * na3 : 0);
+                     na3 * (ni + ns) * 3;
   const int64_t other = 8 * (ns + ni) * (ns + ni) + 4 * ns * ns * ni + 4 * ns * ni * ni * na;
   return 2 * (z * (tb + mx + ci + dens + ac + other) + (64ll << 20));
 }
