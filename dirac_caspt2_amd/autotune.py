@@ -5,6 +5,7 @@ beats the built-in rule is installed in the library's process-wide table, which 
 dispatch consults for products of exactly that shape.  A table can be saved as JSON and
 installed again in another process on the same hardware (load)."""
 import json
+import warnings
 from typing import Callable, Dict, List
 
 from .api import Caspt2Context, gemm_clear_choices, gemm_set_choice
@@ -40,17 +41,27 @@ def tune_workload(ctx: Caspt2Context, run: Callable[[], None], reps: int = 3) ->
             "tuned_us": 1e6 * sum(t["seconds"] for t in table)}
 
 
+# What the variant numbers of a table stand for (rows x columns of a workgroup's tile / K tile):
+# a saved table names it, and one made for other kernels is not installed.
+KERNELS = ["64x64/8", "64x32/16", "64x16/16", "64x16/8"]
+
+
 def save(table: List[Dict], path: str) -> None:
     with open(path, "w") as f:
-        json.dump([t for t in table if t["variant"] > 0], f, indent=1)
+        json.dump({"kernels": KERNELS, "choices": [t for t in table if t["variant"] > 0]}, f, indent=1)
 
 
 def load(path: str, clear: bool = True) -> int:
-    """Install the choices of a saved table; returns how many."""
+    """Install the choices of a saved table; returns how many.  A table saved for other kernels (a
+    bare list, as earlier versions wrote, is one) installs nothing, with a warning."""
     if clear:
         gemm_clear_choices()
     with open(path) as f:
-        table = json.load(f)
+        saved = json.load(f)
+    if not isinstance(saved, dict) or saved.get("kernels") != KERNELS:
+        warnings.warn(f"{path}: choices for other GEMM kernels, not installed; tune again")
+        return 0
+    table = saved["choices"]
     for t in table:
         gemm_set_choice(t["opA"], t["opB"], t["M"], t["N"], t["K"], t["batch"], t["variant"], t["split"])
     return len(table)
