@@ -77,9 +77,9 @@ class DeviceArray:
         return out
 
     def free(self):
-        if self.ptr and self.ctx.h:
-            check("dc2_free", self.ctx.lib.dc2_free(self.ctx.h, self.ptr))
-        self.ptr = 0
+        ptr, self.ptr = self.ptr, 0   # given up first: see Caspt2Context.close
+        if ptr and self.ctx.h:
+            check("dc2_free", self.ctx.lib.dc2_free(self.ctx.h, ptr))
 
     def __del__(self):
         try:
@@ -104,9 +104,11 @@ class Caspt2Context:
         self._keep: Dict[str, object] = {}
 
     def close(self):
-        if self.h:
-            check("dc2_context_destroy", self.lib.dc2_context_destroy(self.h))
-            self.h = None
+        # the handle is given up before the call: at the interpreter's exit check() may be gone
+        # already, and a second close() would destroy the context again
+        h, self.h = self.h, None
+        if h:
+            check("dc2_context_destroy", self.lib.dc2_context_destroy(h))
             self._keep.clear()
 
     def __enter__(self):
@@ -575,9 +577,9 @@ class Server:
                         (int(x) for x in out)))
 
     def close(self):
-        if self.h:
-            check("dc2_server_destroy", self.lib.dc2_server_destroy(self.h))
-            self.h = None
+        h, self.h = self.h, None   # as in Caspt2Context.close
+        if h:
+            check("dc2_server_destroy", self.lib.dc2_server_destroy(h))
 
     def __enter__(self):
         return self
