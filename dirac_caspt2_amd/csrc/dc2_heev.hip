@@ -16,7 +16,7 @@
 // Layout: workgroup w of nwg owns the columns j = w + nwg * l (l = wave + 8 c, c < CPW), held
 // in registers for the whole reduction; lane L of a wave holds rows L + 64 s.  Per step:
 //   (a) every workgroup forms p_j for its columns (a wave reduction per column) and a partial
-//       of Re(v^H p); the owner of column k+1 has published it at the end of step k-1;
+//       of Re(v^H p); the owner of column k+1 publishes that column as it stands;
 //   -- one grid barrier --
 //   (b) every workgroup reads p, the partials and column k+1, updates its columns, applies
 //       the same update to its copy of column k+1 and derives reflector k+1 from it.
@@ -230,22 +230,6 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
   // the loads of the owned columns complete here, once, rather than being waited for again
   // before every store that might use them
   __builtin_amdgcn_s_waitcnt(0);
-  // the owner of column k+1 publishes it for step k as soon as it is up to date: its stores
-  // complete behind the reflector and the products, not between them and the barrier (half of
-  // NC by the parity of k; the step before last has been read by all, see the barrier)
-  auto publish = [&](int k) {
-    cplx* NC = w.NC + (int64_t)(k & 1) * n;
-#pragma unroll
-    for (int c = 0; c < CPW; ++c)
-      if (col[c] == k + 1) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-          const int i = lane + 64 * s;
-          if (i > k && i < n) st_coherent(NC + i, a[c][s]);
-        }
-      }
-  };
-  publish(0);
   reflector(n, 0, x2, sc, sv, redn, &s_tau, &s_delta, d, sub, tau, delta, Vh);
   for (int k = 0; k <= n - 3; ++k) {
     const int par = k & 1;
@@ -275,6 +259,16 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
       }
       if (lane == 0) red[wave] = part;
     }
+    // the owner publishes column k+1
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+      if (col[c] == k + 1) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+          const int i = lane + 64 * s;
+          if (i > k && i < n) st_coherent(NC + i, a[c][s]);
+        }
+      }
     if (!grid_sync(w.bar, k, w.err, t != 0.0 ? Sp + wg : nullptr, red, n, sv, Vh)) return;
     // (b) one round of coherent loads: column k+1, p and the partials (nwg <= 256, one per
     // thread, summed in the same order in every workgroup); q = p - K v is formed where used.
@@ -329,7 +323,6 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
           }
         }
       }
-      if (k < n - 3) publish(k + 1);
       // column k+1 updated by the rows this thread loaded, and its part of the next norm
       const cplx cq1 = cconj(qat(k + 1)), cv1 = cconj(sv[k + 1]);
       for (int i = k + 1 + threadIdx.x; i < n; i += HT_THREADS) {
@@ -340,7 +333,6 @@ __global__ __launch_bounds__(HT_THREADS) void k_hetrd(int n, const cplx* __restr
         if (i > k + 1) x2 += cabs2(x);
       }
     } else {
-      if (k < n - 3) publish(k + 1);
       for (int i = k + 1 + threadIdx.x; i < n; i += HT_THREADS)
         if (i > k + 1) x2 += cabs2(sc[i]);
     }
