@@ -756,10 +756,11 @@ void zgemm(hipStream_t s, char opA, char opB, int64_t M, int64_t N, int64_t K, c
 
 // C (m x m, ldc) = A A^H for A (m x k, lda): the tiles on and above the diagonal on the MFMA
 // kernel, then the lower triangle as the conjugate of the upper one.  Few tiles over a long
-// k (the determinant-space Gram matrices: 91 upper tiles over k = 1728) are split over k
-// into about 1024 workgroups, at most 12 chunks of at least 128, summed in a fixed order by
-// k_herk_reduce (m = 792, k = 1728: 421 us unsplit, 207 / 162 / 164 / 162 / 145 us in 3 / 4
-// / 8 / 12 / 16 chunks).  split: 0 this rule, >= 1 that many k chunks (1: unsplit).
+// k (the determinant-space Gram matrices: 350 upper tiles of 64 x 16 over k = 1728) are split
+// over k towards 2048 workgroups, at most 12 chunks of at least 128, summed in a fixed order by
+// k_herk_reduce (m = 792, k = 1728: 140 us unsplit, 103 / 115 / 102 / 103 / 100 / 108 us in 2 / 3
+// / 4 / 6 / 8 / 12 chunks; m = 210, k = 1000: 51, 29 / 22 / 18 / 20 / 16 / 19).  split: 0 this
+// rule, >= 1 that many k chunks (1: unsplit).
 void zherk_upper(hipStream_t s, int64_t m, int64_t k, const cplx* A, int64_t lda, cplx* C, int64_t ldc, int split) {
   zgemm_herm(s, m, k, A, lda, A, lda, C, ldc, split);
 }

@@ -213,6 +213,8 @@ bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const
     // columns converge from the last one on and the products shrink at every poll
     for (int c = 0; c < CG_CHUNK; ++c, ++it) {
       zgemm(s, 'N', 'N', n, nact, n, one, Bt, n, 0, P, n, 0, zero, Q, n, 0, 1);
+      // rows per thread: the smallest instance that holds n, so that a column stays in registers
+      // with few rows past n (280 columns of 1274 rows: 9.9 us with five, 10.3 with eight)
       if (E <= 1) step<1>(s, ni, nact, Bt, alpha, Q, X, R, P, rho, stop, state);
       else if (E <= 2) step<2>(s, ni, nact, Bt, alpha, Q, X, R, P, rho, stop, state);
       else if (E <= 4) step<4>(s, ni, nact, Bt, alpha, Q, X, R, P, rho, stop, state);
@@ -225,6 +227,10 @@ bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const
     if (nact > 0 && it >= CG_ITMAX) return false;
   }
   if (iterations) *iterations = std::max(it, 1);
+  // a column whose true residual has drifted from the recursive one is refused; over 8 to 16
+  // active spinors and strong and weak correlation it stays below 1.6e-14, and where conditions
+  // up to 6e4 were accepted the sums were 1 to 200 times nearer to exact ones than an
+  // eigendecomposition's
   zgemm(s, 'N', 'N', n, npert, n, one, Bt, n, 0, X, n, 0, zero, Q, n, 0, 1);
   hipLaunchKernelGGL(k_cg_energy, dim3((unsigned)npert), dim3(CG_T), 0, s, ni, alpha, Y, X, Q, 1e-24, partial, state);
   sum_partials(s, npert, partial, out2);
@@ -247,8 +253,8 @@ bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const
 // cores, and one trailing update of the upper tiles (zherk_trailing).  L^-1 from the inverse
 // diagonal blocks by merging neighbours, [[X, 0], [-Z U12^H X, Z]], doubling the block size.
 //
-// Bound by the chain of the 20 steps at n = 1274 (about 60 us each: the elimination 40, the
-// update 15), against 13.4 ms for the tridiagonalisation and 9 ms for the divide and conquer,
+// Bound by the chain of the 20 steps at n = 1274 (42 us for the last to 81 us for the first: the
+// elimination 34, with the block row's product 48, the update 10 to 30), against 13.4 ms for the tridiagonalisation and 9 ms for the divide and conquer,
 // back-transformation and scaled products it replaces; the two factorisations, L^-1 and B~ take
 // 3.3 ms beside the other lanes.  324 spinors, FP64: 49.7 -> 39.9 ms per energy, split 37.7.
 
@@ -590,7 +596,8 @@ __global__ __launch_bounds__(1024) void k_lanczos_small(int n, int np, int j0, i
   }
 }
 
-// a start vector with a part along every direction: unit-modulus entries of an integer hash
+// a start vector with a part along every direction: unit-modulus entries of an integer hash (the
+// first steps of splitmix64's finaliser)
 __global__ void k_lanczos_start(int n, cplx* __restrict__ v) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
@@ -666,7 +673,7 @@ void chol_inverse(hipStream_t s, int64_t n, const cplx* S, int64_t lds, double s
 
 namespace {
 
-// start columns: unit-modulus entries of an integer hash
+// start columns: unit-modulus entries of an integer hash (splitmix64's finaliser)
 __global__ void k_low_start(int64_t count, int n, cplx* __restrict__ x) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= count) return;
@@ -684,7 +691,9 @@ __global__ void k_low_start(int64_t count, int n, cplx* __restrict__ x) {
 
 int64_t low_work_elems(int64_t n) { return 2 * n * LOW_P + 2 * 3 * LOW_P * LOW_P + 64; }
 
-// X <- X L^-H with X^H X = L L^H, twice (the Gram matrix of the iterated columns is far from 1)
+// X <- X L^-H with X^H X = L L^H, passes times: once keeps the iterated columns apart, the last
+// step takes three, to orthonormality at rounding (one pass leaves eps times the condition of the
+// columns' Gram matrix, which is far from 1)
 static void low_orth(hipStream_t s, int64_t n, cplx* X, cplx* Y, cplx* small, int* flags, int passes) {
   const cplx one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
   const int64_t p = LOW_P, pp = p * p;
