@@ -286,8 +286,8 @@ struct dc2_server {
   std::string ckpt_dir;   // per-request checkpoint files (empty: off)
   // applied to every slot context, in order.  Slots start without Davidson graphs: HIP refuses a
   // program's work on the null stream while any slot captures, at moments the program does not
-  // choose; and eight slots replaying graphs wait for each other (16 energies of 156 spinors 89 ms,
-  // 75 with direct launches; one context alone takes the same time either way).
+  // choose, and direct launches take the same time (16 energies of 156 spinors on 8 slots 88.3 ms,
+  // 89.1 with graphs).
   std::vector<std::pair<std::string, int64_t>> options = {{"graphs", 0}};
   std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
   double now() const { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); }
