@@ -228,9 +228,9 @@ bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const
   }
   if (iterations) *iterations = std::max(it, 1);
   // a column whose true residual has drifted from the recursive one is refused; over 8 to 16
-  // active spinors and strong and weak correlation it stays below 1.6e-14, and where conditions
-  // up to 6e4 were accepted the sums were 1 to 200 times nearer to exact ones than an
-  // eigendecomposition's
+  // active spinors and strong and weak correlation it stays below 1.6e-14, and on matrices with
+  // conditions up to 6e4 the sums were exact to rounding or nearer to exact ones than an
+  // eigendecomposition's (by up to 270 times)
   zgemm(s, 'N', 'N', n, npert, n, one, Bt, n, 0, X, n, 0, zero, Q, n, 0, 1);
   hipLaunchKernelGGL(k_cg_energy, dim3((unsigned)npert), dim3(CG_T), 0, s, ni, alpha, Y, X, Q, 1e-24, partial, state);
   sum_partials(s, npert, partial, out2);
@@ -254,9 +254,9 @@ bool cg_resolvent(hipStream_t s, int64_t n, int64_t npert, const cplx* Bt, const
 // diagonal blocks by merging neighbours, [[X, 0], [-Z U12^H X, Z]], doubling the block size.
 //
 // Bound by the chain of the 20 steps at n = 1274 (42 us for the last to 81 us for the first: the
-// elimination 34, with the block row's product 48, the update 10 to 30), against 13.4 ms for the tridiagonalisation and 9 ms for the divide and conquer,
-// back-transformation and scaled products it replaces; the two factorisations, L^-1 and B~ take
-// 3.3 ms beside the other lanes.  324 spinors, FP64: 49.7 -> 39.9 ms per energy, split 37.7.
+// elimination 34, with the block row's product 48, the update 10 to 30), against 13.4 ms for the
+// tridiagonalisation and 9 ms for the divide and conquer, back-transformation and scaled products
+// it replaces; the two factorisations, L^-1 and B~ take 3.3 ms beside the other lanes.  324 spinors, FP64: 49.7 -> 39.9 ms per energy, split 37.7.
 
 namespace {
 

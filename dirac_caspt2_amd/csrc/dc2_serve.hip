@@ -246,8 +246,10 @@ int64_t binom(int n, int k) {
 // leaves out (lane scratch, split-precision slices, the Cholesky factors of A and C, solver
 // workspaces): measured after one energy, a slot with four lanes holds 1.8 GB at 192 spinors and
 // 7.2 GB at 324 (sums 1.3 and 7.7 GB), 1.9 and 7.5 GB where the metrics of a weakly correlated
-// state are factorised and then diagonalised after all; the largest share of the doubled sum over
-// 8 to 16 active and 20 to 280 secondary spinors is 0.81 (238 spinors with 5 active electrons)
+// state are factorised and then diagonalised after all.  With one lane the largest share of the
+// doubled sum over 8 to 16 active and 20 to 280 secondary spinors is 0.58 (238 spinors with 5
+// active electrons); every further lane holds a rocBLAS handle of 160 MB, which only the smallest
+// molecules feel (four lanes at 52 spinors: 500 MB against 212)
 int64_t footprint_bytes(int64_t ni, int64_t na, int64_t ns, int64_t ne) {
   const int64_t z = 16;
   const int64_t blocks[] = {na * ni * na * na, na * ni * ni * ni, na * ni * na * ni, ns * na * na * na,

@@ -189,8 +189,8 @@ int dc2_get_gemm_stats(dc2_context* ctx, int32_t tag, double* out);
  *   codes), at most cap rows written, *count = all of them.
  * dc2_gemm_tune: times every candidate for one shape on scratch operands on the context's
  *   stream (kernel variant 1..4: 64, 32, 16 or 16 columns per workgroup with K tiles of 8, 16,
- *   16 or 8; split-K 1, 2, 4 .. 32 for products with few tiles), installs the fastest in the process-wide table when it
- *   beats the built-in choice; out[4] = {variant, split (0, 0: built-in kept), its seconds,
+ *   16 or 8; split-K 1, 2, 4 .. 32 for products with few tiles), installs the fastest in the
+ *   process-wide table when it beats the built-in choice; out[4] = {variant, split (0, 0: built-in kept), its seconds,
  *   the built-in choice's seconds}.  reps: timed repetitions per candidate.
  * dc2_gemm_set_choice: installs a choice (a table saved from an earlier tuning run of the same
  *   kernels: the variant numbers have meant other tiles before).
